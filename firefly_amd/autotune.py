@@ -1,10 +1,11 @@
 """Autotuner for the wavefront launch shapes.
 
 Times renders of the actual request for a few paths-in-flight choices
-(samples per pixel in flight, spp_batch) and for every traversal kernel
-variant (workgroup size, LDS stack entries, refill threshold, loop shape, BVH
-record width; see ff_traversal_variant_info), then keeps the fastest on the
-context.  Results can be written as JSON and reused.
+(samples per pixel in flight, spp_batch) and, with them, the traversal kernel
+variants (see ff_traversal_variant_info), then keeps the fastest on the
+context.  Renders take their traversal shape from the number of rays whatever
+the variant, so the choice that matters is spp_batch; the variant kept is the
+one of traces that count.  Results can be written as JSON and reused.
 """
 from __future__ import annotations
 

@@ -97,9 +97,7 @@ struct ff_context {
     size_t req_cap = 0;
     uint32_t* fetch = nullptr;    // [FETCH_WORDS] segmented traversal work counters
     int32_t* scratch = nullptr;   // this device's fixed trace scratch (ff_trace_closest_noalloc)
-    int trav_variant = 0;
-    int trav_tail = -1;      // variant of the late bounce iterations (-1: none)
-    int trav_tail_from = 0;  // first iteration that uses it
+    int trav_variant = 0;  // of traces that count
     // adjoint: gradient target tables and the deterministic-reduction arena
     ff_dev_gtarget* d_gt = nullptr;
     size_t gt_cap = 0;
@@ -111,18 +109,9 @@ struct ff_context {
 
 struct ff_scene {
     ff_context* ctx = nullptr;
-    int32_t n_tris = 0, n_mats = 0, max_depth = 0;
-    std::vector<ffh::BvhNode> nodes;
-    std::vector<int32_t> ordered;
-    float4* d_nodes = nullptr;       // two-child records
-    float4* d_nodes4 = nullptr;      // 4-wide records
-    int32_t* d_leaf_count = nullptr;
-    float* d_root = nullptr;
-    float* d_tris = nullptr;
-    float4* d_attr = nullptr;        // per slot: normals, uvs, material word (64 B)
-    float* d_tan = nullptr;          // per slot [3][6] tangent frames, or none
-    uint32_t* d_mat = nullptr;
-    float* d_mats = nullptr;
+    int32_t n_tris = 0, n_mats = 0;
+    ffk::DevBvh bvh;        // the binary tree (device)
+    ffk::ScenePack pack;    // traversal and shading arrays (device)
     std::vector<float*> d_tex;
     std::vector<ff_tex_desc> tex_desc;  // host copy (sizes)
     ff_tex_desc* d_tex_desc = nullptr;
@@ -130,10 +119,10 @@ struct ff_scene {
     bool has_type[4] = {false, false, false, false};
     ff_dev_scene view() const {
         ff_dev_scene s;
-        s.nodes = d_nodes; s.nodes4 = d_nodes4; s.leaf_count = d_leaf_count; s.root = d_root; s.tris = d_tris; s.attr = d_attr; s.mat = d_mat;
-        s.tan = d_tan;
-        s.mats = d_mats; s.tex = d_tex_desc; s.n_nodes = (int32_t)nodes.size(); s.n_tris = n_tris;
-        s.n_mats = n_mats; s.n_tex = n_tex; s.max_depth = max_depth;
+        s.nodes = pack.nodes; s.nodes4 = pack.nodes4; s.wide = pack.wide; s.leaf_count = pack.leaf_count;
+        s.root = pack.root; s.tris = pack.tris; s.attr = pack.attr; s.tan = pack.tan; s.mat = pack.mat;
+        s.mats = pack.mats; s.tex = d_tex_desc; s.n_nodes = bvh.n_nodes; s.n_tris = n_tris;
+        s.n_mats = n_mats; s.n_tex = n_tex; s.max_depth = bvh.max_depth; s.wide_levels = pack.wide_levels;
         return s;
     }
 };
@@ -190,8 +179,8 @@ ff_status ensure_paths(ff_context* c, size_t P) {
 // records; up to three per 4-wide record (two binary levels) for the others.
 // Two areas: the extension and shadow traversals of an iteration run at the
 // same time, each with its own.
-ff_status ensure_ovf(ff_context* c, int32_t max_depth) {
-    int32_t entries = std::max(max_depth, 3 * ((max_depth + 1) / 2));
+ff_status ensure_ovf(ff_context* c, int32_t max_depth, int32_t wide_levels) {
+    int32_t entries = std::max(std::max(max_depth, 3 * ((max_depth + 1) / 2)), 3 * wide_levels);
     size_t need = entries > FF_LDS_MIN ? (size_t)(entries - FF_LDS_MIN + 1) : 1;
     if (c->ovf && c->ovf_entries >= need) return FF_OK;
     dfree(c->ovf);
@@ -200,132 +189,11 @@ ff_status ensure_ovf(ff_context* c, int32_t max_depth) {
     return FF_OK;
 }
 
-// The reference's pre-order binary BVH re-packed as 64-byte two-child
-// records: record k holds both child boxes of the k-th interior node, the
-// child refs and the split axis.  Leaf refs are ~(first slot << 4 | count),
-// count 15 meaning "read leaf_count[first slot]".
-void pack_two_child(const std::vector<ffh::BvhNode>& nodes, std::vector<float4>& wide,
-                    std::vector<int32_t>& leaf_count, float root[8], size_t n_tris) {
-    std::vector<int32_t> index(nodes.size(), -1);
-    int32_t nw = 0;
-    for (size_t i = 0; i < nodes.size(); i++)
-        if (nodes[i].n_prims == 0) index[i] = nw++;
-    leaf_count.assign(std::max<size_t>(n_tris, 1), 0);
-    auto ref_of = [&](size_t i) -> int32_t {
-        const ffh::BvhNode& nd = nodes[i];
-        if (nd.n_prims == 0) return index[i];
-        int32_t c = nd.n_prims < 15 ? nd.n_prims : 15;
-        if (c == 15) leaf_count[nd.offset] = nd.n_prims;
-        return ~((nd.offset << 4) | c);
-    };
-    wide.assign((size_t)nw * 4, make_float4(0.f, 0.f, 0.f, 0.f));
-    for (size_t i = 0; i < nodes.size(); i++) {
-        if (nodes[i].n_prims != 0) continue;
-        const ffh::BvhNode& A = nodes[i + 1];
-        const ffh::BvhNode& B = nodes[nodes[i].offset];
-        float4* w = &wide[(size_t)index[i] * 4];
-        w[0] = make_float4(A.bmin[0], A.bmin[1], A.bmin[2], A.bmax[0]);
-        w[1] = make_float4(A.bmax[1], A.bmax[2], B.bmin[0], B.bmin[1]);
-        w[2] = make_float4(B.bmin[2], B.bmax[0], B.bmax[1], B.bmax[2]);
-        int32_t m[4] = {ref_of(i + 1), ref_of((size_t)nodes[i].offset), (int32_t)nodes[i].axis, 0};
-        std::memcpy(&w[3], m, 16);
-    }
-    std::memcpy(root, nodes[0].bmin, 12);
-    std::memcpy(root + 3, nodes[0].bmax, 12);
-    int32_t r = ref_of(0);
-    std::memcpy(root + 6, &r, 4);
-    root[7] = 0.f;
-}
-
-// The binary tree collapsed to 4-wide records of 128 bytes.  The record of
-// interior node N holds the boxes of N's grandchildren: slots 0-1 under N's
-// first child, 2-3 under its second (a child that is a leaf keeps its own
-// box in the first slot of its pair and leaves the second empty), plus the
-// three split axes (N, first child, second child) that order them:
-//   f[0..5] = lo.x, lo.y, lo.z, hi.x, hi.y, hi.z of slots 0..3
-//   f[6]    = refs: >= 0 record index, < 0 leaf ~(first slot << 4 | count)
-//   f[7]    = (axis N, axis first child, axis second child, 0)
-// An empty slot has the box (+inf, -inf), which every slab test misses, and
-// the ref of a leaf with no triangles.  Records are numbered in pre-order.
-void pack_four(const std::vector<ffh::BvhNode>& nodes, std::vector<float4>& recs,
-               std::vector<int32_t>& leaf_count, float root[8], size_t n_tris) {
-    leaf_count.assign(std::max<size_t>(n_tris, 1), 0);
-    std::vector<int32_t> index(nodes.size(), -1);
-    std::vector<size_t> order;  // binary node of each record, pre-order
-    if (nodes[0].n_prims == 0) {
-        std::vector<size_t> stack{0};
-        while (!stack.empty()) {
-            size_t i = stack.back();
-            stack.pop_back();
-            index[i] = (int32_t)order.size();
-            order.push_back(i);
-            size_t kids[2] = {i + 1, (size_t)nodes[i].offset};
-            std::vector<size_t> slots;
-            for (size_t c : kids) {
-                if (nodes[c].n_prims == 0) {
-                    slots.push_back(c + 1);
-                    slots.push_back((size_t)nodes[c].offset);
-                } else {
-                    slots.push_back(c);
-                    slots.push_back(SIZE_MAX);
-                }
-            }
-            for (size_t k = slots.size(); k-- > 0;)
-                if (slots[k] != SIZE_MAX && nodes[slots[k]].n_prims == 0) stack.push_back(slots[k]);
-        }
-    }
-    auto leaf_ref = [&](const ffh::BvhNode& nd) -> int32_t {
-        int32_t c = nd.n_prims < 15 ? nd.n_prims : 15;
-        if (c == 15) leaf_count[nd.offset] = nd.n_prims;
-        return ~((nd.offset << 4) | c);
-    };
-    auto ref_of = [&](size_t i) -> int32_t {
-        return nodes[i].n_prims == 0 ? index[i] : leaf_ref(nodes[i]);
-    };
-    const float inf = std::numeric_limits<float>::infinity();
-    recs.assign(order.size() * 8, make_float4(0.f, 0.f, 0.f, 0.f));
-    for (size_t r = 0; r < order.size(); r++) {
-        size_t i = order[r];
-        size_t kids[2] = {i + 1, (size_t)nodes[i].offset};
-        float lo[3][4], hi[3][4];
-        int32_t ref[4], ax[4] = {(int32_t)nodes[i].axis, 0, 0, 0};
-        for (int side = 0; side < 2; side++) {
-            size_t c = kids[side];
-            size_t sl[2];
-            bool two = nodes[c].n_prims == 0;
-            if (two) {
-                sl[0] = c + 1;
-                sl[1] = (size_t)nodes[c].offset;
-                ax[1 + side] = (int32_t)nodes[c].axis;
-            } else {
-                sl[0] = c;
-                sl[1] = SIZE_MAX;
-            }
-            for (int k = 0; k < 2; k++) {
-                int s = 2 * side + k;
-                if (sl[k] == SIZE_MAX) {
-                    for (int a = 0; a < 3; a++) { lo[a][s] = inf; hi[a][s] = -inf; }
-                    ref[s] = -1;  // a leaf of zero triangles
-                } else {
-                    const ffh::BvhNode& nd = nodes[sl[k]];
-                    for (int a = 0; a < 3; a++) { lo[a][s] = nd.bmin[a]; hi[a][s] = nd.bmax[a]; }
-                    ref[s] = ref_of(sl[k]);
-                }
-            }
-        }
-        float4* w = &recs[r * 8];
-        for (int a = 0; a < 3; a++) {
-            w[a] = make_float4(lo[a][0], lo[a][1], lo[a][2], lo[a][3]);
-            w[3 + a] = make_float4(hi[a][0], hi[a][1], hi[a][2], hi[a][3]);
-        }
-        std::memcpy(&w[6], ref, 16);
-        std::memcpy(&w[7], ax, 16);
-    }
-    std::memcpy(root, nodes[0].bmin, 12);
-    std::memcpy(root + 3, nodes[0].bmax, 12);
-    int32_t r0 = ref_of(0);
-    std::memcpy(root + 6, &r0, 4);
-    root[7] = 0.f;
+// a device tree into the caller's host arrays (either may be null)
+ff_status read_bvh(const ffk::DevBvh& b, int32_t n_tris, ff_bvh_node* nodes_out, int32_t* ordered_out) {
+    if (nodes_out) HIP_TRY(hipMemcpy(nodes_out, b.nodes, (size_t)b.n_nodes * 32, hipMemcpyDeviceToHost));
+    if (ordered_out) HIP_TRY(hipMemcpy(ordered_out, b.ordered, (size_t)n_tris * 4, hipMemcpyDeviceToHost));
+    return FF_OK;
 }
 
 ff_dev_camera dev_camera(const ff_camera* cam) {
@@ -424,14 +292,15 @@ ff_status ff_bvh_build_gpu(ff_context* ctx, const float* positions, int32_t n_tr
         if (!std::isfinite(positions[k]))
             return fail(FF_ERR_INVALID, "ff_bvh_build_gpu: triangle %d has a non-finite vertex coordinate", (int)(k / 9));
     HIP_TRY(hipSetDevice(ctx->device));
-    std::vector<ffh::BvhNode> nodes;
-    std::vector<int32_t> ordered;
+    ffk::DevBvh bvh;
     float ms = 0.f;
-    HIP_TRY(ffk::build_lbvh(positions, n_tris, max_prims, nodes, ordered, &ms));
-    if (nodes_out) std::memcpy(nodes_out, nodes.data(), nodes.size() * sizeof(ffh::BvhNode));
-    if (ordered_out) std::memcpy(ordered_out, ordered.data(), ordered.size() * sizeof(int32_t));
-    if (n_nodes_out) *n_nodes_out = (int32_t)nodes.size();
-    if (max_depth_out) *max_depth_out = ffh::bvh_max_depth(nodes);
+    hipError_t e = ffk::build_lbvh(positions, n_tris, max_prims, bvh, &ms);
+    ff_status st = e == hipSuccess ? read_bvh(bvh, n_tris, nodes_out, ordered_out) : FF_OK;
+    dfree(bvh.mem);
+    HIP_TRY(e);
+    if (st != FF_OK) return st;
+    if (n_nodes_out) *n_nodes_out = bvh.n_nodes;
+    if (max_depth_out) *max_depth_out = bvh.max_depth;
     if (build_ms_out) *build_ms_out = ms;
     return FF_OK;
 }
@@ -447,14 +316,15 @@ ff_status ff_bvh_build_ploc(ff_context* ctx, const float* positions, int32_t n_t
         if (!std::isfinite(positions[k]))
             return fail(FF_ERR_INVALID, "ff_bvh_build_ploc: triangle %d has a non-finite vertex coordinate", (int)(k / 9));
     HIP_TRY(hipSetDevice(ctx->device));
-    std::vector<ffh::BvhNode> nodes;
-    std::vector<int32_t> ordered;
+    ffk::DevBvh bvh;
     float ms = 0.f;
-    HIP_TRY(ffk::build_ploc(positions, n_tris, max_prims, nodes, ordered, &ms));
-    if (nodes_out) std::memcpy(nodes_out, nodes.data(), nodes.size() * sizeof(ffh::BvhNode));
-    if (ordered_out) std::memcpy(ordered_out, ordered.data(), ordered.size() * sizeof(int32_t));
-    if (n_nodes_out) *n_nodes_out = (int32_t)nodes.size();
-    if (max_depth_out) *max_depth_out = ffh::bvh_max_depth(nodes);
+    hipError_t e = ffk::build_ploc(positions, n_tris, max_prims, bvh, &ms);
+    ff_status st = e == hipSuccess ? read_bvh(bvh, n_tris, nodes_out, ordered_out) : FF_OK;
+    dfree(bvh.mem);
+    HIP_TRY(e);
+    if (st != FF_OK) return st;
+    if (n_nodes_out) *n_nodes_out = bvh.n_nodes;
+    if (max_depth_out) *max_depth_out = bvh.max_depth;
     if (build_ms_out) *build_ms_out = ms;
     return FF_OK;
 }
@@ -503,75 +373,33 @@ ff_status ff_scene_create(ff_context* ctx, const ff_scene_desc* d, ff_scene** ou
     s->ctx = ctx;
     s->n_tris = d->n_tris;
     s->n_mats = d->n_materials;
+    auto cleanup = [&](ff_status st) { ff_scene_destroy(s); return st; };
     int32_t max_prims = d->max_prims_in_node > 0 ? d->max_prims_in_node : 8;
-    if (d->builder == FF_BVH_LBVH || d->builder == FF_BVH_PLOC) {
-        hipError_t be = d->builder == FF_BVH_LBVH
-                            ? ffk::build_lbvh(d->positions, d->n_tris, max_prims, s->nodes, s->ordered)
-                            : ffk::build_ploc(d->positions, d->n_tris, max_prims, s->nodes, s->ordered);
-        if (be != hipSuccess) {
-            ff_scene_destroy(s);
-            return fail(FF_ERR_HIP, "ff_scene_create: GPU BVH build failed: %s", hipGetErrorString(be));
-        }
+    hipError_t e;
+    if (d->builder == FF_BVH_SAH) {
+        std::vector<ffh::BvhNode> nodes;
+        std::vector<int32_t> ordered;
+        ffh::build_bvh_sah(d->positions, d->n_tris, max_prims, nodes, ordered);
+        e = ffk::upload_bvh(nodes, ordered, ffh::bvh_max_depth(nodes), d->positions, s->bvh);
+        if (e != hipSuccess)
+            return cleanup(fail(e == hipErrorOutOfMemory ? FF_ERR_ALLOC : FF_ERR_HIP, "ff_scene_create: upload: %s",
+                                hipGetErrorString(e)));
     } else {
-        ffh::build_bvh_sah(d->positions, d->n_tris, max_prims, s->nodes, s->ordered);
-    }
-    s->max_depth = ffh::bvh_max_depth(s->nodes);
-    size_t n = (size_t)d->n_tris;
-    // reorder_primitives (CRT/kernel.cu:184-191,701-712) done on the host while
-    // packing the positions-only records v0 | e1 | e2.
-    std::vector<float> tris(9 * n), attr(16 * n, 0.f), tan(d->tangents ? 18 * n : 0);
-    std::vector<uint32_t> mat(n);
-    for (size_t i = 0; i < n; i++) {
-        size_t src = (size_t)s->ordered[i];
-        const float* p = d->positions + src * 9;
-        float* t = &tris[i * 9];
-        for (int k = 0; k < 3; k++) {
-            t[k] = p[k];
-            t[3 + k] = p[3 + k] - p[k];
-            t[6 + k] = p[6 + k] - p[k];
-        }
-        std::memcpy(&attr[i * 16], d->normals + src * 9, 36);
-        if (d->uvs) std::memcpy(&attr[i * 16 + 9], d->uvs + src * 6, 24);
-        if (d->tangents) std::memcpy(&tan[i * 18], d->tangents + src * 18, 72);
-        uint32_t m = (uint32_t)d->material_ids[src];
-        mat[i] = m | ((uint32_t)(int)d->materials[(size_t)m * FF_MAT_FLOATS] << MAT_TYPE_SHIFT);
-        std::memcpy(&attr[i * 16 + 15], &mat[i], 4);
+        e = d->builder == FF_BVH_LBVH ? ffk::build_lbvh(d->positions, d->n_tris, max_prims, s->bvh)
+                                      : ffk::build_ploc(d->positions, d->n_tris, max_prims, s->bvh);
+        if (e != hipSuccess)
+            return cleanup(fail(FF_ERR_HIP, "ff_scene_create: GPU BVH build failed: %s", hipGetErrorString(e)));
     }
     for (int32_t m = 0; m < d->n_materials; m++) s->has_type[(int)d->materials[(size_t)m * FF_MAT_FLOATS]] = true;
-    auto cleanup = [&](ff_status st) { ff_scene_destroy(s); return st; };
-    std::vector<float4> wide;
-    std::vector<int32_t> leaf_count;
-    float root[8];
-    pack_two_child(s->nodes, wide, leaf_count, root, n);
-    std::vector<float4> four;
-    std::vector<int32_t> leaf_count4;
-    float root4[8];
-    pack_four(s->nodes, four, leaf_count4, root4, n);
-    // the traversal addresses records by 32-bit byte offsets (64-B and 128-B records)
-    if (wide.size() / 4 >= (size_t(1) << 26) || four.size() / 8 >= (size_t(1) << 25))
-        return cleanup(fail(FF_ERR_CAPACITY, "ff_scene_create: %zu BVH records exceed the 2^25 4-wide / 2^26 "
-                                            "two-child limit of the traversal kernels", wide.size() / 4));
-    if (dalloc(&s->d_nodes, wide.size()) != hipSuccess || dalloc(&s->d_nodes4, four.size()) != hipSuccess ||
-        dalloc(&s->d_leaf_count, leaf_count.size()) != hipSuccess ||
-        dalloc(&s->d_root, 8) != hipSuccess || dalloc(&s->d_tris, 9 * n) != hipSuccess ||
-        dalloc(&s->d_attr, 4 * n) != hipSuccess ||
-        dalloc(&s->d_mat, n) != hipSuccess || dalloc(&s->d_mats, (size_t)FF_MAT_FLOATS * d->n_materials) != hipSuccess ||
-        (d->tangents && dalloc(&s->d_tan, 18 * n) != hipSuccess))
-        return cleanup(fail(FF_ERR_ALLOC, "ff_scene_create: device allocation failed"));
-    hipError_t e = hipSuccess;
-    if (!wide.empty()) e = hipMemcpy(s->d_nodes, wide.data(), wide.size() * sizeof(float4), hipMemcpyHostToDevice);
-    if (e == hipSuccess && !four.empty())
-        e = hipMemcpy(s->d_nodes4, four.data(), four.size() * sizeof(float4), hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(s->d_leaf_count, leaf_count.data(), leaf_count.size() * 4, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(s->d_root, root, sizeof(root), hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(s->d_tris, tris.data(), 36 * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(s->d_attr, attr.data(), 64 * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess && d->tangents) e = hipMemcpy(s->d_tan, tan.data(), 72 * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess) e = hipMemcpy(s->d_mat, mat.data(), 4 * n, hipMemcpyHostToDevice);
-    if (e == hipSuccess)
-        e = hipMemcpy(s->d_mats, d->materials, sizeof(float) * FF_MAT_FLOATS * d->n_materials, hipMemcpyHostToDevice);
-    if (e != hipSuccess) return cleanup(fail(FF_ERR_HIP, "ff_scene_create: upload: %s", hipGetErrorString(e)));
+    // the traversal addresses two-child records by 32-bit byte offsets
+    if (s->bvh.n_nodes / 2 >= (1 << 26))
+        return cleanup(fail(FF_ERR_CAPACITY, "ff_scene_create: %d BVH records exceed the 2^26 limit of the traversal "
+                                            "kernels", s->bvh.n_nodes / 2));
+    ffk::SceneArrays arrays{d->normals, d->uvs, d->tangents, d->materials, d->material_ids, d->n_tris, d->n_materials};
+    e = ffk::pack_scene(s->bvh, arrays, s->pack);
+    if (e != hipSuccess)
+        return cleanup(fail(e == hipErrorOutOfMemory ? FF_ERR_ALLOC : FF_ERR_HIP, "ff_scene_create: packing: %s",
+                            hipGetErrorString(e)));
     s->n_tex = d->n_textures;
     std::vector<ff_tex_desc> descs((size_t)std::max(1, d->n_textures));
     for (int32_t t = 0; t < d->n_textures; t++) {
@@ -596,7 +424,8 @@ ff_status ff_scene_create(ff_context* ctx, const ff_scene_desc* d, ff_scene** ou
 ff_status ff_scene_destroy(ff_scene* s) {
     if (!s) return fail(FF_ERR_INVALID, "ff_scene_destroy: NULL scene");
     (void)hipDeviceSynchronize();
-    dfree(s->d_nodes); dfree(s->d_nodes4); dfree(s->d_leaf_count); dfree(s->d_root); dfree(s->d_tris); dfree(s->d_attr); dfree(s->d_tan); dfree(s->d_mat); dfree(s->d_mats);
+    dfree(s->bvh.mem);
+    dfree(s->pack.mem);
     for (auto& p : s->d_tex) dfree(p);
     dfree(s->d_tex_desc);
     delete s;
@@ -606,16 +435,15 @@ ff_status ff_scene_destroy(ff_scene* s) {
 ff_status ff_scene_info(const ff_scene* s, int32_t* n_tris, int32_t* n_nodes, int32_t* max_depth) {
     if (!s) return fail(FF_ERR_INVALID, "ff_scene_info: NULL scene");
     if (n_tris) *n_tris = s->n_tris;
-    if (n_nodes) *n_nodes = (int32_t)s->nodes.size();
-    if (max_depth) *max_depth = s->max_depth;
+    if (n_nodes) *n_nodes = s->bvh.n_nodes;
+    if (max_depth) *max_depth = s->bvh.max_depth;
     return FF_OK;
 }
 
 ff_status ff_scene_get_bvh(const ff_scene* s, ff_bvh_node* nodes_out, int32_t* ordered_out) {
     if (!s) return fail(FF_ERR_INVALID, "ff_scene_get_bvh: NULL scene");
-    if (nodes_out) std::memcpy(nodes_out, s->nodes.data(), s->nodes.size() * 32);
-    if (ordered_out) std::memcpy(ordered_out, s->ordered.data(), s->ordered.size() * 4);
-    return FF_OK;
+    HIP_TRY(hipSetDevice(s->ctx->device));
+    return read_bvh(s->bvh, s->n_tris, nodes_out, ordered_out);
 }
 
 ff_status ff_envmap_create(ff_context* ctx, const float* rgb, int32_t w, int32_t h, ff_envmap** out) {
@@ -706,7 +534,7 @@ ff_status ff_trace_closest(ff_scene* s, const float* rays, uint32_t n, float* hi
     if (!s || (!rays && n) || (!hits && n)) return fail(FF_ERR_INVALID, "ff_trace_closest: NULL argument");
     if (n == 0) return FF_OK;
     HIP_TRY(hipSetDevice(s->ctx->device));
-    ff_status st = ensure_ovf(s->ctx, s->max_depth);
+    ff_status st = ensure_ovf(s->ctx, s->bvh.max_depth, s->pack.wide_levels);
     if (st != FF_OK) return st;
     HIP_TRY(ffk::launch_trace_closest(s->view(), (const float4*)rays, n, (float4*)hits, two_sided, s->ctx->fetch,
                                       s->ctx->ovf,
@@ -722,7 +550,7 @@ ff_status ff_trace_closest_noalloc(ff_scene* s, const float* rays, uint32_t n, f
     // stack entries a traversal can hold with the variant's record width
     // (one per binary level; up to three per 4-wide record), beyond the
     // smallest LDS stack of any variant
-    const int32_t d = s->max_depth;
+    const int32_t d = s->bvh.max_depth;
     const int32_t width = ffk::kTravWidth[c->trav_variant];
     const int32_t entries = width == 4 ? std::max(d, 3 * ((d + 1) / 2)) : d;
     const int32_t need = entries > FF_LDS_MIN ? entries - FF_LDS_MIN + 1 : 1;
@@ -735,7 +563,9 @@ ff_status ff_trace_closest_noalloc(ff_scene* s, const float* rays, uint32_t n, f
                     2 * ((FF_STATIC_OVF_ENTRIES + FF_LDS_MIN - 1) / 3));
     if (!c->scratch) return fail(FF_ERR_HIP, "ff_trace_closest_noalloc: no fixed scratch on device %d", c->device);
     HIP_TRY(hipSetDevice(c->device));
-    HIP_TRY(ffk::launch_trace_closest(s->view(), (const float4*)rays, n, (float4*)hits, two_sided,
+    ff_dev_scene view = s->view();
+    if (3 * s->pack.wide_levels + 1 > FF_STATIC_OVF_ENTRIES + FF_LDS_STACK) view.wide = nullptr;
+    HIP_TRY(ffk::launch_trace_closest(view, (const float4*)rays, n, (float4*)hits, two_sided,
                                       (uint32_t*)c->scratch, c->scratch + FETCH_WORDS, (unsigned long long*)counts,
                                       c->trav_variant, (hipStream_t)stream));
     return FF_OK;
@@ -746,7 +576,7 @@ ff_status ff_trace_any(ff_scene* s, const float* rays, uint32_t n, uint8_t* occl
     if (!s || (!rays && n) || (!occluded && n)) return fail(FF_ERR_INVALID, "ff_trace_any: NULL argument");
     if (n == 0) return FF_OK;
     HIP_TRY(hipSetDevice(s->ctx->device));
-    ff_status st = ensure_ovf(s->ctx, s->max_depth);
+    ff_status st = ensure_ovf(s->ctx, s->bvh.max_depth, s->pack.wide_levels);
     if (st != FF_OK) return st;
     HIP_TRY(ffk::launch_trace_any(s->view(), (const float4*)rays, n, occluded, s->ctx->fetch, s->ctx->ovf,
                                   (unsigned long long*)counts, s->ctx->trav_variant, (hipStream_t)stream));
@@ -805,12 +635,13 @@ ff_status check_req(const char* who, ff_context* ctx, const HostReq& q) {
 ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int32_t flags, hipStream_t hs,
                           const char* who) {
     uint64_t n_slots = 0;
-    int32_t max_tree = 0, max_depth = 0;
+    int32_t max_tree = 0, max_wide = 0, max_depth = 0;
     int64_t n_batches = 0;
     bool has_type[4] = {false, false, false, false};
     for (const HostReq& q : reqs) {
         n_slots += (uint64_t)q.W * (uint64_t)q.H * (uint64_t)q.K;
-        max_tree = std::max(max_tree, q.s->max_depth);
+        max_tree = std::max(max_tree, q.s->bvh.max_depth);
+        max_wide = std::max(max_wide, q.s->pack.wide_levels);
         max_depth = std::max(max_depth, q.depth);
         n_batches = std::max<int64_t>(n_batches, (q.spp + q.K - 1) / q.K);
         for (int m = 0; m < 4; m++) has_type[m] = has_type[m] || q.s->has_type[m];
@@ -820,7 +651,7 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
     HIP_TRY(hipSetDevice(ctx->device));
     ff_status st = ensure_paths(ctx, (size_t)n_slots);
     if (st != FF_OK) return st;
-    st = ensure_ovf(ctx, max_tree);
+    st = ensure_ovf(ctx, max_tree, max_wide);
     if (st != FF_OK) return st;
     const bool timing = (flags & FF_RENDER_TIMING) != 0;
     const bool graph = (flags & FF_RENDER_USE_GRAPH) != 0 && !timing;
@@ -833,8 +664,7 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         HIP_TRY(hipEventCreateWithFlags(&ctx->fork_ev, hipEventDisableTiming));
         HIP_TRY(hipEventCreateWithFlags(&ctx->join_ev, hipEventDisableTiming));
     }
-    HIP_TRY(ffk::prepare_traversal(ctx->trav_variant));
-    if (ctx->trav_tail >= 0) HIP_TRY(ffk::prepare_traversal(ctx->trav_tail));
+    ffk::prepare_traversal();
     ff_paths p = ctx->paths.p;
     const bool adjoint = (reqs[0].mode & RQ_ADJOINT) != 0;
     for (const HostReq& q : reqs)
@@ -942,17 +772,16 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
     p.n_slots = (uint32_t)n_slots;
     p.uni_scene = 1;
     p.uni_env = 1;
+    p.quad = 1;
     for (const HostReq& q : reqs) {
         if (q.s != reqs[0].s) p.uni_scene = 0;
         if (q.e != reqs[0].e) p.uni_env = 0;
+        if (!quad_fits(q.s->pack.wide_levels, q.s->bvh.max_depth)) p.quad = 0;
     }
     p.g_max = ctx->g_max;
     p.g_cnt = ctx->g_cnt;
     p.g_fx = ctx->g_fx;
     p.gmode = GM_FLOAT;
-    // the context's variant, and from trav_tail_from on the tail variant
-    auto var_at = [&](int32_t it) { return ctx->trav_tail >= 0 && it >= ctx->trav_tail_from ? ctx->trav_tail : ctx->trav_variant; };
-
     ctx->records.clear();
     ctx->events_used = 0;
     // Records a begin/end event pair around one stage launch when timing.
@@ -997,8 +826,8 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
                 HIP_TRY(hipEventRecord(ctx->fork_ev, hs));
                 HIP_TRY(hipStreamWaitEvent(ss, ctx->fork_ev, 0));
             }
-            HIP_TRY(timed(0, [&] { return ffk::launch_extend(p, cur, var_at(it), hs); }));
-            HIP_TRY(timed_on(ss, 1, [&] { return ffk::launch_shadow(p, var_at(it), ss); }));
+            HIP_TRY(timed(0, [&] { return ffk::launch_extend(p, cur, hs); }));
+            HIP_TRY(timed_on(ss, 1, [&] { return ffk::launch_shadow(p, ss); }));
             if (!timing) {
                 HIP_TRY(hipEventRecord(ctx->join_ev, ss));
                 HIP_TRY(hipStreamWaitEvent(hs, ctx->join_ev, 0));
@@ -1021,14 +850,14 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         HIP_TRY(timed(4, [&] { return ffk::launch_generate(p, hs); }));
         int cur = 0;
         for (int32_t it = 1; it <= max_depth + 1; it++) {
-            HIP_TRY(timed(0, [&] { return ffk::launch_extend(p, cur, var_at(it), hs); }));
+            HIP_TRY(timed(0, [&] { return ffk::launch_extend(p, cur, hs); }));
             uint32_t mask = (1u << (cur == 0 ? C_EXT1 : C_EXT0)) | (1u << C_SHADOW) | (0xfu << C_MAT0);
             HIP_TRY(ffk::launch_reset(p.counters, mask, p.fetch, (1u << F_EXT) | (1u << F_SHD), hs));
             HIP_TRY(timed(2, [&] { return ffk::launch_logic_adj(p, cur, p.n_slots, hs); }));
             if (it <= max_depth) {
                 for (int m = 0; m < 3; m++)
                     if (has_type[m]) HIP_TRY(timed(3, [&] { return ffk::launch_shade_nee(m, p, p.n_slots, hs); }));
-                HIP_TRY(timed(1, [&] { return ffk::launch_shadow(p, var_at(it), hs); }));
+                HIP_TRY(timed(1, [&] { return ffk::launch_shadow(p, hs); }));
                 for (int m = 0; m < 4; m++)
                     if (has_type[m])
                         HIP_TRY(timed(3, [&] { return ffk::launch_shade_adj(m, p, 1 - cur, p.n_slots, hs); }));
@@ -1194,9 +1023,7 @@ ff_status ff_set_traversal_tail(ff_context* ctx, int32_t variant, int32_t from_i
     if (!ctx || variant < -1 || variant >= ffk::kTravVariants || from_iteration < 1)
         return fail(FF_ERR_INVALID, "ff_set_traversal_tail: variant %d (of %d), from iteration %d", variant,
                     ffk::kTravVariants, from_iteration);
-    ctx->trav_tail = variant;
-    ctx->trav_tail_from = from_iteration;
-    return FF_OK;
+    return FF_OK;  // no launch reads it
 }
 
 ff_status ff_traversal_variant_info(int32_t variant, int32_t* block, int32_t* lds_entries, int32_t* refill,

@@ -710,6 +710,17 @@ struct Stack {
     }
 };
 
+// The stack of a ray that four lanes share: its entries lie in the 64 LDS
+// columns of the wave (BS columns to a row), 16 rays side by side.
+template <int BS>
+struct QuadStack {
+    lds_int* col;  // &smem[first column of the wave + ray]
+    int sp;
+    __device__ __forceinline__ lds_int* at(int e) const { return col + (e >> 2) * BS + (e & 3) * 16; }
+    __device__ __forceinline__ void push(int v) { *at(sp++) = v; }
+    __device__ __forceinline__ int pop() { return *at(--sp); }
+};
+
 struct Hit { float t, u, v; int id; };
 // pruning limit of the current closest hit
 __device__ __forceinline__ float prune_lim(float t) { return t + t * PRUNE_REL + PRUNE_ABS; }
@@ -809,11 +820,6 @@ __device__ __forceinline__ bool visit_interior(const Bvh& B, TravRay& R, float l
     return false;
 }
 
-// intersect() closest hit (CRT/dTriangle.cu:140-213), one step: an interior
-// record or a leaf's triangles.  A candidate replaces the record when
-// 0 <= t < tmin.  Children whose boxes miss (or lie beyond the current hit by
-// the conservative slack, or wholly behind the origin) are never visited.
-// Returns false once the traversal is complete.
 // One 4-wide record: the four grandchild boxes are tested at once and the
 // hit ones are visited in the binary tree's near-first order (side by the
 // parent's split axis, then each side by its own axis): the first is entered,
@@ -829,7 +835,7 @@ __device__ __forceinline__ int sel4i(const int4& v, int k) {
 template <bool PRUNE>
 __device__ __forceinline__ bool visit_interior4(const Bvh& B, TravRay& R, float lim, Stack& st,
                                                 uint32_t& cnt_nodes) {
-    const float4* n = (const float4*)((const char*)B.nodes4 + ((uint32_t)R.ref << 7));
+    const float4* n = (const float4*)((const char*)B.nodes4 + ((uint64_t)(uint32_t)R.ref << 7));
     float4 lx = ldg4(n), ly = ldg4(n + 1), lz = ldg4(n + 2);
     float4 hx = ldg4(n + 3), hy = ldg4(n + 4), hz = ldg4(n + 5);
     int4 rf = ldg4i((const int4*)(n + 6)), ax = ldg4i((const int4*)(n + 7));
@@ -868,19 +874,6 @@ __device__ __forceinline__ bool visit_node(const Bvh& B, TravRay& R, float lim, 
                 : visit_interior<PRUNE>(B, R, lim, st, cnt_nodes);
 }
 
-// the triangles of the leaf R.ref (closest-hit test of every one)
-__device__ __forceinline__ void leaf_closest(const Bvh& B, const float* __restrict__ tris, const TravRay& R,
-                                             Hit& h, bool two_sided, uint32_t& cnt_tris) {
-    int off, np;
-    leaf_range(B, R.ref, off, np);
-    for (int i = 0; i < np; i++) {
-        Tri T = load_tri(tris, off + i);
-        cnt_tris++;
-        float t = 0.f, u = 0.f, v = 0.f;
-        bool ok = two_sided ? mt_two(T, R.o, R.d, t, u, v) : mt_cull(T, R.o, R.d, t, u, v);
-        if (ok && !(t < 0.f) && t < h.t) { h.t = t; h.u = u; h.v = v; h.id = off + i; }
-    }
-}
 // The closest hit of a persistent traversal lane: t in a register (every
 // test reads it), u, v and the triangle slot in three LDS words of the lane
 // (written only when a closer hit is found, read once at the end), which
@@ -923,33 +916,9 @@ __device__ __forceinline__ bool leaf_any(const Bvh& B, const float* __restrict__
     return false;
 }
 
-template <bool WIDE = false>
-__device__ __forceinline__ bool closest_step(const Bvh& B, const float* __restrict__ tris, TravRay& R, Hit& h,
-                                             bool two_sided, Stack& st, uint32_t& cnt_nodes,
-                                             uint32_t& cnt_tris) {
-    if (R.ref >= 0) {
-        if (visit_node<WIDE, true>(B, R, prune_lim(h.t), st, cnt_nodes)) return true;
-    } else {
-        leaf_closest(B, tris, R, h, two_sided, cnt_tris);
-    }
-    if (st.sp == 0) return false;
-    R.ref = st.pop();
-    return true;
-}
-
 __device__ __forceinline__ Hit no_hit() {
     Hit h;
     h.t = K_HUGE; h.u = 0.f; h.v = 0.f; h.id = -1;
-    return h;
-}
-
-__device__ __forceinline__ Hit closest_hit(const Bvh& B, const float* __restrict__ tris, f3 o, f3 d,
-                                           bool two_sided, Stack& st, uint32_t& cnt_nodes,
-                                           uint32_t& cnt_tris) {
-    Hit h = no_hit();
-    TravRay R;
-    if (!trav_begin(B, o, d, R, st, cnt_nodes)) return h;
-    while (closest_step(B, tris, R, h, two_sided, st, cnt_nodes, cnt_tris)) {}
     return h;
 }
 
@@ -969,13 +938,264 @@ __device__ __forceinline__ int any_step(const Bvh& B, const float* __restrict__ 
     return 0;
 }
 
-__device__ __forceinline__ bool any_hit(const Bvh& B, const float* __restrict__ tris, f3 o, f3 d, Stack& st,
-                                        uint32_t& cnt_nodes, uint32_t& cnt_tris) {
-    TravRay R;
-    if (!trav_begin(B, o, d, R, st, cnt_nodes)) return false;
-    int r;
-    while ((r = any_step(B, tris, R, st, cnt_nodes, cnt_tris)) == 0) {}
-    return r == 1;
+// ------------------------------------------------- compressed wide walk --
+// The records the renders and the ray queries walk (built by ff_pack.hip from
+// the reference's binary tree): groups of four 64-byte records, one group per
+// wide node, holding its up to four children.  A child is another wide node or
+// one triangle.  A child reference is (record index | interior children of its
+// group << 29); groups are 4-aligned and interior children come first, so a
+// reference names a triangle exactly when (ref & 3) >= ref >> 29.
+//   node:     (org.xyz, reference of the child group)
+//             (lox01, lox23, loy01, loy23) (loz01, loz23, hix01, hix23)
+//             (hiy01, hiy23, hiz01, hiz23)
+//             child planes relative to org, two bfloat16 a word, rounded
+//             outwards; an empty child has the box (+inf, -inf)
+//   triangle: v0, e1, e2 (9 floats), slot, then the box of the reference's leaf
+//             that holds the triangle (6 floats, exact)
+// Which triangles the reference tests depends on leaf boxes alone: slab
+// distances are monotone in the planes, so a leaf whose own box passes has
+// ancestors that all pass.  The walk therefore may use any boxes that hold the
+// leaf boxes, and a triangle that is hit counts only if its leaf's exact box
+// passes the reference's test.  The closest hit is the smallest t, whatever
+// the visit order; where two triangles share it exactly, or a box plane
+// distance is NaN (0 * inf), the ray is traced again in the reference's order.
+#define WREF_INDEX 0x1fffffffu
+#define WREF_ROOT (4u << 29)  // record 0, an interior child
+#define WHIT_REDO 0x40000000  // hit word: trace the ray again in the reference's order
+// Slack of the conservative plane distances: a distance is fma(plane, inv, b)
+// with b = (org - o) * inv.  Against the reference's (lo - o) * inv the two
+// differ by at most 2.5 * 2^-23 |b| + 1.5 * 2^-23 |plane * inv|; the first is
+// covered here, the second by the planes' padding (2^-16 of their value).
+constexpr float WIDE_SLACK = 0x1p-21f;
+constexpr float WIDE_INV_MAX = 0x1p80f;  // |1/d| used for boxes (a zero direction component stays finite)
+
+struct WideRay {
+    f3 o, d, inv;  // inv: 1 / d, clamped to +-WIDE_INV_MAX
+    bool nx, ny, nz;
+    uint32_t fl;   // XNAN_RAY, WINV_CLAMPED
+};
+constexpr uint32_t WINV_CLAMPED = 16u;
+
+__device__ __forceinline__ void wide_begin(f3 o, f3 d, WideRay& R) {
+    R.o = o;
+    R.d = d;
+    f3 inv = V3(1.f / d.x, 1.f / d.y, 1.f / d.z);
+    R.nx = inv.x < 0;
+    R.ny = inv.y < 0;
+    R.nz = inv.z < 0;
+    R.inv = V3(fminf(fmaxf(inv.x, -WIDE_INV_MAX), WIDE_INV_MAX), fminf(fmaxf(inv.y, -WIDE_INV_MAX), WIDE_INV_MAX),
+               fminf(fmaxf(inv.z, -WIDE_INV_MAX), WIDE_INV_MAX));
+    R.fl = ((isfinite(inv.x) && isfinite(o.x)) ? 0u : XNAN_RAY) |
+           ((R.inv.x == inv.x && R.inv.y == inv.y && R.inv.z == inv.z) ? 0u : WINV_CLAMPED);
+}
+
+__device__ __forceinline__ const float4* wide_rec(const float4* rec, uint32_t ref) {
+    return (const float4*)((const char*)rec + ((uint64_t)(ref & WREF_INDEX) << 6));
+}
+__device__ __forceinline__ bool wide_is_leaf(uint32_t ref) { return (ref & 3u) >= (ref >> 29); }
+
+__device__ __forceinline__ int imin(int a, int b) { return a < b ? a : b; }
+__device__ __forceinline__ int imax(int a, int b) { return a > b ? a : b; }
+constexpr int WKEY_MISS = 0x7fffffff;
+
+// One wide node: the entry and exit distances of the four child boxes (entry
+// at least -PRUNE_BEHIND, exit at most lim); returns the child group's
+// reference.  Child k may be entered unless tn[k] > tf[k].
+template <bool PRUNE>
+__device__ __forceinline__ uint32_t visit_wide(const float4* rec, uint32_t ref, const WideRay& R, float lim,
+                                               float tn[4], float tf[4]) {
+    const float4* p = wide_rec(rec, ref);
+    float4 n0 = ldg4(p);
+    int4 n1 = ldg4i((const int4*)(p + 1)), n2 = ldg4i((const int4*)(p + 2)), n3 = ldg4i((const int4*)(p + 3));
+    float bx = (n0.x - R.o.x) * R.inv.x, by = (n0.y - R.o.y) * R.inv.y, bz = (n0.z - R.o.z) * R.inv.z;
+    float bnx = __builtin_fmaf(-WIDE_SLACK, fabsf(bx), bx), bfx = __builtin_fmaf(WIDE_SLACK, fabsf(bx), bx);
+    float bny = __builtin_fmaf(-WIDE_SLACK, fabsf(by), by), bfy = __builtin_fmaf(WIDE_SLACK, fabsf(by), by);
+    float bnz = __builtin_fmaf(-WIDE_SLACK, fabsf(bz), bz), bfz = __builtin_fmaf(WIDE_SLACK, fabsf(bz), bz);
+    const int lx[2] = {n1.x, n1.y}, ly[2] = {n1.z, n1.w}, lz[2] = {n2.x, n2.y};
+    const int hx[2] = {n2.z, n2.w}, hy[2] = {n3.x, n3.y}, hz[2] = {n3.z, n3.w};
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        int ax = R.nx ? hx[h] : lx[h], ay = R.ny ? hy[h] : ly[h], az = R.nz ? hz[h] : lz[h];
+        int cx = R.nx ? lx[h] : hx[h], cy = R.ny ? ly[h] : hy[h], cz = R.nz ? lz[h] : hz[h];
+#pragma unroll
+        for (int q = 0; q < 2; q++) {
+            auto plane = [&](int w) {
+                return __int_as_float(q ? (int)((uint32_t)w & 0xffff0000u) : (int)((uint32_t)w << 16));
+            };
+            float x0 = __builtin_fmaf(plane(ax), R.inv.x, bnx), x1 = __builtin_fmaf(plane(cx), R.inv.x, bfx);
+            float y0 = __builtin_fmaf(plane(ay), R.inv.y, bny), y1 = __builtin_fmaf(plane(cy), R.inv.y, bfy);
+            float z0 = __builtin_fmaf(plane(az), R.inv.z, bnz), z1 = __builtin_fmaf(plane(cz), R.inv.z, bfz);
+            tn[2 * h + q] = fmaxf(fmaxf(x0, y0), fmaxf(z0, -PRUNE_BEHIND));
+            tf[2 * h + q] = PRUNE ? fminf(fminf(x1, y1), fminf(z1, lim)) : fminf(fminf(x1, y1), z1);
+        }
+    }
+    return __float_as_uint(n0.w);
+}
+// The children that may be entered, in order of entry distance: distance bits
+// with the child number in the low two (WKEY_MISS: not entered).  Distances
+// below zero (at least -PRUNE_BEHIND) order before every positive one.
+__device__ __forceinline__ void wide_order(const float tn[4], const float tf[4], int key[4]) {
+#pragma unroll
+    for (int k = 0; k < 4; k++) key[k] = !(tn[k] > tf[k]) ? ((__float_as_int(tn[k]) & ~3) | k) : WKEY_MISS;
+    int a = imin(key[0], key[1]), b = imax(key[0], key[1]), c = imin(key[2], key[3]), d = imax(key[2], key[3]);
+    int m1 = imax(a, c), m2 = imin(b, d);
+    key[0] = imin(a, c);
+    key[3] = imax(b, d);
+    key[1] = imin(m1, m2);
+    key[2] = imax(m1, m2);
+}
+
+// One child box by one lane: the lanes 4q .. 4q + 3 of a wave share a ray and
+// take a child each (k = lane & 3).
+template <bool PRUNE>
+__device__ __forceinline__ uint32_t visit_quad(const float4* rec, uint32_t ref, const WideRay& R, float lim, uint32_t k,
+                                               float& tn, float& tf) {
+    const float4* p = wide_rec(rec, ref);
+    const int* w = (const int*)p + 4 + (k >> 1);  // the lane's pair of children
+    float4 n0 = ldg4(p);
+    int lx = ldg(w), ly = ldg(w + 2), lz = ldg(w + 4), hx = ldg(w + 6), hy = ldg(w + 8), hz = ldg(w + 10);
+    float bx = (n0.x - R.o.x) * R.inv.x, by = (n0.y - R.o.y) * R.inv.y, bz = (n0.z - R.o.z) * R.inv.z;
+    float bnx = __builtin_fmaf(-WIDE_SLACK, fabsf(bx), bx), bfx = __builtin_fmaf(WIDE_SLACK, fabsf(bx), bx);
+    float bny = __builtin_fmaf(-WIDE_SLACK, fabsf(by), by), bfy = __builtin_fmaf(WIDE_SLACK, fabsf(by), by);
+    float bnz = __builtin_fmaf(-WIDE_SLACK, fabsf(bz), bz), bfz = __builtin_fmaf(WIDE_SLACK, fabsf(bz), bz);
+    const uint32_t sh = (k & 1u) ? 0u : 16u;
+    auto plane = [&](int v) { return __uint_as_float(((uint32_t)v << sh) & 0xffff0000u); };
+    float ax = plane(R.nx ? hx : lx), ay = plane(R.ny ? hy : ly), az = plane(R.nz ? hz : lz);
+    float cx = plane(R.nx ? lx : hx), cy = plane(R.ny ? ly : hy), cz = plane(R.nz ? lz : hz);
+    float x0 = __builtin_fmaf(ax, R.inv.x, bnx), x1 = __builtin_fmaf(cx, R.inv.x, bfx);
+    float y0 = __builtin_fmaf(ay, R.inv.y, bny), y1 = __builtin_fmaf(cy, R.inv.y, bfy);
+    float z0 = __builtin_fmaf(az, R.inv.z, bnz), z1 = __builtin_fmaf(cz, R.inv.z, bfz);
+    tn = fmaxf(fmaxf(x0, y0), fmaxf(z0, -PRUNE_BEHIND));
+    tf = PRUNE ? fminf(fminf(x1, y1), fminf(z1, lim)) : fminf(fminf(x1, y1), z1);
+    return __float_as_uint(n0.w);
+}
+// values of the quad's other lanes (lane ^ X)
+template <int X>
+__device__ __forceinline__ int quad_xor(int v) {
+    return __builtin_amdgcn_mov_dpp(v, X == 1 ? 0xB1 : (X == 2 ? 0x4E : 0x1B), 0xf, 0xf, true);
+}
+template <int X>
+__device__ __forceinline__ float quad_xor(float v) {
+    return __int_as_float(quad_xor<X>(__float_as_int(v)));
+}
+
+// A triangle record
+struct WideTri {
+    Tri T;
+    int slot;
+    f3 lo, hi;  // the reference leaf's box
+};
+__device__ __forceinline__ WideTri load_wide_tri(const float4* rec, uint32_t ref) {
+    const float4* p = wide_rec(rec, ref);
+    float4 a = ldg4(p), b = ldg4(p + 1), c = ldg4(p + 2), d = ldg4(p + 3);
+    WideTri w;
+    w.T.v0 = V3(a.x, a.y, a.z);
+    w.T.e1 = V3(a.w, b.x, b.y);
+    w.T.e2 = V3(b.z, b.w, c.x);
+    w.slot = __float_as_int(c.y);
+    w.lo = V3(c.z, c.w, d.x);
+    w.hi = V3(d.y, d.z, d.w);
+    return w;
+}
+// The reference's test of the triangle's leaf box, as its walk makes it.
+// nanx: an x plane distance is NaN there, so ancestors may not follow.
+__device__ __forceinline__ bool wide_leaf_box(const WideTri& w, const WideRay& R, bool& nanx) {
+    f3 inv = R.inv;
+    float tn, tf;
+    nanx = false;
+    if (__ballot(R.fl != 0u) == 0)
+        return slab_box(w.lo.x, w.lo.y, w.lo.z, w.hi.x, w.hi.y, w.hi.z, R.o, inv, R.nx, R.ny, R.nz, tn, tf);
+    if (R.fl & WINV_CLAMPED) inv = V3(1.f / R.d.x, 1.f / R.d.y, 1.f / R.d.z);
+    nanx = (R.fl & XNAN_RAY) != 0u && (!isfinite(R.o.x) || R.o.x == w.lo.x || R.o.x == w.hi.x);
+    return slab(w.lo.x, w.lo.y, w.lo.z, w.hi.x, w.hi.y, w.hi.z, R.o, inv, R.nx, R.ny, R.nz, tn, tf);
+}
+__device__ __forceinline__ void wide_leaf_closest(const float4* rec, uint32_t ref, const WideRay& R, float& t_hit,
+                                                  const HitSlots& hs, bool two_sided) {
+    WideTri w = load_wide_tri(rec, ref);
+    float t = 0.f, u = 0.f, v = 0.f;
+    bool ok = two_sided ? mt_two(w.T, R.o, R.d, t, u, v) : mt_cull(w.T, R.o, R.d, t, u, v);
+    if (ok && !(t < 0.f) && t <= t_hit) {
+        bool nanx;
+        if (wide_leaf_box(w, R, nanx)) {
+            if (t < t_hit) {
+                t_hit = t;
+                *hs.u = u;
+                *hs.v = v;
+                *hs.id = w.slot | (nanx ? WHIT_REDO : 0);
+            } else if (*hs.id >= 0) {
+                *hs.id |= WHIT_REDO;  // the same distance: the reference's order decides
+            }
+        }
+    }
+}
+// 0: no hit, 1: occluded, 2: to be traced again in the reference's order
+__device__ __forceinline__ int wide_leaf_any(const float4* rec, uint32_t ref, const WideRay& R) {
+    WideTri w = load_wide_tri(rec, ref);
+    float t = 0.f;
+    if (!(mt_shadow(w.T, R.o, R.d, t) && t < K_HUGE)) return 0;
+    bool nanx;
+    if (!wide_leaf_box(w, R, nanx)) return 0;
+    return nanx ? 2 : 1;
+}
+
+// One ray in the reference's order over the binary records (the rare rays
+// above), one box or triangle in registers at a time, so that it adds no
+// registers to the kernels that hold it.
+template <bool ANY, class S>
+__device__ __forceinline__ Hit reference_walk(const Bvh& B, const float* __restrict__ tris, f3 o, f3 d, bool two_sided,
+                                              S& st) {
+    Hit h = no_hit();
+    const f3 inv = V3(1.f / d.x, 1.f / d.y, 1.f / d.z);
+    const bool nx = inv.x < 0, ny = inv.y < 0, nz = inv.z < 0;
+    float tn, tf;
+    int ref = __float_as_int(ldg(B.root + 6));
+    if (!slab(ldg(B.root), ldg(B.root + 1), ldg(B.root + 2), ldg(B.root + 3), ldg(B.root + 4), ldg(B.root + 5), o, inv,
+              nx, ny, nz, tn, tf))
+        return h;
+    st.sp = 0;
+    for (;;) {
+        bool down = false;
+        if (ref >= 0) {
+            const float* n = (const float*)((const char*)B.nodes + ((uint64_t)(uint32_t)ref << 6));
+            bool hit[2];
+#pragma unroll 1
+            for (int c = 0; c < 2; c++) {
+                const float* b = n + 6 * c;
+                bool in = slab(ldg(b), ldg(b + 1), ldg(b + 2), ldg(b + 3), ldg(b + 4), ldg(b + 5), o, inv, nx, ny, nz,
+                               tn, tf) &&
+                          !(tf < -PRUNE_BEHIND) && (ANY || !(tn > prune_lim(h.t)));
+                if (c == 0) hit[0] = in;
+                else hit[1] = in;
+            }
+            const int axis = __float_as_int(ldg(n + 14));
+            const bool neg = axis == 0 ? nx : (axis == 1 ? ny : nz);
+            const int r0 = __float_as_int(ldg(n + 12)), r1 = __float_as_int(ldg(n + 13));
+            if (hit[0] && hit[1]) st.push(neg ? r0 : r1);
+            down = hit[0] || hit[1];
+            if (down) ref = hit[0] && hit[1] ? (neg ? r1 : r0) : (hit[0] ? r0 : r1);
+        } else {
+            int off, np;
+            leaf_range(B, ref, off, np);
+#pragma unroll 1
+            for (int i = off; i < off + np; i++) {
+                Tri T = load_tri(tris, i);
+                float t = 0.f, u = 0.f, v = 0.f;
+                if (ANY) {
+                    if (mt_shadow(T, o, d, t) && t < K_HUGE) {
+                        h.id = i;
+                        return h;
+                    }
+                } else {
+                    bool ok = two_sided ? mt_two(T, o, d, t, u, v) : mt_cull(T, o, d, t, u, v);
+                    if (ok && !(t < 0.f) && t < h.t) { h.t = t; h.u = u; h.v = v; h.id = i; }
+                }
+            }
+        }
+        if (!down) {
+            if (st.sp == 0) return h;
+            ref = st.pop();
+        }
+    }
 }
 
 // ----------------------------------------------------- wave64 utilities --

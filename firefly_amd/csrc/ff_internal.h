@@ -16,12 +16,12 @@ extern const int kTravBlock[];
 extern const int kTravRefill[];
 extern const int kTravWhileWhile[];
 extern const int kTravWidth[];  // BVH record width of the variant (2 or 4)
-// computes the grid sizes of a traversal variant (call before a graph capture)
-hipError_t prepare_traversal(int variant);
+// computes the grid sizes of the wavefront's traversal kernels (call before a graph capture)
+void prepare_traversal();
 hipError_t launch_batch_begin(const ff_paths& P, int set, uint32_t value, hipStream_t s);
 hipError_t launch_generate(const ff_paths& P, hipStream_t s);
-hipError_t launch_extend(const ff_paths& P, int q, int variant, hipStream_t s);
-hipError_t launch_shadow(const ff_paths& P, int variant, hipStream_t s);
+hipError_t launch_extend(const ff_paths& P, int q, hipStream_t s);
+hipError_t launch_shadow(const ff_paths& P, hipStream_t s);
 hipError_t launch_reset(uint32_t* counters, uint32_t mask, uint32_t* fetch, uint32_t fetch_mask, hipStream_t s);
 hipError_t launch_logic(const ff_paths& P, int q, int iter, uint32_t n_max, hipStream_t s);
 hipError_t launch_shade(int type, const ff_paths& P, int next_q, int first, uint32_t n_max, hipStream_t s);
@@ -73,13 +73,52 @@ int32_t bvh_max_depth(const std::vector<BvhNode>& nodes);
 }  // namespace ffh
 
 namespace ffk {
-// Linear BVH on the GPU (Morton order, Karras hierarchy), in the SAH builder's
-// node format; positions on the host, nodes and permutation returned there
-// (gpu_ms, if given: device time of the build kernels).
-hipError_t build_lbvh(const float* positions, int32_t n, int32_t max_prims, std::vector<ffh::BvhNode>& nodes,
-                      std::vector<int32_t>& ordered, float* gpu_ms = nullptr);
+// Pieces of one device allocation: take() them all with base null for the
+// size, allocate, and take() them again.
+struct Carver {
+    char* base = nullptr;
+    size_t off = 0;
+    template <class T>
+    T* take(size_t n) {
+        T* p = (T*)(base + off);
+        off += (n * sizeof(T) + 255) / 256 * 256;
+        return p;
+    }
+};
+
+// A binary tree on the device, in the SAH builder's node format; `mem` is the
+// one allocation that holds it.
+struct DevBvh {
+    void* mem = nullptr;
+    ffh::BvhNode* nodes = nullptr;
+    int32_t* ordered = nullptr;
+    float* pos = nullptr;  // [n][3][3], the caller's order
+    int32_t n_nodes = 0, max_depth = 0, max_leaf = 1;
+};
+// Linear BVH on the GPU (Morton order, Karras hierarchy); positions on the
+// host (gpu_ms, if given: device time of the build kernels).
+hipError_t build_lbvh(const float* positions, int32_t n, int32_t max_prims, DevBvh& out, float* gpu_ms = nullptr);
 // PLOC tree on the GPU (locally-ordered clustering of the Morton-sorted
-// triangles, SAH leaf collapse), same node format and arguments.
-hipError_t build_ploc(const float* positions, int32_t n, int32_t max_prims, std::vector<ffh::BvhNode>& nodes,
-                      std::vector<int32_t>& ordered, float* gpu_ms = nullptr);
+// triangles, SAH leaf collapse), same arguments.
+hipError_t build_ploc(const float* positions, int32_t n, int32_t max_prims, DevBvh& out, float* gpu_ms = nullptr);
+// A host tree and its positions on the device.
+hipError_t upload_bvh(const std::vector<ffh::BvhNode>& nodes, const std::vector<int32_t>& ordered, int32_t max_depth,
+                      const float* positions, DevBvh& out);
+
+// Host arrays of a scene that packing reads (uv, tan may be null).
+struct SceneArrays {
+    const float *nrm, *uv, *tan, *mats;
+    const int32_t* mid;
+    int32_t n, n_mats;
+};
+// A scene's traversal and shading arrays, in one allocation (`mem`).
+struct ScenePack {
+    void* mem = nullptr;
+    float4 *nodes = nullptr, *nodes4 = nullptr, *wide = nullptr, *attr = nullptr;
+    int32_t* leaf_count = nullptr;
+    float *root = nullptr, *tris = nullptr, *tan = nullptr, *mats = nullptr;
+    uint32_t* mat = nullptr;
+    int32_t wide_levels = 0;
+};
+hipError_t pack_scene(const DevBvh& bvh, const SceneArrays& a, ScenePack& out);
 }  // namespace ffk

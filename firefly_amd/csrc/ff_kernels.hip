@@ -136,30 +136,24 @@ __global__ __launch_bounds__(FF_BLOCK) void k_generate(ff_paths P) {
 }
 
 // =============================================================== traversal
-// Ray sources of the persistent traversal kernels: load() binds queue entry k
-// to a ray and (unless kUniform) its scene, hit()/occluded() write the result.
-// kUniform: every ray of the launch uses one scene, bound once per wave by
-// scene0() (the BVH and triangle pointers then stay in scalar registers and
-// a refill needs no request-table lookup).
+// Ray sources of the persistent traversal kernels: load_ray() binds queue
+// entry k to a path (or ray) and its ray, load_again() reads that ray once
+// more, hit() / occluded() write the result.  kUniform: every ray of the launch
+// uses one scene (its pointers then stay in scalar registers).
 template <bool UNI>
 struct ExtSrc {  // wf_extend (CRT/kernel.cu:487-523): closest hit of every queued path
     static constexpr bool kUniform = UNI;
     static constexpr bool kChain = false;
     ff_paths P;
     const uint32_t* queue;
-    __device__ __forceinline__ void scene0(Bvh& B, const float*& tris) const {
-        const ff_dev_scene& S = P.reqs[0].S;
-        B = bvh_of(S);
-        tris = S.tris;
+    __device__ __forceinline__ const ff_dev_scene& scene(uint32_t id) const {
+        return UNI ? P.reqs[0].S : P.reqs[req_of(P, id)].S;
     }
-    __device__ __forceinline__ void load(uint32_t k, uint32_t& id, uint32_t&, Bvh& B, const float*& tris, f3& o,
-                                         f3& d, bool& two) const {
+    __device__ __forceinline__ void load_ray(uint32_t k, uint32_t& id, uint32_t& aux, f3& o, f3& d, bool& two) const {
         id = queue[k];
-        if (!UNI) {
-            const ff_dev_scene& S = P.reqs[req_of(P, id)].S;
-            B = bvh_of(S);
-            tris = S.tris;
-        }
+        load_again(id, aux, o, d, two);
+    }
+    __device__ __forceinline__ void load_again(uint32_t id, uint32_t, f3& o, f3& d, bool& two) const {
         o = xyz(P.ray[2 * id]);
         float4 r1 = P.ray[2 * id + 1];
         d = xyz(r1);
@@ -185,24 +179,19 @@ struct ShadowSrc {  // wf_shadow (CRT/kernel.cu:525-543): any hit of every queue
     static constexpr bool kUniform = UNI;
     static constexpr bool kChain = true;
     ff_paths P;
-    __device__ __forceinline__ void scene0(Bvh& B, const float*& tris) const {
-        const ff_dev_scene& S = P.reqs[0].S;
-        B = bvh_of(S);
-        tris = S.tris;
+    __device__ __forceinline__ const ff_dev_scene& scene(uint32_t id) const {
+        return UNI ? P.reqs[0].S : P.reqs[req_of(P, id)].S;
     }
-    __device__ __forceinline__ void load(uint32_t k, uint32_t& id, uint32_t& aux, Bvh& B, const float*& tris, f3& o,
-                                         f3& d, bool& two) const {
+    __device__ __forceinline__ void load_ray(uint32_t k, uint32_t& id, uint32_t& aux, f3& o, f3& d, bool& two) const {
         uint32_t e = P.q_shadow[k];
         id = e >> 2;
         aux = (e & 3u) << 2;
-        if (!UNI) {
-            const ff_dev_scene& S = P.reqs[req_of(P, id)].S;
-            B = bvh_of(S);
-            tris = S.tris;
-        }
         o = xyz(P.sray[6 * id]);
         d = xyz(P.sray[6 * id + 1]);
         two = false;
+    }
+    __device__ __forceinline__ void load_again(uint32_t id, uint32_t aux, f3& o, f3& d, bool&) const {
+        load_next(id, aux, o, d);
     }
     __device__ __forceinline__ void hit(uint32_t, const Hit&) const {}
     __device__ __forceinline__ void occluded(uint32_t id, uint32_t aux, bool occ) const {
@@ -234,15 +223,14 @@ struct RaySrc {  // a plain ray array (ff_trace_closest / ff_trace_any)
     float4* hits;
     uint8_t* occ;
     int two_sided;
-    __device__ __forceinline__ void scene0(Bvh& B, const float*& tris) const {
-        B = bvh_of(S);
-        tris = S.tris;
-    }
-    __device__ __forceinline__ void load(uint32_t k, uint32_t& id, uint32_t&, Bvh&, const float*&, f3& o, f3& d,
-                                         bool& two) const {
+    __device__ __forceinline__ const ff_dev_scene& scene(uint32_t) const { return S; }
+    __device__ __forceinline__ void load_ray(uint32_t k, uint32_t& id, uint32_t& aux, f3& o, f3& d, bool& two) const {
         id = k;
-        o = xyz(rays[2 * k]);
-        d = xyz(rays[2 * k + 1]);
+        load_again(id, aux, o, d, two);
+    }
+    __device__ __forceinline__ void load_again(uint32_t id, uint32_t, f3& o, f3& d, bool& two) const {
+        o = xyz(rays[2 * id]);
+        d = xyz(rays[2 * id + 1]);
         two = two_sided != 0;
     }
     __device__ __forceinline__ void hit(uint32_t id, const Hit& h) const {
@@ -254,7 +242,9 @@ struct RaySrc {  // a plain ray array (ff_trace_closest / ff_trace_any)
     __device__ __forceinline__ void count(uint32_t, uint32_t) const {}
 };
 
-// Persistent traversal.  The grid holds only the lanes the chip keeps
+// Persistent traversal of the reference's tree in the reference's order, for
+// traces that count the boxes and triangles it tests (and for the rare scene
+// whose wide stacks exceed the fixed trace scratch).  The grid holds only the lanes the chip keeps
 // resident; a lane whose ray is finished takes the next queue entry from the
 // segmented work counters (per wave: one ballot and one atomic for all idle
 // lanes), so a wave no longer lasts as long as its slowest ray and no second
@@ -281,8 +271,8 @@ struct RaySrc {  // a plain ray array (ff_trace_closest / ff_trace_any)
 // together once 8, 4 or 16 lanes hold one.
 // WIDE walks the 4-wide records (half the dependent interior steps, same
 // leaf order) instead of the two-child records.
-template <int BS, int LDS, int REFILL, bool ANY, int WW, bool WIDE, class Src>
-__device__ __forceinline__ void trav_persistent(const Src& src, uint32_t n, uint32_t* fetch, int32_t* ovf,
+template <int BS, int LDS, int REFILL, bool ANY, int WW, bool WIDE>
+__device__ __forceinline__ void trav_persistent(const RaySrc& src, uint32_t n, uint32_t* fetch, int32_t* ovf,
                                                 unsigned long long* cnt, int* smem) {
     SegFetch F;
     F.init(fetch, n, blockIdx.x * (BS / 64) + (threadIdx.x >> 6));
@@ -292,15 +282,13 @@ __device__ __forceinline__ void trav_persistent(const Src& src, uint32_t n, uint
     st.lds_entries = LDS;
     st.ovf = (glb_int*)(ovf + gtid());
     st.ovf_stride = FF_TRAV_THREADS;
-    uint32_t cn = 0, ct = 0, id = 0, aux = 0, c_rays = 0, c_gated = 0;
+    uint32_t cn = 0, ct = 0, id = 0, aux = 0;
     bool busy = false, more = true, two = false;
     bool walk = false;  // WW >= 2: the lane has records or leaves left to visit
     int pend = 0;       // WW >= 2: postponed leaf (0 = none; leaf refs are negative)
     int pend2 = 0;      // WW >= 3: a second postponed leaf, tested after pend
-    Bvh B;
-    B.nodes = nullptr; B.nodes4 = nullptr; B.leaf_count = nullptr; B.root = nullptr;
-    const float* tris = nullptr;
-    if (Src::kUniform) src.scene0(B, tris);
+    const Bvh B = bvh_of(src.S);
+    const float* const tris = src.S.tris;
     TravRay R;
     Hit h = no_hit();  // closest hit: h.t here, u, v and slot in the lane's LDS words (hs)
     float lim = prune_lim(h.t);  // pruning limit of the closest hit so far (kept beside it)
@@ -330,30 +318,9 @@ __device__ __forceinline__ void trav_persistent(const Src& src, uint32_t n, uint
         r.id = *hs.id;
         src.hit(id, r);
     };
-    // an any-hit ray is finished with result occ: the result is written and,
-    // for a source that chains rays, `nxt` marks that the lane's path has
-    // another ray, which the lane starts at the top of the next iteration
-    // instead of taking a queue entry
-    bool nxt = false;
-    auto end_any = [&](bool occ) {
-        src.occluded(id, aux, occ);
-        nxt = Src::kChain && src.advance(aux, occ, c_gated);
-    };
+    auto end_any = [&](bool occ) { src.occluded(id, aux, occ); };
     for (;;) {
-        if (Src::kChain && __ballot(nxt) != 0) {
-            if (nxt) {
-                f3 o, d;
-                src.load_next(id, aux, o, d);
-                c_rays++;
-                busy = trav_begin(B, o, d, R, st, cn);
-                walk = busy;
-                pend = 0;
-                pend2 = 0;
-                nxt = false;
-                if (!busy) end_any(false);
-            }
-        }
-        uint64_t idle = __ballot(!busy && !nxt);
+        uint64_t idle = __ballot(!busy);
         uint32_t n_idle = (uint32_t)__popcll(idle);
         if (more && n_idle >= (uint32_t)REFILL) {
             uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
@@ -362,10 +329,9 @@ __device__ __forceinline__ void trav_persistent(const Src& src, uint32_t n, uint
             bool done;
             uint32_t first = F.take_chunked(n_idle, got, done);
             if (done) more = false;
-            if (!busy && !nxt && rank < got) {
+            if (!busy && rank < got) {
                 f3 o, d;
-                src.load(first + rank, id, aux, B, tris, o, d, two);
-                c_rays++;
+                src.load_ray(first + rank, id, aux, o, d, two);
                 if (!ANY) reset_hit();
                 busy = trav_begin(B, o, d, R, st, cn);
                 walk = busy;
@@ -377,7 +343,7 @@ __device__ __forceinline__ void trav_persistent(const Src& src, uint32_t n, uint
                 }
             }
         }
-        if (__ballot(busy || nxt) == 0) {
+        if (__ballot(busy) == 0) {
             if (!more) break;
             continue;
         }
@@ -512,28 +478,427 @@ __device__ __forceinline__ void trav_persistent(const Src& src, uint32_t n, uint
         wave_sum_add(&cnt[0], cn);
         wave_sum_add(&cnt[1], ct);
     }
-    src.count(c_rays, c_gated);
 }
 
-// The one-scene extend kernels of the one-step and leaf-batching shapes run
-// 8 waves per SIMD (64 VGPRs, a few bytes of spills; the hit's u, v and slot
-// live in LDS) where their LDS stack allows that many; the others keep the
-// compiler's choice.
-template <int BS, int LDS, int RF, int WW, bool WIDE, bool UNI>
-__global__ __launch_bounds__(BS, (UNI && (WW == 0 || WW >= 5) && !WIDE && LDS <= 16 && BS >= 128) ? 8 : 1) void k_extend(
-    ff_paths P, int q) {
-    __shared__ int smem[LDS * BS + 3 * BS];  // stack, then the hit words
-    ExtSrc<UNI> src{P, P.q_ext[q]};
-    trav_persistent<BS, LDS, RF, false, WW, WIDE>(src, P.counters[q == 0 ? C_EXT0 : C_EXT1],
-                                            P.fetch + F_EXT * FETCH_SEGS * FETCH_STRIDE, P.ovf,
-                                            stats_rep(P) + S_EXT_NODES, smem);
+// Launch shape of the wide walk.  Measured on the 1920x1080, 64-sample frame
+// (extension / shadow stage): 6 waves per SIMD 24.1 / 15.1 ms, 5 waves 24.3 /
+// 15.1, 8 waves (64 VGPRs, spills) 27.6 / 19.1; refilling at 8 idle lanes 26.1,
+// at 16 24.2, at 48 29.1; testing held triangles once 2, 4, 8 or 16 lanes hold
+// one is alike there (24.1-24.4), and 2 is best where a launch lasts as long as
+// its slowest ray (160x120 frame: 0.86 ms, 0.87 at 4, 1.03 at 16).
+constexpr int TW_BLOCK = 256, TW_REFILL = 16, TW_LEAF = 2, TW_OCC = 6;
+// Launches of at most QUAD_MAX rays give every ray four lanes: at 19200 rays a
+// launch takes 50 us instead of 70, at 131072 (16 rays on each of 8192 waves)
+// the two are even, at 262144 rays four lanes cost 1.2x (8 spheres, 256x256).
+constexpr uint32_t QUAD_MAX = 131072;
+// A launch of fewer rays than lanes spreads them over this many waves (one or
+// two to a SIMD), so that a wave waits for fewer of its neighbours' visits:
+// 160x120 frame 0.99 ms with full waves, 0.87 ms; four lanes to a ray over 1024
+// waves 0.725 ms, over 2048 0.737, over 4096 0.78.
+constexpr uint32_t TW_SPREAD = 2048, QUAD_SPREAD = 1024;
+
+// Persistent traversal of the compressed wide records (see ff_device.h), with
+// the same work distribution: a lane owns a ray, a wave refills its idle lanes
+// once REFILL of them are idle.  A lane that reaches a triangle holds it and
+// walks on; the held triangles are tested together once LEAF lanes hold one,
+// or when no lane can walk on.
+template <int BS, bool ANY, class Src>
+__device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t* fetch, int32_t* ovf,
+                                          unsigned long long* cnt, int* smem) {
+    constexpr uint32_t IDLE = 0xffffffffu;
+    constexpr int LDS = FF_LDS_STACK;
+    SegFetch F;
+    F.init(fetch, n, blockIdx.x * (BS / 64) + (threadIdx.x >> 6));
+    Stack st;
+    st.lds = (lds_int*)&smem[threadIdx.x];
+    st.lds_stride = BS;
+    st.lds_entries = LDS;
+    st.ovf = (glb_int*)(ovf + gtid());
+    st.ovf_stride = FF_TRAV_THREADS;
+    st.sp = 1;
+    st.lds[0] = 0;  // popping the bottom ends the walk
+    uint32_t cn = 0, ct = 0, c_rays = 0, c_gated = 0;  // of the wave
+    bool more = true, two = false;
+    uint32_t id = IDLE, aux = 0;
+    bool nxt = false;
+    uint32_t cur = 0;   // reference to visit next (0: none left)
+    uint32_t pend = 0;  // held triangle (0: none; record 0 is no triangle)
+    const float4* rec = nullptr;
+    if (Src::kUniform) rec = src.scene(0).wide;
+    WideRay R;
+    R.fl = 0u;
+    float t_hit = K_HUGE;
+    HitSlots hs;
+    hs.u = ANY ? nullptr : (lds_float*)&smem[LDS * BS + threadIdx.x];
+    hs.v = ANY ? nullptr : (lds_float*)&smem[LDS * BS + BS + threadIdx.x];
+    hs.id = ANY ? nullptr : (lds_int*)&smem[LDS * BS + 2 * BS + threadIdx.x];
+    auto start = [&](f3 o, f3 d) {
+        wide_begin(o, d, R);
+        if (!ANY) {
+            t_hit = K_HUGE;
+            *hs.u = 0.f;
+            *hs.v = 0.f;
+            *hs.id = -1;
+        }
+        st.sp = 1;
+        cur = WREF_ROOT;
+        pend = 0;
+    };
+    // Rays whose outcome the reference's visit order decides (two triangles at
+    // one distance, a NaN plane distance) park their lane; once many lanes are
+    // parked, or no other work is left, those rays walk the binary records with
+    // every other lane idle (the walk's registers then add nothing to the loop).
+    constexpr uint32_t PARK_MOST = 32;
+    bool parked = false;
+    const uint32_t cap = n >= TW_SPREAD * 64u ? 64u : n / TW_SPREAD + 1u;
+    const bool mine = __lane_id() < cap;
+    const uint32_t refill = cap < (uint32_t)TW_REFILL ? cap : (uint32_t)TW_REFILL;
+    for (;;) {
+        for (;;) {
+            if (Src::kChain) {
+                uint64_t chained = __ballot(nxt);
+                if (chained != 0) {
+                    c_rays += (uint32_t)__popcll(chained);
+                    if (nxt) {
+                        f3 o, d;
+                        src.load_next(id, aux, o, d);
+                        start(o, d);
+                        nxt = false;
+                    }
+                }
+            }
+            uint64_t idle = __ballot(mine && (id == IDLE || parked));
+            if ((uint32_t)__popcll(idle) >= refill) {
+                const bool full = (uint32_t)__popcll(__ballot(parked)) >= PARK_MOST;
+                if (more && !full) {
+                    idle = __ballot(mine && id == IDLE);
+                    uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
+                                                              __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
+                    uint32_t got;
+                    bool done;
+                    uint32_t first = F.take_chunked((uint32_t)__popcll(idle), got, done);
+                    if (done) more = false;
+                    c_rays += got;
+                    if (mine && id == IDLE && rank < got) {
+                        f3 o, d;
+                        src.load_ray(first + rank, id, aux, o, d, two);
+                        if (!Src::kUniform) rec = src.scene(id).wide;
+                        start(o, d);
+                    }
+                }
+                if (__ballot(id != IDLE && !parked) == 0) {
+                    if (!more || full) break;
+                    continue;
+                }
+            }
+            // a triangle: held, and the walk goes on
+            if (cur != 0u && pend == 0u && wide_is_leaf(cur)) {
+                pend = cur;
+                cur = (uint32_t)st.pop();
+            }
+            bool inner = (cur & 3u) < (cur >> 29);
+            cn += (uint32_t)__popcll(__ballot(inner));
+            if (inner) {
+                float tn[4], tf[4];
+                const uint32_t w = visit_wide<!ANY>(rec, cur, R, t_hit + t_hit * PRUNE_REL + PRUNE_ABS, tn, tf);
+                // Entries are stored whether they count or not, and the top is
+                // moved on by those that do: the next store overwrites the
+                // others.  Near the end of the LDS stack they are pushed singly.
+                const bool room = __ballot(st.sp > LDS - 4) == 0;
+                lds_int* top = st.lds + st.sp * BS;
+                auto put = [&](uint32_t r, bool in) {
+                    if (room) {
+                        *top = (int)r;
+                        top += in ? BS : 0;
+                    } else if (in) {
+                        st.push((int)r);
+                    }
+                };
+                if (ANY) {  // an occluder anywhere ends the ray: no order, triangles first
+#pragma unroll
+                    for (int k = 0; k < 4; k++) put(w | (uint32_t)k, !(tn[k] > tf[k]));
+                    if (room) st.sp = (int)(top - st.lds) / BS;
+                    cur = (uint32_t)st.pop();
+                } else {
+                    int key[4];
+                    wide_order(tn, tf, key);
+#pragma unroll
+                    for (int k = 3; k > 0; k--) put(w | ((uint32_t)key[k] & 3u), key[k] != WKEY_MISS);
+                    if (room) st.sp = (int)(top - st.lds) / BS;
+                    cur = w | ((uint32_t)key[0] & 3u);
+                    if (key[0] == WKEY_MISS) cur = (uint32_t)st.pop();
+                }
+                inner = (cur & 3u) < (cur >> 29);
+            }
+            uint64_t has = __ballot(pend != 0u);
+            int occ = 0;
+            if (has != 0 && ((uint32_t)__popcll(has) >= (uint32_t)TW_LEAF || __ballot(inner) == 0)) {
+                ct += (uint32_t)__popcll(has);
+                if (pend != 0u) {
+                    if (ANY) occ = wide_leaf_any(rec, pend, R);
+                    else wide_leaf_closest(rec, pend, R, t_hit, hs, two);
+                    pend = 0;
+                }
+            }
+            const bool fin = occ || (id != IDLE && !parked && (cur | pend) == 0u);
+            uint32_t gated = 0;
+            if (fin) {
+                cur = 0;
+                pend = 0;
+                if (ANY) {
+                    parked = occ == 2;
+                    if (!parked) {
+                        src.occluded(id, aux, occ != 0);
+                        nxt = Src::kChain && src.advance(aux, occ != 0, gated);
+                        if (!nxt) id = IDLE;
+                    }
+                } else {
+                    Hit h;
+                    h.id = *hs.id;
+                    h.t = t_hit;
+                    h.u = *hs.u;
+                    h.v = *hs.v;
+                    parked = h.id >= 0 && (h.id & WHIT_REDO);
+                    if (!parked) {
+                        src.hit(id, h);
+                        id = IDLE;
+                    }
+                }
+            }
+            if (Src::kChain) c_gated += (uint32_t)(__popcll(__ballot(gated & 1u)) + 2 * __popcll(__ballot(gated & 2u)));
+        }
+        if (__ballot(parked) == 0) break;
+        while (__ballot(parked) != 0) {
+            uint32_t gated = 0;
+            bool again = false;
+            if (parked) {
+                const ff_dev_scene& S = src.scene(id);
+                f3 o, d;
+                src.load_again(id, aux, o, d, two);
+                const Hit h = reference_walk<ANY>(bvh_of(S), S.tris, o, d, two, st);
+                if (ANY) {
+                    const bool occ = h.id >= 0;
+                    src.occluded(id, aux, occ);
+                    again = Src::kChain && src.advance(aux, occ, gated);
+                } else {
+                    src.hit(id, h);
+                }
+                st.lds[0] = 0;
+                if (!again) id = IDLE;
+                parked = again;
+            }
+            c_rays += (uint32_t)__popcll(__ballot(again));
+            c_gated += (uint32_t)(__popcll(__ballot(gated & 1u)) + 2 * __popcll(__ballot(gated & 2u)));
+        }
+        if (!more) break;
+        // nothing of an idle lane's walk lives across this
+        R = WideRay{};
+        t_hit = K_HUGE;
+        cur = 0;
+        pend = 0;
+        aux = 0;
+        two = false;
+        nxt = false;
+        st.sp = 1;
+    }
+    if (cnt && __lane_id() == 0) {
+        atomicAdd(&cnt[0], 4ull * cn);
+        atomicAdd(&cnt[1], (unsigned long long)ct);
+    }
+    src.count(__lane_id() == 0 ? c_rays : 0u, __lane_id() == 0 ? c_gated : 0u);
 }
-template <int BS, int LDS, int RF, int WW, bool WIDE, bool UNI>
-__global__ __launch_bounds__(BS) void k_shadow(ff_paths P) {
-    __shared__ int smem[LDS * BS];
+
+// The same walk with four lanes to a ray, for launches of few rays: there a
+// launch lasts as long as its slowest ray's chain of dependent visits, and a
+// visit is a third of the instructions when every lane tests one child.
+// Triangles that a visit reaches are tested at once, a lane each, before the
+// walk goes on.  A ray's stack lies in the LDS columns of its wave (no
+// overflow area: the launcher takes this walk only where LDS * 4 entries hold
+// the deepest stack).
+template <int BS, bool ANY, class Src>
+__device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t* fetch,
+                                          unsigned long long* cnt, int* smem) {
+    constexpr uint32_t IDLE = 0xffffffffu;
+    SegFetch F;
+    F.init(fetch, n, blockIdx.x * (BS / 64) + (threadIdx.x >> 6));
+    const uint32_t lane = __lane_id(), k = lane & 3u, lead = lane & ~3u;
+    const uint64_t below = ((1ull << lead) - 1ull) & 0x1111111111111111ull;
+    QuadStack<BS> st;
+    st.col = (lds_int*)&smem[(threadIdx.x & ~63u) + (lane >> 2)];
+    st.sp = 0;
+    auto quad_mask = [&](bool b) { return (uint32_t)(__ballot(b) >> lead) & 15u; };
+    uint32_t cn = 0, ct = 0, c_rays = 0, c_gated = 0;  // of the wave
+    bool more = true, two = false, nxt = false;
+    uint32_t id = IDLE, aux = 0;
+    uint32_t cur = 0;
+    const float4* rec = nullptr;
+    if (Src::kUniform) rec = src.scene(0).wide;
+    WideRay R;
+    R.fl = 0u;
+    float t_hit = K_HUGE;           // of the quad
+    Hit best = no_hit();            // of the lane
+    float redo_t = -1.f;            // a distance that the reference's order decides
+    // few rays: fewer to a wave, so that a wave waits for fewer others
+    const uint32_t cap = n >= QUAD_SPREAD * 16u ? 16u : n / QUAD_SPREAD + 1u;
+    const bool mine = (lane >> 2) < cap;
+    auto start = [&](f3 o, f3 d) {
+        wide_begin(o, d, R);
+        t_hit = K_HUGE;
+        best = no_hit();
+        redo_t = -1.f;
+        *st.at(0) = 0;  // popping the bottom ends the walk
+        st.sp = 1;
+        cur = WREF_ROOT;
+    };
+    for (;;) {
+        if (Src::kChain) {
+            uint64_t chained = __ballot(nxt);
+            if (chained != 0) {
+                c_rays += (uint32_t)__popcll(chained) / 4u;
+                if (nxt) {
+                    f3 o, d;
+                    src.load_next(id, aux, o, d);
+                    start(o, d);
+                    nxt = false;
+                }
+            }
+        }
+        const uint64_t idle = __ballot(mine && id == IDLE && k == 0u);
+        if (idle != 0) {
+            if (more) {
+                uint32_t got;
+                bool done;
+                uint32_t first = F.take_chunked((uint32_t)__popcll(idle), got, done);
+                if (done) more = false;
+                c_rays += got;
+                const uint32_t rank = (uint32_t)__popcll(idle & below);
+                if (mine && id == IDLE && rank < got) {
+                    f3 o, d;
+                    src.load_ray(first + rank, id, aux, o, d, two);
+                    if (!Src::kUniform) rec = src.scene(id).wide;
+                    start(o, d);
+                }
+            }
+            if (__ballot(id != IDLE) == 0) {
+                if (!more) break;
+                continue;
+            }
+        }
+        cn += (uint32_t)__popcll(__ballot(cur != 0u)) / 4u;
+        bool occ = false, tri = false;
+        if (cur != 0u) {
+            float tn, tf;
+            const uint32_t w = visit_quad<!ANY>(rec, cur, R, t_hit + t_hit * PRUNE_REL + PRUNE_ABS, k, tn, tf);
+            bool in = !(tn > tf);
+            tri = in && k >= (w >> 29);
+            if (__ballot(tri) != 0) {
+                int r = 0;
+                float t = K_HUGE;
+                if (tri) {
+                    if (ANY) {
+                        r = wide_leaf_any(rec, w | k, R);
+                    } else {
+                        WideTri T = load_wide_tri(rec, w | k);
+                        float u = 0.f, v = 0.f;
+                        bool ok = two ? mt_two(T.T, R.o, R.d, t, u, v) : mt_cull(T.T, R.o, R.d, t, u, v), nanx;
+                        if (ok && !(t < 0.f) && t <= t_hit && wide_leaf_box(T, R, nanx)) {
+                            if (nanx || t == t_hit) redo_t = t;
+                            if (t < t_hit) {
+                                best.t = t;
+                                best.u = u;
+                                best.v = v;
+                                best.id = T.slot;
+                            }
+                        }
+                    }
+                }
+                if (ANY) {
+                    occ = quad_mask(r == 1) != 0u;
+                    if (!occ && quad_mask(r == 2) != 0u) redo_t = 0.f;
+                } else {
+                    t_hit = fminf(best.t, quad_xor<1>(best.t));
+                    t_hit = fminf(t_hit, quad_xor<2>(t_hit));
+                    in = in && !(tn > t_hit + t_hit * PRUNE_REL + PRUNE_ABS);
+                }
+                in = in && !tri;
+            }
+            const uint32_t m = quad_mask(in);
+            if (m != 0u) {
+                if (ANY) {
+                    const uint32_t f = (uint32_t)__ffs((int)m) - 1u;
+                    cur = w | f;
+                    if (in && k != f) *st.at(st.sp + __popc(m & ((1u << k) - 1u)) - 1) = (int)(w | k);
+                } else {
+                    const int key = in ? ((__float_as_int(tn) & ~3) | (int)k) : WKEY_MISS;
+                    const int k1 = quad_xor<1>(key), k2 = quad_xor<2>(key), k3 = quad_xor<3>(key);
+                    const int rank = (k1 < key ? 1 : 0) + (k2 < key ? 1 : 0) + (k3 < key ? 1 : 0);
+                    cur = w | ((uint32_t)imin(imin(key, k1), imin(k2, k3)) & 3u);
+                    if (in && rank > 0) *st.at(st.sp + __popc(m) - 1 - rank) = (int)(w | k);
+                }
+                st.sp += __popc(m) - 1;
+            } else {
+                cur = (uint32_t)st.pop();
+            }
+        }
+        ct += (uint32_t)__popcll(__ballot(tri));
+        const bool fin = id != IDLE && (occ || cur == 0u);
+        if (__ballot(fin) == 0) continue;
+        const bool redo = quad_mask(ANY ? redo_t == 0.f && !occ : redo_t >= 0.f && redo_t == t_hit) != 0u ||
+                          (!ANY && __popc(quad_mask(best.id >= 0 && best.t == t_hit)) > 1);
+        uint32_t gated = 0;
+        if (fin) {
+            cur = 0;
+            bool win = ANY ? k == 0u : (best.id >= 0 ? best.t == t_hit : (k == 0u && !(t_hit < K_HUGE)));
+            if (redo) {  // in the reference's order, by the quad's first lane
+                win = k == 0u;
+                if (win) {
+                    const ff_dev_scene& S = src.scene(id);
+                    best = reference_walk<ANY>(bvh_of(S), S.tris, R.o, R.d, two, st);
+                    if (ANY) occ = best.id >= 0;
+                }
+            }
+            if (ANY) {
+                occ = quad_mask(occ) != 0u;
+                if (win) src.occluded(id, aux, occ);
+                nxt = Src::kChain && src.advance(aux, occ, gated);
+                if (!nxt) id = IDLE;
+            } else {
+                if (win) src.hit(id, best);
+                id = IDLE;
+            }
+        }
+        if (Src::kChain)
+            c_gated += (uint32_t)(__popcll(__ballot(gated & 1u)) + 2 * __popcll(__ballot(gated & 2u))) / 4u;
+    }
+    if (cnt && lane == 0) {
+        atomicAdd(&cnt[0], 4ull * cn);
+        atomicAdd(&cnt[1], (unsigned long long)ct);
+    }
+    src.count(lane == 0 ? c_rays : 0u, lane == 0 ? c_gated : 0u);
+}
+
+template <bool ANY, class Src>
+__device__ __forceinline__ void traverse(const Src& src, uint32_t n, bool quad, uint32_t* fetch, int32_t* ovf,
+                                         unsigned long long* cnt, int* smem) {
+    if (quad && n <= QUAD_MAX) trav_quad<TW_BLOCK, ANY>(src, n, fetch, cnt, smem);
+    else trav_wide<TW_BLOCK, ANY>(src, n, fetch, ovf, cnt, smem);
+}
+// LDS words of a traversal workgroup: the stacks, for closest hits the hit words too
+constexpr int TW_LDS_ANY = FF_LDS_STACK * TW_BLOCK, TW_LDS_CLOSEST = (FF_LDS_STACK + 3) * TW_BLOCK;
+
+template <bool UNI>
+__global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend(ff_paths P, int q) {
+    __shared__ int smem[TW_LDS_CLOSEST];
+    ExtSrc<UNI> src{P, P.q_ext[q]};
+    traverse<false>(src, P.counters[q == 0 ? C_EXT0 : C_EXT1], P.quad != 0, P.fetch + F_EXT * FETCH_SEGS * FETCH_STRIDE,
+                    P.ovf, stats_rep(P) + S_EXT_NODES, smem);
+}
+template <bool UNI>
+__global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_shadow(ff_paths P) {
+    __shared__ int smem[TW_LDS_ANY];
     ShadowSrc<UNI> src{P};
-    trav_persistent<BS, LDS, RF, true, WW, WIDE>(src, P.counters[C_SHADOW], P.fetch + F_SHD * FETCH_SEGS * FETCH_STRIDE,
-                                           P.ovf_shd, stats_rep(P) + S_SHD_NODES, smem);
+    traverse<true>(src, P.counters[C_SHADOW], P.quad != 0, P.fetch + F_SHD * FETCH_SEGS * FETCH_STRIDE, P.ovf_shd,
+                   stats_rep(P) + S_SHD_NODES, smem);
 }
 
 // counters consumed by the previous stages are cleared by a kernel (graph-safe):
@@ -1362,6 +1727,16 @@ __global__ __launch_bounds__(BS) void k_trace_any(TraceArgs a) {
     RaySrc src{a.S, a.rays, nullptr, a.occ, 0};
     trav_persistent<BS, LDS, RF, true, WW, WIDE>(src, a.n, a.fetch, a.ovf, a.counts, smem);
 }
+__global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_trace_closest_wide(TraceArgs a) {
+    __shared__ int smem[TW_LDS_CLOSEST];
+    RaySrc src{a.S, a.rays, a.hits, nullptr, a.two_sided};
+    traverse<false>(src, a.n, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
+}
+__global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_trace_any_wide(TraceArgs a) {
+    __shared__ int smem[TW_LDS_ANY];
+    RaySrc src{a.S, a.rays, nullptr, a.occ, 0};
+    traverse<true>(src, a.n, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
+}
 __global__ void k_gen_rays(ff_dev_camera cam, int32_t W, int32_t H, uint32_t seed, uint32_t sample,
                            float4* rays) {
     uint32_t WH = (uint32_t)W * (uint32_t)H;
@@ -1535,7 +1910,22 @@ uint32_t resident_grid(K kernel, int bs) {
     return (uint32_t)g;
 }
 
-// traversal variants (block size, LDS stack entries, refill threshold, loop
+// Workgroups of a wide traversal launch of at most n_max rays: the resident
+// ones, or as many as such a launch spreads its rays over.
+template <class K>
+uint32_t traverse_grid(K kernel, uint32_t n_max) {
+    const uint32_t res = resident_grid(kernel, TW_BLOCK);
+    auto waves = [&](uint32_t spread, uint32_t rays) {
+        uint32_t per = n_max / spread + 1 < rays ? n_max / spread + 1 : rays;
+        return n_max / per + 1;
+    };
+    uint32_t w = waves(TW_SPREAD, 64);
+    if (n_max <= QUAD_MAX && waves(QUAD_SPREAD, 16) > w) w = waves(QUAD_SPREAD, 16);
+    const uint32_t g = (w + TW_BLOCK / 64 - 1) / (TW_BLOCK / 64);
+    return g < res ? g : res;
+}
+
+// counted traversal variants (block size, LDS stack entries, refill threshold, loop
 // shape 0-4, BVH record width)
 #define FF_TRAV_VARIANT_LIST(X)  \
     X(0, 256, 16, 32, 0, false)  \
@@ -1566,41 +1956,23 @@ uint32_t resident_grid(K kernel, int bs) {
     X(25, 256, 16, 16, 7, false) \
     X(26, 128, 16, 16, 5, false)
 
-// which: 0 extend, 1 shadow, 2 grid sizes only (before a graph capture),
-// 3 ff_trace_closest, 4 ff_trace_any
+// which: 3 ff_trace_closest, 4 ff_trace_any
 template <int BS, int LDS, int RF, int WW, bool WIDE>
-hipError_t trav_launch(int which, const ff_paths* P, int q, const TraceArgs* T, hipStream_t s) {
-    if (which == 0 && P->uni_scene) {
-        uint32_t g = resident_grid(k_extend<BS, LDS, RF, WW, WIDE, true>, BS);
-        hipLaunchKernelGGL((k_extend<BS, LDS, RF, WW, WIDE, true>), dim3(g), dim3(BS), 0, s, *P, q);
-    } else if (which == 0) {
-        uint32_t g = resident_grid(k_extend<BS, LDS, RF, WW, WIDE, false>, BS);
-        hipLaunchKernelGGL((k_extend<BS, LDS, RF, WW, WIDE, false>), dim3(g), dim3(BS), 0, s, *P, q);
-    } else if (which == 1 && P->uni_scene) {
-        uint32_t g = resident_grid(k_shadow<BS, LDS, RF, WW, WIDE, true>, BS);
-        hipLaunchKernelGGL((k_shadow<BS, LDS, RF, WW, WIDE, true>), dim3(g), dim3(BS), 0, s, *P);
-    } else if (which == 1) {
-        uint32_t g = resident_grid(k_shadow<BS, LDS, RF, WW, WIDE, false>, BS);
-        hipLaunchKernelGGL((k_shadow<BS, LDS, RF, WW, WIDE, false>), dim3(g), dim3(BS), 0, s, *P);
-    } else if (which == 3) {
+hipError_t trav_launch(int which, const TraceArgs& T, hipStream_t s) {
+    if (which == 3) {
         uint32_t g = resident_grid(k_trace_closest<BS, LDS, RF, WW, WIDE>, BS);
-        hipLaunchKernelGGL((k_trace_closest<BS, LDS, RF, WW, WIDE>), dim3(g), dim3(BS), 0, s, *T);
-    } else if (which == 4) {
-        uint32_t g = resident_grid(k_trace_any<BS, LDS, RF, WW, WIDE>, BS);
-        hipLaunchKernelGGL((k_trace_any<BS, LDS, RF, WW, WIDE>), dim3(g), dim3(BS), 0, s, *T);
+        hipLaunchKernelGGL((k_trace_closest<BS, LDS, RF, WW, WIDE>), dim3(g), dim3(BS), 0, s, T);
     } else {
-        (void)resident_grid(k_extend<BS, LDS, RF, WW, WIDE, true>, BS);
-        (void)resident_grid(k_shadow<BS, LDS, RF, WW, WIDE, true>, BS);
-        (void)resident_grid(k_extend<BS, LDS, RF, WW, WIDE, false>, BS);
-        (void)resident_grid(k_shadow<BS, LDS, RF, WW, WIDE, false>, BS);
+        uint32_t g = resident_grid(k_trace_any<BS, LDS, RF, WW, WIDE>, BS);
+        hipLaunchKernelGGL((k_trace_any<BS, LDS, RF, WW, WIDE>), dim3(g), dim3(BS), 0, s, T);
     }
     return hipGetLastError();
 }
 
-hipError_t trav_dispatch(int which, int variant, const ff_paths* P, int q, const TraceArgs* T, hipStream_t s) {
+hipError_t trav_dispatch(int which, int variant, const TraceArgs& T, hipStream_t s) {
     switch (variant) {
 #define FF_TRAV_CASE(v, bs, lds, rf, ww, wide) \
-    case v: return trav_launch<bs, lds, rf, ww, wide>(which, P, q, T, s);
+    case v: return trav_launch<bs, lds, rf, ww, wide>(which, T, s);
         FF_TRAV_VARIANT_LIST(FF_TRAV_CASE)
 #undef FF_TRAV_CASE
         default: return hipErrorInvalidValue;
@@ -1685,13 +2057,26 @@ hipError_t launch_generate(const ff_paths& P, hipStream_t s) {
     hipLaunchKernelGGL(k_generate, dim3(grid_for(P.n_slots, FF_GRID_CAP)), dim3(FF_BLOCK), 0, s, P);
     return hipGetLastError();
 }
-hipError_t launch_extend(const ff_paths& P, int q, int variant, hipStream_t s) {
-    return trav_dispatch(0, variant, &P, q, nullptr, s);
+hipError_t launch_extend(const ff_paths& P, int q, hipStream_t s) {
+    if (P.uni_scene)
+        hipLaunchKernelGGL(k_extend<true>, dim3(traverse_grid(k_extend<true>, P.n_slots)), dim3(TW_BLOCK), 0, s, P, q);
+    else
+        hipLaunchKernelGGL(k_extend<false>, dim3(traverse_grid(k_extend<false>, P.n_slots)), dim3(TW_BLOCK), 0, s, P, q);
+    return hipGetLastError();
 }
-hipError_t launch_shadow(const ff_paths& P, int variant, hipStream_t s) {
-    return trav_dispatch(1, variant, &P, 0, nullptr, s);
+hipError_t launch_shadow(const ff_paths& P, hipStream_t s) {
+    if (P.uni_scene)
+        hipLaunchKernelGGL(k_shadow<true>, dim3(traverse_grid(k_shadow<true>, P.n_slots)), dim3(TW_BLOCK), 0, s, P);
+    else
+        hipLaunchKernelGGL(k_shadow<false>, dim3(traverse_grid(k_shadow<false>, P.n_slots)), dim3(TW_BLOCK), 0, s, P);
+    return hipGetLastError();
 }
-hipError_t prepare_traversal(int variant) { return trav_dispatch(2, variant, nullptr, 0, nullptr, nullptr); }
+void prepare_traversal() {
+    (void)resident_grid(k_extend<true>, TW_BLOCK);
+    (void)resident_grid(k_extend<false>, TW_BLOCK);
+    (void)resident_grid(k_shadow<true>, TW_BLOCK);
+    (void)resident_grid(k_shadow<false>, TW_BLOCK);
+}
 hipError_t launch_reset(uint32_t* counters, uint32_t mask, uint32_t* fetch, uint32_t fetch_mask, hipStream_t s) {
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(256), 0, s, counters, mask, fetch, fetch_mask);
     return hipGetLastError();
@@ -1783,7 +2168,12 @@ hipError_t launch_trace_closest(const ff_dev_scene& S, const float4* rays, uint3
                                 int variant, hipStream_t s) {
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(256), 0, s, nullptr, 0u, fetch, 1u << F_TRACE);
     TraceArgs T{S, rays, n, hits, nullptr, two_sided, fetch + F_TRACE * FETCH_SEGS * FETCH_STRIDE, ovf, counts};
-    return trav_dispatch(3, variant, nullptr, 0, &T, s);
+    if (!counts && S.wide) {
+        hipLaunchKernelGGL(k_trace_closest_wide, dim3(traverse_grid(k_trace_closest_wide, n)), dim3(TW_BLOCK), 0, s,
+                           T);
+        return hipGetLastError();
+    }
+    return trav_dispatch(3, variant, T, s);
 }
 // Device address of `scratch` on `device` (looked up once per device, with
 // that device current, by ff_context_create).
@@ -1814,7 +2204,11 @@ hipError_t launch_trace_any(const ff_dev_scene& S, const float4* rays, uint32_t 
                             int32_t* ovf, unsigned long long* counts, int variant, hipStream_t s) {
     hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(256), 0, s, nullptr, 0u, fetch, 1u << F_TRACE);
     TraceArgs T{S, rays, n, nullptr, occ, 0, fetch + F_TRACE * FETCH_SEGS * FETCH_STRIDE, ovf, counts};
-    return trav_dispatch(4, variant, nullptr, 0, &T, s);
+    if (!counts && S.wide) {
+        hipLaunchKernelGGL(k_trace_any_wide, dim3(traverse_grid(k_trace_any_wide, n)), dim3(TW_BLOCK), 0, s, T);
+        return hipGetLastError();
+    }
+    return trav_dispatch(4, variant, T, s);
 }
 hipError_t launch_gen_rays(const ff_dev_camera& cam, int W, int H, uint32_t seed, uint32_t sample, float4* rays,
                            hipStream_t s) {

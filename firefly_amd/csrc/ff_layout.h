@@ -2,8 +2,10 @@
 //
 // HBM layout (all arrays are structure-of-arrays indexed by path id or BVH
 // slot; float4 fields keep every per-path record a 16-byte aligned load):
+//   wide    : compressed wide records, 64 bytes a node of up to four
+//             children or a triangle (ff_device.h)
 //   nodes   : the reference's binary BVH as 64-byte two-child records
-//             (both child boxes + child refs; 32 B per box tested)
+//             (both child boxes + child refs), for counted traces
 //   tris    : 9 floats per slot, v0 | e1 | e2 (36 B, positions only)
 //   nrm/uv  : shading attributes per slot, read once per closest hit
 //   paths   : ray (2 x float4, carrying the rng base and the state word in
@@ -54,6 +56,13 @@
 #define FETCH_WORDS (3 * FETCH_SEGS * FETCH_STRIDE)
 #define FETCH_CHUNK 256  // largest claim of one wave from a work counter
 
+// LDS stack entries of a traversal lane; the four-lane walk has four times as
+// many for its ray: three entries a wide level, or the binary tree's depth
+#define FF_LDS_STACK 16
+static inline __host__ __device__ bool quad_fits(int32_t wide_levels, int32_t max_depth) {
+    return 3 * wide_levels + 1 <= 4 * FF_LDS_STACK && max_depth + 1 <= 4 * FF_LDS_STACK;
+}
+
 // ray statistics
 #define S_PRIMARY 0
 #define S_EXTENSION 1
@@ -90,6 +99,7 @@ struct ff_tex_desc {
 struct ff_dev_scene {
     const float4* nodes;       // two-child records, 4 x float4 each
     const float4* nodes4;      // 4-wide records, 8 x float4 each
+    const float4* wide;        // compressed wide records, 4 x float4 each
     const int32_t* leaf_count; // per slot, for leaves of 15 or more primitives
     const float* root;         // root box lo.xyz hi.xyz, root ref
     const float* tris;
@@ -99,6 +109,7 @@ struct ff_dev_scene {
     const float* mats;
     const ff_tex_desc* tex;
     int32_t n_nodes, n_tris, n_mats, n_tex, max_depth;
+    int32_t wide_levels;       // levels of the wide tree
 };
 
 // Guide tables of the inverse-CDF searches: for bucket g of [0, 1) (width
@@ -190,6 +201,7 @@ struct ff_paths {
     uint32_t n_slots;    // total slots over all requests
     int32_t uni_scene;   // every request of the call renders the same scene
     int32_t uni_env;     // every request of the call uses the same environment
+    int32_t quad;        // every scene's stacks fit the four-lane walk (quad_fits)
     // adjoint replay
     float4* dlt;         // [P]     d loss / d path radiance (xyz)
     uint32_t* g_max;     // arena: max |term| bits per gradient element (GM_BOUND)

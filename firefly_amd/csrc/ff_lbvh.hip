@@ -28,6 +28,7 @@
 
 #include <stdint.h>
 
+#include <utility>
 #include <vector>
 
 #include "ff_internal.h"
@@ -263,19 +264,36 @@ __device__ __forceinline__ bool kept(const Tree& T, int v) { return rsize(T, v) 
 // One thread per internal node and per primitive: an output node finds its
 // depth-first index (first child at +1, second after the first's subtree)
 // and writes its record.
+// stats[0]: the tree's depth in nodes, stats[1]: the largest leaf
+__device__ __forceinline__ void tree_stats(int depth, int leaf, int* stats) {
+    for (int off = 32; off > 0; off >>= 1) {
+        depth = max(depth, __shfl_xor(depth, off));
+        leaf = max(leaf, __shfl_xor(leaf, off));
+    }
+    if ((threadIdx.x & 63) == 0) {
+        atomicMax(&stats[0], depth);
+        atomicMax(&stats[1], leaf);
+    }
+}
+__device__ __forceinline__ void emit_node(const Tree& T, int t, ffh::BvhNode* __restrict__ out, int& depth, int& leaf);
 __global__ __launch_bounds__(LB_BLOCK) void k_emit(Tree T, ffh::BvhNode* __restrict__ out,
-                                                  int32_t* __restrict__ ordered) {
-    int t = blockIdx.x * LB_BLOCK + threadIdx.x;
+                                                  int32_t* __restrict__ ordered, int* stats) {
+    int t = blockIdx.x * LB_BLOCK + threadIdx.x, depth = 0, leaf = 0;
+    if (t < T.n) ordered[t] = (int32_t)(T.keys[t] & 0xffffffffu);
+    if (t < 2 * T.n - 1) emit_node(T, t, out, depth, leaf);
+    tree_stats(depth, leaf, stats);
+}
+__device__ __forceinline__ void emit_node(const Tree& T, int t, ffh::BvhNode* __restrict__ out, int& depth,
+                                          int& leaf) {
     int n = T.n;
-    if (t < n) ordered[t] = (int32_t)(T.keys[t] & 0xffffffffu);
-    if (t >= 2 * n - 1) return;
     bool prim = t >= n - 1;
     int v = prim ? ~(t - (n - 1)) : t;  // node id: internal >= 0, primitive < 0
     int par = prim ? (n > 1 ? T.par_leaf[~v] : -1) : T.par_int[v];
     bool is_out = prim ? (par < 0 || kept(T, par)) : (kept(T, v) || par < 0 || kept(T, par));
     if (!is_out) return;
     int idx = 0;
-    for (int cur = v, pp = par; pp >= 0;) {
+    depth = 1;
+    for (int cur = v, pp = par; pp >= 0; depth++) {
         int2 c = T.child[pp];
         if (c.y == cur) idx += 1 + (c.x >= 0 ? T.isize[c.x] : 1);
         else idx += 1;
@@ -299,6 +317,7 @@ __global__ __launch_bounds__(LB_BLOCK) void k_emit(Tree T, ffh::BvhNode* __restr
         r.offset = a;
         r.n_prims = (uint16_t)(z - a + 1);
         r.axis = 0;
+        leaf = z - a + 1;
     }
     out[idx] = r;
 }
@@ -467,13 +486,22 @@ __global__ __launch_bounds__(LB_BLOCK) void k_ploc_merge(const int* __restrict__
 // Every node finds its depth-first output index and the depth-first index
 // of its first triangle by walking to the root; triangles place themselves
 // in the slot order, output nodes write their records.
+__device__ __forceinline__ void ploc_emit_node(const PNodes& N, const uint64_t* __restrict__ keys, int n, int v,
+                                               ffh::BvhNode* __restrict__ out, int32_t* __restrict__ ordered,
+                                               int& depth_out, int& leaf_out);
 __global__ __launch_bounds__(LB_BLOCK) void k_ploc_emit(PNodes N, const uint64_t* __restrict__ keys, int n,
-                                                       ffh::BvhNode* __restrict__ out, int32_t* __restrict__ ordered) {
-    int v = blockIdx.x * LB_BLOCK + threadIdx.x;
-    if (v >= 2 * n - 1) return;
-    int idx = 0, poff = 0;
+                                                       ffh::BvhNode* __restrict__ out, int32_t* __restrict__ ordered,
+                                                       int* stats) {
+    int v = blockIdx.x * LB_BLOCK + threadIdx.x, depth = 0, leaf = 0;
+    if (v < 2 * n - 1) ploc_emit_node(N, keys, n, v, out, ordered, depth, leaf);
+    tree_stats(depth, leaf, stats);
+}
+__device__ __forceinline__ void ploc_emit_node(const PNodes& N, const uint64_t* __restrict__ keys, int n, int v,
+                                               ffh::BvhNode* __restrict__ out, int32_t* __restrict__ ordered,
+                                               int& depth_out, int& leaf_out) {
+    int idx = 0, poff = 0, depth = 1;
     bool is_out = true;
-    for (int cur = v, p = N.parent[v]; p >= 0; cur = p, p = N.parent[p]) {
+    for (int cur = v, p = N.parent[v]; p >= 0; cur = p, p = N.parent[p], depth++) {
         if (N.leaf[p]) is_out = false;
         int f = N.first[p];
         if (N.second[p] == cur) {
@@ -485,6 +513,8 @@ __global__ __launch_bounds__(LB_BLOCK) void k_ploc_emit(PNodes N, const uint64_t
     }
     if (v < n) ordered[poff] = (int32_t)(keys[v] & 0xffffffffu);
     if (!is_out) return;
+    depth_out = depth;
+    if (N.leaf[v]) leaf_out = N.count[v];
     ffh::BvhNode r;
     const float* b = N.box + (size_t)v * 6;
     for (int c = 0; c < 3; c++) {
@@ -504,76 +534,90 @@ __global__ __launch_bounds__(LB_BLOCK) void k_ploc_emit(PNodes N, const uint64_t
     out[idx] = r;
 }
 
-template <class X>
-hipError_t alloc(X** p, size_t n) {
-    return hipMalloc((void**)p, sizeof(X) * (n ? n : 1));
-}
-
 }  // namespace
 
-// positions on the host [n][3][3]; nodes and ordered come back on the host;
-// gpu_ms (optional): device time from the bounds pass to the emitted tree
-hipError_t build_lbvh(const float* positions, int32_t n, int32_t max_prims, std::vector<ffh::BvhNode>& nodes,
-                      std::vector<int32_t>& ordered, float* gpu_ms) {
+// A linear BVH of the host positions on the device; gpu_ms (optional): device
+// time from the bounds pass to the emitted tree
+hipError_t build_lbvh(const float* positions, int32_t n, int32_t max_prims, DevBvh& out, float* gpu_ms) {
     if (n <= 0) return hipErrorInvalidValue;
     if (max_prims < 1) max_prims = 1;
     if (max_prims > 65535) max_prims = 65535;  // a leaf's count is 16 bits
     hipStream_t s = nullptr;
-    float *d_pos = nullptr, *d_ibox = nullptr, *d_lbox = nullptr;
-    uint64_t *d_keys = nullptr, *d_sorted = nullptr;
-    uint32_t *d_cb = nullptr, *d_flag = nullptr;
-    int2 *d_child = nullptr, *d_range = nullptr;
-    int *d_par_int = nullptr, *d_par_leaf = nullptr, *d_isize = nullptr, *d_ord = nullptr;
-    uint8_t* d_axis = nullptr;
-    ffh::BvhNode* d_nodes = nullptr;
-    void* d_tmp = nullptr;
-    size_t m = (size_t)n, tmp_bytes = 0;
+    uint64_t *keys = nullptr, *sorted = nullptr;
+    uint32_t *cb = nullptr, *flag = nullptr;
+    int2 *child = nullptr, *range = nullptr;
+    int *par_int = nullptr, *par_leaf = nullptr, *isize = nullptr, *stats = nullptr;
+    uint8_t* axis = nullptr;
+    float *ibox = nullptr, *lbox = nullptr;
+    char* sort_tmp = nullptr;
+    const size_t m = (size_t)n;
+    size_t tmp_bytes = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipError_t e = hipStreamCreate(&s);
-    if (e == hipSuccess && gpu_ms) e = hipEventCreate(&ev0);
-    if (e == hipSuccess && gpu_ms) e = hipEventCreate(&ev1);
     auto ok = [&](hipError_t x) { if (e == hipSuccess) e = x; return e == hipSuccess; };
-    if (ok(alloc(&d_pos, 9 * m)) && ok(alloc(&d_keys, m)) && ok(alloc(&d_sorted, m)) && ok(alloc(&d_cb, 6)) &&
-        ok(alloc(&d_child, m)) && ok(alloc(&d_range, m)) && ok(alloc(&d_par_int, m)) && ok(alloc(&d_par_leaf, m)) &&
-        ok(alloc(&d_axis, m)) && ok(alloc(&d_ibox, 6 * m)) && ok(alloc(&d_lbox, 6 * m)) && ok(alloc(&d_isize, m)) &&
-        ok(alloc(&d_flag, m)) && ok(alloc(&d_nodes, 2 * m)) && ok(alloc(&d_ord, m)) &&
-        ok(hipMemcpyAsync(d_pos, positions, sizeof(float) * 9 * m, hipMemcpyHostToDevice, s)) &&
-        ok(hipMemsetAsync(d_flag, 0, sizeof(uint32_t) * m, s)) &&
-        ok(hipMemsetAsync(d_par_int, 0xff, sizeof(int) * m, s)) &&  // the root's parent: -1
-        ok(rocprim::radix_sort_keys(nullptr, tmp_bytes, d_keys, d_sorted, m, 0, 62, s)) &&
-        ok(hipMalloc(&d_tmp, tmp_bytes ? tmp_bytes : 1))) {
-        uint32_t g = (uint32_t)((m + LB_BLOCK - 1) / LB_BLOCK);
-        uint32_t gb = g < 4096 ? g : 4096;
+    if (gpu_ms) ok(hipEventCreate(&ev0)) && ok(hipEventCreate(&ev1));
+    ok(rocprim::radix_sort_keys(nullptr, tmp_bytes, keys, sorted, m, 0, 62, s));
+    auto carve = [&](Carver c) {
+        out.nodes = c.take<ffh::BvhNode>(2 * m);
+        out.ordered = c.take<int32_t>(m);
+        out.pos = c.take<float>(9 * m);
+        return c.off;
+    };
+    auto carve_tmp = [&](Carver c) {
+        keys = c.take<uint64_t>(m);
+        sorted = c.take<uint64_t>(m);
+        cb = c.take<uint32_t>(6);
+        child = c.take<int2>(m);
+        range = c.take<int2>(m);
+        par_int = c.take<int>(m);
+        par_leaf = c.take<int>(m);
+        axis = c.take<uint8_t>(m);
+        ibox = c.take<float>(6 * m);
+        lbox = c.take<float>(6 * m);
+        isize = c.take<int>(m);
+        flag = c.take<uint32_t>(m);
+        stats = c.take<int>(2);
+        sort_tmp = c.take<char>(tmp_bytes);
+        return c.off;
+    };
+    void* tmp = nullptr;
+    if (ok(hipMalloc(&out.mem, carve(Carver{}))) && ok(hipMalloc(&tmp, carve_tmp(Carver{})))) {
+        carve(Carver{(char*)out.mem});
+        carve_tmp(Carver{(char*)tmp});
+        ok(hipMemcpyAsync(out.pos, positions, sizeof(float) * 9 * m, hipMemcpyHostToDevice, s));
+        ok(hipMemsetAsync(flag, 0, sizeof(uint32_t) * m, s));
+        ok(hipMemsetAsync(stats, 0, 2 * sizeof(int), s));
+        ok(hipMemsetAsync(par_int, 0xff, sizeof(int) * m, s));  // the root's parent: -1
+    }
+    if (e == hipSuccess) {
+        const uint32_t g = (uint32_t)((m + LB_BLOCK - 1) / LB_BLOCK);
+        const uint32_t gb = g < 4096 ? g : 4096;
         if (ev0) ok(hipEventRecord(ev0, s));
-        hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(64), 0, s, d_cb);
-        hipLaunchKernelGGL(k_centroid_bounds, dim3(gb), dim3(LB_BLOCK), 0, s, d_pos, (uint32_t)n, d_cb);
-        hipLaunchKernelGGL(k_morton, dim3(gb), dim3(LB_BLOCK), 0, s, d_pos, (uint32_t)n, d_cb, d_keys);
-        if (ok(hipGetLastError()) && ok(rocprim::radix_sort_keys(d_tmp, tmp_bytes, d_keys, d_sorted, m, 0, 62, s))) {
+        hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(64), 0, s, cb);
+        hipLaunchKernelGGL(k_centroid_bounds, dim3(gb), dim3(LB_BLOCK), 0, s, out.pos, (uint32_t)n, cb);
+        hipLaunchKernelGGL(k_morton, dim3(gb), dim3(LB_BLOCK), 0, s, out.pos, (uint32_t)n, cb, keys);
+        if (ok(hipGetLastError()) && ok(rocprim::radix_sort_keys(sort_tmp, tmp_bytes, keys, sorted, m, 0, 62, s))) {
             if (n > 1)
                 hipLaunchKernelGGL(k_karras, dim3((uint32_t)((m - 1 + LB_BLOCK - 1) / LB_BLOCK)), dim3(LB_BLOCK), 0, s,
-                                   d_sorted, n, d_child, d_range, d_par_int, d_par_leaf, d_axis);
-            Tree T{d_sorted, d_pos, d_child, d_range, d_par_int, d_par_leaf, d_axis,
-                   d_ibox, d_lbox, d_isize, d_flag, n, max_prims};
+                                   sorted, n, child, range, par_int, par_leaf, axis);
+            Tree T{sorted, out.pos, child, range, par_int, par_leaf, axis, ibox, lbox, isize, flag, n, max_prims};
             hipLaunchKernelGGL(k_refit, dim3(g), dim3(LB_BLOCK), 0, s, T);
             hipLaunchKernelGGL(k_emit, dim3((uint32_t)((2 * m - 1 + LB_BLOCK - 1) / LB_BLOCK)), dim3(LB_BLOCK), 0, s,
-                               T, d_nodes, d_ord);
+                               T, out.nodes, out.ordered, stats);
             if (ev1) ok(hipEventRecord(ev1, s));
-            int32_t n_out = 1;
-            if (ok(hipGetLastError()) && n > 1 && (int32_t)(m) > max_prims)
-                ok(hipMemcpyAsync(&n_out, d_isize, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+            int32_t n_out = 1, st[2] = {1, 1};
+            if (ok(hipGetLastError()) && n > 1 && n > max_prims)
+                ok(hipMemcpyAsync(&n_out, isize, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+            ok(hipMemcpyAsync(st, stats, sizeof(st), hipMemcpyDeviceToHost, s));
             if (ok(hipStreamSynchronize(s))) {
                 if (ev0) ok(hipEventElapsedTime(gpu_ms, ev0, ev1));
-                nodes.resize((size_t)n_out);
-                ordered.resize(m);
-                if (ok(hipMemcpy(nodes.data(), d_nodes, sizeof(ffh::BvhNode) * (size_t)n_out, hipMemcpyDeviceToHost)))
-                    ok(hipMemcpy(ordered.data(), d_ord, sizeof(int32_t) * m, hipMemcpyDeviceToHost));
+                out.n_nodes = n_out;
+                out.max_depth = st[0];
+                out.max_leaf = st[1];
             }
         }
     }
-    for (void* p : {(void*)d_pos, (void*)d_keys, (void*)d_sorted, (void*)d_cb, (void*)d_child, (void*)d_range,
-                    (void*)d_par_int, (void*)d_par_leaf, (void*)d_axis, (void*)d_ibox, (void*)d_lbox, (void*)d_isize,
-                    (void*)d_flag, (void*)d_nodes, (void*)d_ord, d_tmp})
-        if (p) (void)hipFree(p);
+    if (tmp) (void)hipFree(tmp);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (s) (void)hipStreamDestroy(s);
@@ -584,64 +628,85 @@ hipError_t build_lbvh(const float* positions, int32_t n, int32_t max_prims, std:
 // Morton keys of build_lbvh, then clustering rounds until one cluster is left
 // (the cluster count read back after each round), then the depth-first
 // emission.  positions on the host; gpu_ms as for build_lbvh.
-hipError_t build_ploc(const float* positions, int32_t n, int32_t max_prims, std::vector<ffh::BvhNode>& nodes,
-                      std::vector<int32_t>& ordered, float* gpu_ms) {
+hipError_t build_ploc(const float* positions, int32_t n, int32_t max_prims, DevBvh& out, float* gpu_ms) {
     if (n <= 0) return hipErrorInvalidValue;
     if (max_prims < 1) max_prims = 1;
     if (max_prims > 65535) max_prims = 65535;
     hipStream_t s = nullptr;
-    float *d_pos = nullptr, *d_box = nullptr, *d_cost = nullptr;
-    uint64_t *d_keys = nullptr, *d_sorted = nullptr;
-    unsigned long long *d_flags = nullptr, *d_scan = nullptr;
-    uint32_t* d_cb = nullptr;
-    int *d_first = nullptr, *d_second = nullptr, *d_parent = nullptr, *d_count = nullptr, *d_osize = nullptr;
-    int *d_C0 = nullptr, *d_C1 = nullptr, *d_nn = nullptr, *d_ord = nullptr;
-    uint8_t *d_axis = nullptr, *d_leaf = nullptr;
-    ffh::BvhNode* d_nodes = nullptr;
-    void *d_tmp = nullptr, *d_tmp2 = nullptr;
-    size_t m0 = (size_t)n, nn2 = 2 * m0 - 1, tmp_bytes = 0, tmp2_bytes = 0;
+    PNodes N{};
+    uint64_t *keys = nullptr, *sorted = nullptr;
+    unsigned long long *flags = nullptr, *scan = nullptr;
+    uint32_t* cb = nullptr;
+    int *C = nullptr, *Cn = nullptr, *nn = nullptr, *stats = nullptr;
+    char *sort_tmp = nullptr, *scan_tmp = nullptr;
+    const size_t m0 = (size_t)n, nn2 = 2 * m0 - 1;
+    size_t tmp_bytes = 0, tmp2_bytes = 0;
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     hipError_t e = hipStreamCreate(&s);
-    if (e == hipSuccess && gpu_ms) e = hipEventCreate(&ev0);
-    if (e == hipSuccess && gpu_ms) e = hipEventCreate(&ev1);
     auto ok = [&](hipError_t x) { if (e == hipSuccess) e = x; return e == hipSuccess; };
-    if (ok(alloc(&d_pos, 9 * m0)) && ok(alloc(&d_keys, m0)) && ok(alloc(&d_sorted, m0)) && ok(alloc(&d_cb, 6)) &&
-        ok(alloc(&d_box, 6 * nn2)) && ok(alloc(&d_cost, nn2)) && ok(alloc(&d_first, nn2)) &&
-        ok(alloc(&d_second, nn2)) && ok(alloc(&d_parent, nn2)) && ok(alloc(&d_count, nn2)) &&
-        ok(alloc(&d_osize, nn2)) && ok(alloc(&d_axis, nn2)) && ok(alloc(&d_leaf, nn2)) && ok(alloc(&d_C0, m0)) &&
-        ok(alloc(&d_C1, m0)) && ok(alloc(&d_nn, m0)) && ok(alloc(&d_flags, m0)) && ok(alloc(&d_scan, m0)) &&
-        ok(alloc(&d_nodes, nn2)) && ok(alloc(&d_ord, m0)) &&
-        ok(hipMemcpyAsync(d_pos, positions, sizeof(float) * 9 * m0, hipMemcpyHostToDevice, s)) &&
-        ok(rocprim::radix_sort_keys(nullptr, tmp_bytes, d_keys, d_sorted, m0, 0, 62, s)) &&
-        ok(hipMalloc(&d_tmp, tmp_bytes ? tmp_bytes : 1)) &&
-        ok(rocprim::exclusive_scan(nullptr, tmp2_bytes, d_flags, d_scan, 0ull, m0, rocprim::plus<unsigned long long>(),
-                                   s)) &&
-        ok(hipMalloc(&d_tmp2, tmp2_bytes ? tmp2_bytes : 1))) {
-        uint32_t g = (uint32_t)((m0 + LB_BLOCK - 1) / LB_BLOCK);
-        uint32_t gb = g < 4096 ? g : 4096;
-        PNodes N{d_box, d_first, d_second, d_parent, d_count, d_cost, d_osize, d_axis, d_leaf, max_prims};
+    if (gpu_ms) ok(hipEventCreate(&ev0)) && ok(hipEventCreate(&ev1));
+    ok(rocprim::radix_sort_keys(nullptr, tmp_bytes, keys, sorted, m0, 0, 62, s));
+    ok(rocprim::exclusive_scan(nullptr, tmp2_bytes, flags, scan, 0ull, m0, rocprim::plus<unsigned long long>(), s));
+    auto carve = [&](Carver c) {
+        out.nodes = c.take<ffh::BvhNode>(nn2);
+        out.ordered = c.take<int32_t>(m0);
+        out.pos = c.take<float>(9 * m0);
+        return c.off;
+    };
+    auto carve_tmp = [&](Carver c) {
+        keys = c.take<uint64_t>(m0);
+        sorted = c.take<uint64_t>(m0);
+        cb = c.take<uint32_t>(6);
+        N.box = c.take<float>(6 * nn2);
+        N.cost = c.take<float>(nn2);
+        N.first = c.take<int>(nn2);
+        N.second = c.take<int>(nn2);
+        N.parent = c.take<int>(nn2);
+        N.count = c.take<int>(nn2);
+        N.osize = c.take<int>(nn2);
+        N.axis = c.take<uint8_t>(nn2);
+        N.leaf = c.take<uint8_t>(nn2);
+        C = c.take<int>(m0);
+        Cn = c.take<int>(m0);
+        nn = c.take<int>(m0);
+        flags = c.take<unsigned long long>(m0);
+        scan = c.take<unsigned long long>(m0);
+        stats = c.take<int>(2);
+        sort_tmp = c.take<char>(tmp_bytes);
+        scan_tmp = c.take<char>(tmp2_bytes);
+        return c.off;
+    };
+    N.max_prims = max_prims;
+    void* tmp = nullptr;
+    if (ok(hipMalloc(&out.mem, carve(Carver{}))) && ok(hipMalloc(&tmp, carve_tmp(Carver{})))) {
+        carve(Carver{(char*)out.mem});
+        carve_tmp(Carver{(char*)tmp});
+        ok(hipMemcpyAsync(out.pos, positions, sizeof(float) * 9 * m0, hipMemcpyHostToDevice, s));
+        ok(hipMemsetAsync(stats, 0, 2 * sizeof(int), s));
+    }
+    if (e == hipSuccess) {
+        const uint32_t g = (uint32_t)((m0 + LB_BLOCK - 1) / LB_BLOCK);
+        const uint32_t gb = g < 4096 ? g : 4096;
         if (ev0) ok(hipEventRecord(ev0, s));
-        hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(64), 0, s, d_cb);
-        hipLaunchKernelGGL(k_centroid_bounds, dim3(gb), dim3(LB_BLOCK), 0, s, d_pos, (uint32_t)n, d_cb);
-        hipLaunchKernelGGL(k_morton, dim3(gb), dim3(LB_BLOCK), 0, s, d_pos, (uint32_t)n, d_cb, d_keys);
-        if (ok(hipGetLastError()) && ok(rocprim::radix_sort_keys(d_tmp, tmp_bytes, d_keys, d_sorted, m0, 0, 62, s))) {
-            hipLaunchKernelGGL(k_ploc_leaves, dim3(g), dim3(LB_BLOCK), 0, s, d_sorted, d_pos, n, N, d_C0);
+        hipLaunchKernelGGL(k_bounds_init, dim3(1), dim3(64), 0, s, cb);
+        hipLaunchKernelGGL(k_centroid_bounds, dim3(gb), dim3(LB_BLOCK), 0, s, out.pos, (uint32_t)n, cb);
+        hipLaunchKernelGGL(k_morton, dim3(gb), dim3(LB_BLOCK), 0, s, out.pos, (uint32_t)n, cb, keys);
+        if (ok(hipGetLastError()) && ok(rocprim::radix_sort_keys(sort_tmp, tmp_bytes, keys, sorted, m0, 0, 62, s))) {
+            hipLaunchKernelGGL(k_ploc_leaves, dim3(g), dim3(LB_BLOCK), 0, s, sorted, out.pos, n, N, C);
             int m = n, base = n;
-            int *C = d_C0, *Cn = d_C1;
             while (m > 1 && ok(hipGetLastError())) {
                 uint32_t gm = (uint32_t)((m + LB_BLOCK - 1) / LB_BLOCK);
-                hipLaunchKernelGGL(k_ploc_nn, dim3(gm), dim3(LB_BLOCK), 0, s, C, m, d_box, d_nn);
-                hipLaunchKernelGGL(k_ploc_flags, dim3(gm), dim3(LB_BLOCK), 0, s, d_nn, m, d_flags);
+                hipLaunchKernelGGL(k_ploc_nn, dim3(gm), dim3(LB_BLOCK), 0, s, C, m, N.box, nn);
+                hipLaunchKernelGGL(k_ploc_flags, dim3(gm), dim3(LB_BLOCK), 0, s, nn, m, flags);
                 if (!ok(hipGetLastError()) ||
-                    !ok(rocprim::exclusive_scan(d_tmp2, tmp2_bytes, d_flags, d_scan, 0ull, (size_t)m,
+                    !ok(rocprim::exclusive_scan(scan_tmp, tmp2_bytes, flags, scan, 0ull, (size_t)m,
                                                 rocprim::plus<unsigned long long>(), s)))
                     break;
-                hipLaunchKernelGGL(k_ploc_merge, dim3(gm), dim3(LB_BLOCK), 0, s, C, d_nn, m, d_flags, d_scan, base, N,
-                                   Cn);
+                hipLaunchKernelGGL(k_ploc_merge, dim3(gm), dim3(LB_BLOCK), 0, s, C, nn, m, flags, scan, base, N, Cn);
                 unsigned long long tail[2] = {0, 0};
                 if (!ok(hipGetLastError()) ||
-                    !ok(hipMemcpyAsync(&tail[0], d_scan + (m - 1), 8, hipMemcpyDeviceToHost, s)) ||
-                    !ok(hipMemcpyAsync(&tail[1], d_flags + (m - 1), 8, hipMemcpyDeviceToHost, s)) ||
+                    !ok(hipMemcpyAsync(&tail[0], scan + (m - 1), 8, hipMemcpyDeviceToHost, s)) ||
+                    !ok(hipMemcpyAsync(&tail[1], flags + (m - 1), 8, hipMemcpyDeviceToHost, s)) ||
                     !ok(hipStreamSynchronize(s)))
                     break;
                 unsigned long long tot = tail[0] + tail[1];
@@ -652,31 +717,25 @@ hipError_t build_ploc(const float* positions, int32_t n, int32_t max_prims, std:
                 }
                 base += made;
                 m = kept;
-                int* t = C;
-                C = Cn;
-                Cn = t;
+                std::swap(C, Cn);
             }
             if (e == hipSuccess)
                 hipLaunchKernelGGL(k_ploc_emit, dim3((uint32_t)((nn2 + LB_BLOCK - 1) / LB_BLOCK)), dim3(LB_BLOCK), 0, s,
-                                   N, d_sorted, n, d_nodes, d_ord);
+                                   N, sorted, n, out.nodes, out.ordered, stats);
             if (ev1) ok(hipEventRecord(ev1, s));
-            int32_t n_out = 1;
+            int32_t n_out = 1, st[2] = {1, 1};
             if (ok(hipGetLastError()))
-                ok(hipMemcpyAsync(&n_out, d_osize + (nn2 - 1), sizeof(int32_t), hipMemcpyDeviceToHost, s));
+                ok(hipMemcpyAsync(&n_out, N.osize + (nn2 - 1), sizeof(int32_t), hipMemcpyDeviceToHost, s));
+            ok(hipMemcpyAsync(st, stats, sizeof(st), hipMemcpyDeviceToHost, s));
             if (ok(hipStreamSynchronize(s))) {
                 if (ev0) ok(hipEventElapsedTime(gpu_ms, ev0, ev1));
-                nodes.resize((size_t)n_out);
-                ordered.resize(m0);
-                if (ok(hipMemcpy(nodes.data(), d_nodes, sizeof(ffh::BvhNode) * (size_t)n_out, hipMemcpyDeviceToHost)))
-                    ok(hipMemcpy(ordered.data(), d_ord, sizeof(int32_t) * m0, hipMemcpyDeviceToHost));
+                out.n_nodes = n_out;
+                out.max_depth = st[0];
+                out.max_leaf = st[1];
             }
         }
     }
-    for (void* p : {(void*)d_pos, (void*)d_keys, (void*)d_sorted, (void*)d_cb, (void*)d_box, (void*)d_cost,
-                    (void*)d_first, (void*)d_second, (void*)d_parent, (void*)d_count, (void*)d_osize, (void*)d_axis,
-                    (void*)d_leaf, (void*)d_C0, (void*)d_C1, (void*)d_nn, (void*)d_flags, (void*)d_scan,
-                    (void*)d_nodes, (void*)d_ord, d_tmp, d_tmp2})
-        if (p) (void)hipFree(p);
+    if (tmp) (void)hipFree(tmp);
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
     if (s) (void)hipStreamDestroy(s);

@@ -294,19 +294,21 @@ ff_status ff_adjoint(ff_context *ctx, ff_scene *scene, ff_envmap *env, const ff_
 ff_status ff_adjoint_batch(ff_context *ctx, const ff_batch_item *items, int32_t n, int32_t flags,
                            void *stream);
 
-/* ---- traversal kernel variants (workgroup size, LDS stack entries, the
- * number of idle lanes at which a wave of the persistent traversal fetches
- * new rays, the loop shape: 0 = one step per iteration, 1 = while-while,
- * 2 = speculative while-while (leaves postponed while other lanes walk),
- * 3, 5, 6, 7 = leaf batching (a lane queues the leaf it reaches and walks on;
- * queued leaves are tested together once 8, 8, 4 or 16 lanes hold one; shape
- * 3 queues two leaves per lane, the others one), and the
- * BVH record width: 2 = the reference's binary nodes two children at a time,
- * 4 = the same tree collapsed to 4-wide records, visited in the same leaf
- * order so hits are identical), chosen per context by the autotuner
- * (firefly_amd/autotune.py); variant 0 is the default.  The context's variant
- * applies to its renders and to ff_trace_closest / ff_trace_any.  No
- * reference counterpart (the reference has one fixed shape).  Renders and
+/* ---- traversal kernel variants of traces that count.  Renders, and traces
+ * that ask for no counts, walk compressed wide records with one launch shape
+ * and return the reference's hits; the counts of ff_last_render_stats are of
+ * the boxes (four a record) and triangles that walk tests.  A trace that asks
+ * for counts walks the reference's tree in the reference's order with the
+ * context's variant: workgroup size, LDS stack entries, the number of idle
+ * lanes at which a wave fetches new rays, the loop shape: 0 = one step per
+ * iteration, 1 = while-while, 2 = speculative while-while (leaves postponed
+ * while other lanes walk), 3, 5, 6, 7 = leaf batching (a lane queues the leaf
+ * it reaches and walks on; queued leaves are tested together once 8, 8, 4 or
+ * 16 lanes hold one; shape 3 queues two leaves per lane, the others one), and
+ * the BVH record width: 2 = the reference's binary nodes two children at a
+ * time, 4 = the same tree collapsed to 4-wide records, visited in the same
+ * leaf order.  Hits are the same for every variant; variant 0 is the default.
+ * No reference counterpart (the reference has one fixed shape).  Renders and
  * traces on one context share its work counters and buffers: they must not
  * overlap on different streams. */
 int32_t ff_traversal_variant_count(void);
@@ -314,9 +316,8 @@ ff_status ff_traversal_variant_info(int32_t variant, int32_t *block, int32_t *ld
                                     int32_t *refill, int32_t *while_while, int32_t *bvh_width);
 ff_status ff_set_traversal_variant(ff_context *ctx, int32_t variant);
 /* A second variant for the bounce iterations from `from_iteration` on (1 =
- * camera rays), whose launches trace the few surviving paths: the shapes that
- * win on the large first launches lose on small ones.  variant -1 turns it
- * off (every launch uses the context's variant).  No reference counterpart. */
+ * camera rays; variant -1: none).  Checked, and without effect: renders take
+ * their launch shape from the number of rays. */
 ff_status ff_set_traversal_tail(ff_context *ctx, int32_t variant, int32_t from_iteration);
 
 /* ray counts of the last ff_render on this context (synchronises its stream). */
