@@ -86,10 +86,6 @@ struct ff_context {
     size_t ovf_entries = 0;  // stack entries per grid thread
     hipStream_t last_stream = nullptr;
     hipStream_t own_stream = nullptr;  // graph capture when the caller passes the null stream
-    // a second stream for the shadow traversal, which runs beside the
-    // extension traversal of the same iteration (fork / join events)
-    hipStream_t side = nullptr;
-    hipEvent_t fork_ev = nullptr, join_ev = nullptr;
     bool have_stats = false;
     uint32_t* bstate = nullptr;
     ff_dev_request* d_reqs = nullptr;
@@ -249,9 +245,6 @@ ff_status ff_context_destroy(ff_context* c) {
     c->paths.release();
     for (hipEvent_t e : c->event_pool) (void)hipEventDestroy(e);
     if (c->own_stream) (void)hipStreamDestroy(c->own_stream);
-    if (c->side) (void)hipStreamDestroy(c->side);
-    if (c->fork_ev) (void)hipEventDestroy(c->fork_ev);
-    if (c->join_ev) (void)hipEventDestroy(c->join_ev);
     dfree(c->bstate);
     dfree(c->d_reqs);
     dfree(c->d_qbase);
@@ -659,11 +652,6 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         if (!ctx->own_stream) HIP_TRY(hipStreamCreate(&ctx->own_stream));
         hs = ctx->own_stream;
     }
-    if (!ctx->side) {
-        HIP_TRY(hipStreamCreateWithFlags(&ctx->side, hipStreamNonBlocking));
-        HIP_TRY(hipEventCreateWithFlags(&ctx->fork_ev, hipEventDisableTiming));
-        HIP_TRY(hipEventCreateWithFlags(&ctx->join_ev, hipEventDisableTiming));
-    }
     ffk::prepare_traversal();
     ff_paths p = ctx->paths.p;
     const bool adjoint = (reqs[0].mode & RQ_ADJOINT) != 0;
@@ -756,10 +744,26 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         HIP_TRY(dalloc(&ctx->d_qbase, table.size() + 1));
         ctx->req_cap = table.size();
     }
-    HIP_TRY(hipStreamSynchronize(hs));
-    HIP_TRY(hipMemcpy(ctx->d_reqs, table.data(), table.size() * sizeof(ff_dev_request), hipMemcpyHostToDevice));
-    if (adjoint && !gt.empty())
-        HIP_TRY(hipMemcpy(ctx->d_gt, gt.data(), gt.size() * sizeof(ff_dev_gtarget), hipMemcpyHostToDevice));
+    // One request travels with the first launch, in stream order behind the
+    // call before it; a table of them is copied once the stream has finished
+    // with the last one.  (A call on another stream than the last waits.)
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    HIP_TRY(hipStreamIsCapturing(hs, &capturing));
+    if (capturing != hipStreamCaptureStatusNone)
+        return fail(FF_ERR_HIP, "%s: the stream is being captured (FF_RENDER_USE_GRAPH captures inside the call)", who);
+    ff_begin begin{};
+    if (table.size() == 1 && gt.size() <= FF_BEGIN_GT && ctx->have_stats && ctx->last_stream == hs) {
+        begin.req = table[0];
+        begin.n_req = 1;
+        begin.n_gt = (int32_t)gt.size();
+        begin.gt_dst = ctx->d_gt;
+        for (size_t i = 0; i < gt.size(); i++) begin.gt[i] = gt[i];
+    } else {
+        HIP_TRY(hipStreamSynchronize(hs));
+        HIP_TRY(hipMemcpy(ctx->d_reqs, table.data(), table.size() * sizeof(ff_dev_request), hipMemcpyHostToDevice));
+        if (adjoint && !gt.empty())
+            HIP_TRY(hipMemcpy(ctx->d_gt, gt.data(), gt.size() * sizeof(ff_dev_gtarget), hipMemcpyHostToDevice));
+    }
     p.counters = ctx->counters;
     p.fetch = ctx->fetch;
     p.qbase = ctx->d_qbase;
@@ -785,7 +789,7 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
     ctx->records.clear();
     ctx->events_used = 0;
     // Records a begin/end event pair around one stage launch when timing.
-    auto timed_on = [&](hipStream_t ts, int stage, auto&& launch) -> hipError_t {
+    auto timed = [&](int stage, auto&& launch) -> hipError_t {
         if (!timing) return launch();
         while (ctx->event_pool.size() < ctx->events_used + 2) {
             hipEvent_t e;
@@ -795,13 +799,12 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         }
         StageRecord rec{stage, ctx->event_pool[ctx->events_used], ctx->event_pool[ctx->events_used + 1]};
         ctx->events_used += 2;
-        hipError_t e = hipEventRecord(rec.begin, ts);
+        hipError_t e = hipEventRecord(rec.begin, hs);
         if (e == hipSuccess) e = launch();
-        if (e == hipSuccess) e = hipEventRecord(rec.end, ts);
+        if (e == hipSuccess) e = hipEventRecord(rec.end, hs);
         ctx->records.push_back(rec);
         return e;
     };
-    auto timed = [&](int stage, auto&& launch) -> hipError_t { return timed_on(hs, stage, launch); };
     // the first batch stores every layer of a request whose spp covers its
     // samples in flight (wf_logic writes it without reading); only a request
     // with fewer samples than layers keeps layers that no path writes
@@ -809,31 +812,23 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         for (size_t r = 0; r < reqs.size(); r++)
             if (reqs[r].K > 1 && reqs[r].spp < reqs[r].K)
                 HIP_TRY(ffk::launch_fill4(table[r].layers, (uint32_t)((uint64_t)reqs[r].W * reqs[r].H * reqs[r].K), hs));
-    HIP_TRY(ffk::launch_fill_u64(p.stats, S_WORDS, hs));
+    bool first_pass = true;  // (the deterministic adjoint's second pass adds to the first's counts)
 
     // one batch of the forward: identical launches for every batch (the index is on the device)
     auto batch = [&]() -> ff_status {
-        HIP_TRY(ffk::launch_batch_begin(p, 0, 0, hs));
+        HIP_TRY(ffk::launch_batch_begin(p, hs));
         HIP_TRY(timed(4, [&] { return ffk::launch_generate(p, hs); }));
         int cur = 0;
         for (int32_t it = 1; it <= max_depth + 1; it++) {
-            // the iteration's extension rays and its vertices' shadow rays are
-            // independent: the shadow traversal runs on the side stream, so
-            // either kernel's waves fill the other's tail (with per-launch
-            // timing the two run one after another, so each time is its own)
-            hipStream_t ss = timing ? hs : ctx->side;
-            if (!timing) {
-                HIP_TRY(hipEventRecord(ctx->fork_ev, hs));
-                HIP_TRY(hipStreamWaitEvent(ss, ctx->fork_ev, 0));
+            // the iteration's extension rays and its vertices' shadow rays
+            // are independent: one launch traces both (with per-launch timing
+            // a launch each, so that each time is its own)
+            if (timing) {
+                HIP_TRY(timed(0, [&] { return ffk::launch_extend(p, cur, hs); }));
+                HIP_TRY(timed(1, [&] { return ffk::launch_shadow(p, hs); }));
+            } else {
+                HIP_TRY(ffk::launch_extend_shadow(p, cur, hs));
             }
-            HIP_TRY(timed(0, [&] { return ffk::launch_extend(p, cur, hs); }));
-            HIP_TRY(timed_on(ss, 1, [&] { return ffk::launch_shadow(p, ss); }));
-            if (!timing) {
-                HIP_TRY(hipEventRecord(ctx->join_ev, ss));
-                HIP_TRY(hipStreamWaitEvent(hs, ctx->join_ev, 0));
-            }
-            uint32_t mask = (1u << (cur == 0 ? C_EXT1 : C_EXT0)) | (1u << C_SHADOW) | (0xfu << C_MAT0);
-            HIP_TRY(ffk::launch_reset(p.counters, mask, p.fetch, (1u << F_EXT) | (1u << F_SHD), hs));
             HIP_TRY(timed(2, [&] { return ffk::launch_logic(p, cur, it, p.n_slots, hs); }));
             if (it <= max_depth) {
                 for (int m = 0; m < 4; m++)
@@ -846,13 +841,11 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
     // one batch of the adjoint replay: a vertex's shadow rays are traced
     // between its NEE replay and its gradient kernel
     auto batch_adj = [&]() -> ff_status {
-        HIP_TRY(ffk::launch_batch_begin(p, 0, 0, hs));
+        HIP_TRY(ffk::launch_batch_begin(p, hs));
         HIP_TRY(timed(4, [&] { return ffk::launch_generate(p, hs); }));
         int cur = 0;
         for (int32_t it = 1; it <= max_depth + 1; it++) {
             HIP_TRY(timed(0, [&] { return ffk::launch_extend(p, cur, hs); }));
-            uint32_t mask = (1u << (cur == 0 ? C_EXT1 : C_EXT0)) | (1u << C_SHADOW) | (0xfu << C_MAT0);
-            HIP_TRY(ffk::launch_reset(p.counters, mask, p.fetch, (1u << F_EXT) | (1u << F_SHD), hs));
             HIP_TRY(timed(2, [&] { return ffk::launch_logic_adj(p, cur, p.n_slots, hs); }));
             if (it <= max_depth) {
                 for (int m = 0; m < 3; m++)
@@ -867,7 +860,9 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         return FF_OK;
     };
     auto run = [&]() -> ff_status {
-        HIP_TRY(ffk::launch_batch_begin(p, 1, 0xffffffffu, hs));  // the first batch_begin makes it 0
+        begin.clear_stats = first_pass ? 1 : 0;
+        HIP_TRY(ffk::launch_begin(p, begin, hs));
+        first_pass = false;
         if (graph) {
             hipGraph_t g = nullptr;
             hipGraphExec_t ge = nullptr;

@@ -18,11 +18,12 @@ extern const int kTravWhileWhile[];
 extern const int kTravWidth[];  // BVH record width of the variant (2 or 4)
 // computes the grid sizes of the wavefront's traversal kernels (call before a graph capture)
 void prepare_traversal();
-hipError_t launch_batch_begin(const ff_paths& P, int set, uint32_t value, hipStream_t s);
+hipError_t launch_begin(const ff_paths& P, const ff_begin& B, hipStream_t s);
+hipError_t launch_batch_begin(const ff_paths& P, hipStream_t s);
 hipError_t launch_generate(const ff_paths& P, hipStream_t s);
 hipError_t launch_extend(const ff_paths& P, int q, hipStream_t s);
 hipError_t launch_shadow(const ff_paths& P, hipStream_t s);
-hipError_t launch_reset(uint32_t* counters, uint32_t mask, uint32_t* fetch, uint32_t fetch_mask, hipStream_t s);
+hipError_t launch_extend_shadow(const ff_paths& P, int q, hipStream_t s);
 hipError_t launch_logic(const ff_paths& P, int q, int iter, uint32_t n_max, hipStream_t s);
 hipError_t launch_shade(int type, const ff_paths& P, int next_q, int first, uint32_t n_max, hipStream_t s);
 hipError_t launch_logic_adj(const ff_paths& P, int q, uint32_t n_max, hipStream_t s);
@@ -32,7 +33,6 @@ hipError_t launch_fixed_to_float(const unsigned long long* fx, const uint32_t* m
                                  float* out, hipStream_t s);
 hipError_t launch_fill4(float4* p, uint32_t n, hipStream_t s);
 hipError_t launch_fill_u32(uint32_t* p, uint64_t n, hipStream_t s);
-hipError_t launch_fill_u64(unsigned long long* p, uint32_t n, hipStream_t s);
 hipError_t launch_resolve_layers(const float4* layers, uint32_t K, uint32_t WH, float4* film, hipStream_t s);
 hipError_t launch_trace_closest(const ff_dev_scene& S, const float4* rays, uint32_t n,
                                 float4* hits, int two_sided, uint32_t* fetch, int32_t* ovf,

@@ -10,6 +10,7 @@
 // launches is identical from batch to batch and can be replayed as a graph.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <map>
 #include <mutex>
 #include <utility>
@@ -73,20 +74,19 @@ __device__ __forceinline__ uint32_t find_req(const ff_dev_request* __restrict__ 
 }
 
 // ============================================================ batch state
-// Starts a batch: batch index += 1 (or = value), queue and work counters
+// Starts a batch: batch index += 1, queue and work counters
 // cleared, and the extension queue laid out for the batch's new samples:
 // request r's active slots (its first min(K, spp - b*K) layers, a contiguous
 // slot range) occupy queue entries [qbase[r], qbase[r] + count), so
 // generate places every path without an atomic.
-__global__ void k_batch_begin(ff_paths P, int set, uint32_t value) {
+__global__ void k_batch_begin(ff_paths P) {
     uint32_t i = threadIdx.x;
     if (i < C_COUNT) P.counters[i] = 0;
     for (uint32_t k = i; k < 3 * FETCH_SEGS; k += blockDim.x) P.fetch[(size_t)k * FETCH_STRIDE] = 0;
     __syncthreads();
     if (i == 0) {
-        uint32_t b = set ? value : P.bstate[B_BATCH] + 1u;
+        uint32_t b = P.bstate[B_BATCH] + 1u;
         P.bstate[B_BATCH] = b;
-        if (set) return;  // (re)initialisation only
         uint32_t q = 0;
         for (uint32_t r = 0; r < P.n_req; r++) {
             const ff_dev_request& R = P.reqs[r];
@@ -97,6 +97,19 @@ __global__ void k_batch_begin(ff_paths P, int set, uint32_t value) {
         }
         P.qbase[P.n_req] = q;
         P.counters[C_EXT0] = q;
+    }
+}
+// Starts a pass over the batches: the next k_batch_begin makes the batch index
+// 0.  A call of one request carries it (and its gradient targets) here, so that
+// the host waits for nothing before it launches the call.
+__global__ __launch_bounds__(FF_BLOCK) void k_begin(ff_paths P, ff_begin B) {
+    if (threadIdx.x == 0) P.bstate[B_BATCH] = 0xffffffffu;
+    if (B.clear_stats)
+        for (uint32_t i = threadIdx.x; i < S_WORDS; i += FF_BLOCK) P.stats[i] = 0ull;
+    if (B.n_req) {
+        uint32_t* dst = (uint32_t*)P.reqs;
+        for (uint32_t i = threadIdx.x; i < sizeof(ff_dev_request) / 4; i += FF_BLOCK) dst[i] = ((const uint32_t*)&B.req)[i];
+        if (threadIdx.x < (uint32_t)B.n_gt) B.gt_dst[threadIdx.x] = B.gt[threadIdx.x];
     }
 }
 
@@ -144,7 +157,7 @@ template <bool UNI>
 struct ExtSrc {  // wf_extend (CRT/kernel.cu:487-523): closest hit of every queued path
     static constexpr bool kUniform = UNI;
     static constexpr bool kChain = false;
-    ff_paths P;
+    const ff_paths& P;
     const uint32_t* queue;
     __device__ __forceinline__ const ff_dev_scene& scene(uint32_t id) const {
         return UNI ? P.reqs[0].S : P.reqs[req_of(P, id)].S;
@@ -178,7 +191,7 @@ template <bool UNI>
 struct ShadowSrc {  // wf_shadow (CRT/kernel.cu:525-543): any hit of every queued shadow ray
     static constexpr bool kUniform = UNI;
     static constexpr bool kChain = true;
-    ff_paths P;
+    const ff_paths& P;
     __device__ __forceinline__ const ff_dev_scene& scene(uint32_t id) const {
         return UNI ? P.reqs[0].S : P.reqs[req_of(P, id)].S;
     }
@@ -503,12 +516,12 @@ constexpr uint32_t TW_SPREAD = 2048, QUAD_SPREAD = 1024;
 // walks on; the held triangles are tested together once LEAF lanes hold one,
 // or when no lane can walk on.
 template <int BS, bool ANY, class Src>
-__device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t* fetch, int32_t* ovf,
-                                          unsigned long long* cnt, int* smem) {
+__device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t block, uint32_t* fetch,
+                                          int32_t* ovf, unsigned long long* cnt, int* smem) {
     constexpr uint32_t IDLE = 0xffffffffu;
     constexpr int LDS = FF_LDS_STACK;
     SegFetch F;
-    F.init(fetch, n, blockIdx.x * (BS / 64) + (threadIdx.x >> 6));
+    F.init(fetch, n, block * (BS / 64) + (threadIdx.x >> 6));
     Stack st;
     st.lds = (lds_int*)&smem[threadIdx.x];
     st.lds_stride = BS;
@@ -716,11 +729,11 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t* 
 // overflow area: the launcher takes this walk only where LDS * 4 entries hold
 // the deepest stack).
 template <int BS, bool ANY, class Src>
-__device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t* fetch,
+__device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t block, uint32_t* fetch,
                                           unsigned long long* cnt, int* smem) {
     constexpr uint32_t IDLE = 0xffffffffu;
     SegFetch F;
-    F.init(fetch, n, blockIdx.x * (BS / 64) + (threadIdx.x >> 6));
+    F.init(fetch, n, block * (BS / 64) + (threadIdx.x >> 6));
     const uint32_t lane = __lane_id(), k = lane & 3u, lead = lane & ~3u;
     const uint64_t below = ((1ull << lead) - 1ull) & 0x1111111111111111ull;
     QuadStack<BS> st;
@@ -877,36 +890,84 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t* 
     src.count(lane == 0 ? c_rays : 0u, lane == 0 ? c_gated : 0u);
 }
 
+// block: the workgroup's number among those that draw from the same queue (its
+// waves start on the queue's segments in turn)
 template <bool ANY, class Src>
-__device__ __forceinline__ void traverse(const Src& src, uint32_t n, bool quad, uint32_t* fetch, int32_t* ovf,
-                                         unsigned long long* cnt, int* smem) {
-    if (quad && n <= QUAD_MAX) trav_quad<TW_BLOCK, ANY>(src, n, fetch, cnt, smem);
-    else trav_wide<TW_BLOCK, ANY>(src, n, fetch, ovf, cnt, smem);
+__device__ __forceinline__ void traverse(const Src& src, uint32_t n, uint32_t block, bool quad, uint32_t* fetch,
+                                         int32_t* ovf, unsigned long long* cnt, int* smem) {
+    if (quad && n <= QUAD_MAX) trav_quad<TW_BLOCK, ANY>(src, n, block, fetch, cnt, smem);
+    else trav_wide<TW_BLOCK, ANY>(src, n, block, fetch, ovf, cnt, smem);
 }
 // LDS words of a traversal workgroup: the stacks, for closest hits the hit words too
 constexpr int TW_LDS_ANY = FF_LDS_STACK * TW_BLOCK, TW_LDS_CLOSEST = (FF_LDS_STACK + 3) * TW_BLOCK;
 
+// SMALL: a call with at most QUAD_MAX paths in flight
+template <bool UNI, bool SMALL>
+__device__ __forceinline__ void extend_rays(const ff_paths& P, int q, uint32_t block, int* smem) {
+    // the counters that the coming stages of the iteration add to (nothing
+    // reads them during the traversal; those it reads are cleared by the logic)
+    if (block == 0 && threadIdx.x < 5)
+        P.counters[threadIdx.x < 4 ? C_MAT0 + threadIdx.x : (q == 0 ? C_EXT1 : C_EXT0)] = 0u;
+    const ExtSrc<UNI> src{P, P.q_ext[q]};
+    const uint32_t n = P.counters[q == 0 ? C_EXT0 : C_EXT1];
+    uint32_t* const fetch = P.fetch + F_EXT * FETCH_SEGS * FETCH_STRIDE;
+    unsigned long long* const cnt = stats_rep(P) + S_EXT_NODES;
+    if (SMALL) trav_quad<TW_BLOCK, false>(src, n, block, fetch, cnt, smem);
+    else traverse<false>(src, n, block, P.quad != 0, fetch, P.ovf, cnt, smem);
+}
+template <bool UNI, bool SMALL>
+__device__ __forceinline__ void shadow_rays(const ff_paths& P, uint32_t block, int* smem) {
+    const ShadowSrc<UNI> src{P};
+    const uint32_t n = P.counters[C_SHADOW];
+    uint32_t* const fetch = P.fetch + F_SHD * FETCH_SEGS * FETCH_STRIDE;
+    unsigned long long* const cnt = stats_rep(P) + S_SHD_NODES;
+    if (SMALL) trav_quad<TW_BLOCK, true>(src, n, block, fetch, cnt, smem);
+    else traverse<true>(src, n, block, P.quad != 0, fetch, P.ovf_shd, cnt, smem);
+}
 template <bool UNI>
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_CLOSEST];
-    ExtSrc<UNI> src{P, P.q_ext[q]};
-    traverse<false>(src, P.counters[q == 0 ? C_EXT0 : C_EXT1], P.quad != 0, P.fetch + F_EXT * FETCH_SEGS * FETCH_STRIDE,
-                    P.ovf, stats_rep(P) + S_EXT_NODES, smem);
+    extend_rays<UNI, false>(P, q, blockIdx.x, smem);
 }
 template <bool UNI>
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_shadow(ff_paths P) {
     __shared__ int smem[TW_LDS_ANY];
-    ShadowSrc<UNI> src{P};
-    traverse<true>(src, P.counters[C_SHADOW], P.quad != 0, P.fetch + F_SHD * FETCH_SEGS * FETCH_STRIDE, P.ovf_shd,
-                   stats_rep(P) + S_SHD_NODES, smem);
+    shadow_rays<UNI, false>(P, blockIdx.x, smem);
+}
+// An iteration's extension rays and its vertices' shadow rays (both come from
+// the previous shading pass) in one launch: workgroups alternate between the
+// two queues by eights (one to each XCD), and each goes on to the other queue,
+// so that either queue's waves fill the other's tail.
+template <bool UNI>
+__global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend_shadow(ff_paths P, int q) {
+    __shared__ int smem[TW_LDS_CLOSEST];
+    const uint32_t block = (blockIdx.x >> 4) * 8u + (blockIdx.x & 7u);
+    for (uint32_t ph = 0; ph < 2; ph++) {
+        if ((((blockIdx.x >> 3) + ph) & 1u) == 0u) extend_rays<UNI, false>(P, q, block, smem);
+        else shadow_rays<UNI, false>(P, block, smem);
+    }
+}
+// The same for a call with at most QUAD_MAX paths in flight: each queue has
+// workgroups enough, so they keep to one, and hold the four-lane walk only.
+template <bool UNI>
+__global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend_shadow_small(ff_paths P, int q) {
+    __shared__ int smem[TW_LDS_ANY];
+    const uint32_t block = (blockIdx.x >> 4) * 8u + (blockIdx.x & 7u);
+    if (blockIdx.x & 8u) shadow_rays<UNI, true>(P, block, smem);
+    else extend_rays<UNI, true>(P, q, block, smem);
 }
 
-// counters consumed by the previous stages are cleared by a kernel (graph-safe):
-// queue counters by `mask`, traversal work counters by kind (`fetch_mask`)
-__global__ void k_reset_counters(uint32_t* c, uint32_t mask, uint32_t* fetch, uint32_t fetch_mask) {
-    uint32_t i = threadIdx.x;
-    if (c && i < C_COUNT && ((mask >> i) & 1u)) c[i] = 0;
-    if (fetch && i < 3 * FETCH_SEGS && ((fetch_mask >> (i / FETCH_SEGS)) & 1u)) fetch[(size_t)i * FETCH_STRIDE] = 0;
+// clears the work counters of the standalone traces (a kernel: graph-safe)
+__global__ void k_reset_fetch(uint32_t* fetch) {
+    if (threadIdx.x < FETCH_SEGS) fetch[(size_t)(F_TRACE * FETCH_SEGS + threadIdx.x) * FETCH_STRIDE] = 0;
+}
+// the counters that the iteration's traversals have consumed, cleared by the
+// first workgroup of the logic that follows them
+__device__ __forceinline__ void clear_traversed(const ff_paths& P) {
+    if (blockIdx.x != 0) return;
+    static_assert(F_EXT == 0 && F_SHD == 1 && 2 * FETCH_SEGS <= FF_BLOCK, "one thread per work counter");
+    if (threadIdx.x < 2 * FETCH_SEGS) P.fetch[(size_t)threadIdx.x * FETCH_STRIDE] = 0;
+    if (threadIdx.x == 0) P.counters[C_SHADOW] = 0;
 }
 
 // =================================================================== logic
@@ -935,6 +996,7 @@ __global__ __launch_bounds__(FF_BLOCK, NP == 1 ? 8 : 5) void k_logic(ff_paths P,
     const int qidx[4] = {C_MAT0, C_MAT0 + 1, C_MAT0 + 2, C_MAT0 + 3};
     uint32_t* const qs[4] = {P.q_mat[0], P.q_mat[1], P.q_mat[2], P.q_mat[3]};
     st.init();
+    clear_traversed(P);
     const uint32_t n = P.counters[q == 0 ? C_EXT0 : C_EXT1];
     const uint32_t* queue = P.q_ext[q];
     const bool first_batch = P.bstate[B_BATCH] == 0;
@@ -1496,6 +1558,7 @@ __global__ __launch_bounds__(FF_BLOCK) void k_logic_adj(ff_paths P, int q) {
     const int qidx[4] = {C_MAT0, C_MAT0 + 1, C_MAT0 + 2, C_MAT0 + 3};
     uint32_t* const qs[4] = {P.q_mat[0], P.q_mat[1], P.q_mat[2], P.q_mat[3]};
     st.init();
+    clear_traversed(P);
     const uint32_t n = P.counters[q == 0 ? C_EXT0 : C_EXT1];
     const uint32_t* queue = P.q_ext[q];
     const uint32_t n_round = (n + FF_BLOCK - 1) / FF_BLOCK * FF_BLOCK;  // uniform trip count per workgroup
@@ -1686,9 +1749,6 @@ __global__ void k_fill4(float4* p, uint32_t n) {
 __global__ void k_fill_u32(uint32_t* p, uint64_t n) {
     for (uint64_t i = gtid(); i < n; i += gstride()) p[i] = 0u;
 }
-__global__ void k_fill_u64(unsigned long long* p, uint32_t n) {
-    for (uint32_t i = gtid(); i < n; i += gstride()) p[i] = 0ull;
-}
 // film[pixel] += sum over layers k (in k order) of layers[k*WH + pixel]
 __global__ void k_resolve_layers(const float4* layers, uint32_t K, uint32_t WH, float4* film) {
     for (uint32_t p = gtid(); p < WH; p += gstride()) {
@@ -1730,12 +1790,12 @@ __global__ __launch_bounds__(BS) void k_trace_any(TraceArgs a) {
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_trace_closest_wide(TraceArgs a) {
     __shared__ int smem[TW_LDS_CLOSEST];
     RaySrc src{a.S, a.rays, a.hits, nullptr, a.two_sided};
-    traverse<false>(src, a.n, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
+    traverse<false>(src, a.n, blockIdx.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
 }
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_trace_any_wide(TraceArgs a) {
     __shared__ int smem[TW_LDS_ANY];
     RaySrc src{a.S, a.rays, nullptr, a.occ, 0};
-    traverse<true>(src, a.n, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
+    traverse<true>(src, a.n, blockIdx.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
 }
 __global__ void k_gen_rays(ff_dev_camera cam, int32_t W, int32_t H, uint32_t seed, uint32_t sample,
                            float4* rays) {
@@ -1910,8 +1970,8 @@ uint32_t resident_grid(K kernel, int bs) {
     return (uint32_t)g;
 }
 
-// Workgroups of a wide traversal launch of at most n_max rays: the resident
-// ones, or as many as such a launch spreads its rays over.
+// Workgroups of a wide traversal launch of at most n_max rays a queue: the
+// resident ones, or as many as such a launch spreads its rays over.
 template <class K>
 uint32_t traverse_grid(K kernel, uint32_t n_max) {
     const uint32_t res = resident_grid(kernel, TW_BLOCK);
@@ -2049,8 +2109,12 @@ const int kTravWidth[] = {FF_TRAV_VARIANT_LIST(FF_TRAV_WIDTH)};
 // every request of the call shades the same scene and environment
 static bool uni_shading(const ff_paths& P) { return P.uni_scene && P.uni_env; }
 
-hipError_t launch_batch_begin(const ff_paths& P, int set, uint32_t value, hipStream_t s) {
-    hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(256), 0, s, P, set, value);
+hipError_t launch_begin(const ff_paths& P, const ff_begin& B, hipStream_t s) {
+    hipLaunchKernelGGL(k_begin, dim3(1), dim3(FF_BLOCK), 0, s, P, B);
+    return hipGetLastError();
+}
+hipError_t launch_batch_begin(const ff_paths& P, hipStream_t s) {
+    hipLaunchKernelGGL(k_batch_begin, dim3(1), dim3(256), 0, s, P);
     return hipGetLastError();
 }
 hipError_t launch_generate(const ff_paths& P, hipStream_t s) {
@@ -2071,15 +2135,30 @@ hipError_t launch_shadow(const ff_paths& P, hipStream_t s) {
         hipLaunchKernelGGL(k_shadow<false>, dim3(traverse_grid(k_shadow<false>, P.n_slots)), dim3(TW_BLOCK), 0, s, P);
     return hipGetLastError();
 }
+template <bool UNI>
+hipError_t extend_shadow_launch(const ff_paths& P, int q, hipStream_t s) {
+    if (P.n_slots <= QUAD_MAX && P.quad) {
+        const uint32_t g = (traverse_grid(k_extend_shadow_small<UNI>, P.n_slots) + 7u) / 8u * 16u;
+        hipLaunchKernelGGL(k_extend_shadow_small<UNI>, dim3(g), dim3(TW_BLOCK), 0, s, P, q);
+    } else {
+        const uint32_t g = std::min((traverse_grid(k_extend_shadow<UNI>, P.n_slots) + 7u) / 8u * 16u,
+                                    resident_grid(k_extend_shadow<UNI>, TW_BLOCK));
+        hipLaunchKernelGGL(k_extend_shadow<UNI>, dim3(g), dim3(TW_BLOCK), 0, s, P, q);
+    }
+    return hipGetLastError();
+}
+hipError_t launch_extend_shadow(const ff_paths& P, int q, hipStream_t s) {
+    return P.uni_scene ? extend_shadow_launch<true>(P, q, s) : extend_shadow_launch<false>(P, q, s);
+}
 void prepare_traversal() {
     (void)resident_grid(k_extend<true>, TW_BLOCK);
     (void)resident_grid(k_extend<false>, TW_BLOCK);
     (void)resident_grid(k_shadow<true>, TW_BLOCK);
     (void)resident_grid(k_shadow<false>, TW_BLOCK);
-}
-hipError_t launch_reset(uint32_t* counters, uint32_t mask, uint32_t* fetch, uint32_t fetch_mask, hipStream_t s) {
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(256), 0, s, counters, mask, fetch, fetch_mask);
-    return hipGetLastError();
+    (void)resident_grid(k_extend_shadow<true>, TW_BLOCK);
+    (void)resident_grid(k_extend_shadow<false>, TW_BLOCK);
+    (void)resident_grid(k_extend_shadow_small<true>, TW_BLOCK);
+    (void)resident_grid(k_extend_shadow_small<false>, TW_BLOCK);
 }
 template <bool UNI>
 hipError_t logic_launch(const ff_paths& P, int q, int iter, uint32_t n_max, hipStream_t s) {
@@ -2154,10 +2233,6 @@ hipError_t launch_fill_u32(uint32_t* p, uint64_t n, hipStream_t s) {
     hipLaunchKernelGGL(k_fill_u32, dim3(grid_for(n, FF_GRID_CAP)), dim3(FF_BLOCK), 0, s, p, n);
     return hipGetLastError();
 }
-hipError_t launch_fill_u64(unsigned long long* p, uint32_t n, hipStream_t s) {
-    hipLaunchKernelGGL(k_fill_u64, dim3(grid_for(n, FF_GRID_CAP)), dim3(FF_BLOCK), 0, s, p, n);
-    return hipGetLastError();
-}
 hipError_t launch_resolve_layers(const float4* layers, uint32_t K, uint32_t WH, float4* film, hipStream_t s) {
     hipLaunchKernelGGL(k_resolve_layers, dim3(grid_for(WH, FF_GRID_CAP)), dim3(FF_BLOCK), 0, s, layers, K, WH,
                        film);
@@ -2166,7 +2241,7 @@ hipError_t launch_resolve_layers(const float4* layers, uint32_t K, uint32_t WH, 
 hipError_t launch_trace_closest(const ff_dev_scene& S, const float4* rays, uint32_t n, float4* hits,
                                 int two_sided, uint32_t* fetch, int32_t* ovf, unsigned long long* counts,
                                 int variant, hipStream_t s) {
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(256), 0, s, nullptr, 0u, fetch, 1u << F_TRACE);
+    hipLaunchKernelGGL(k_reset_fetch, dim3(1), dim3(64), 0, s, fetch);
     TraceArgs T{S, rays, n, hits, nullptr, two_sided, fetch + F_TRACE * FETCH_SEGS * FETCH_STRIDE, ovf, counts};
     if (!counts && S.wide) {
         hipLaunchKernelGGL(k_trace_closest_wide, dim3(traverse_grid(k_trace_closest_wide, n)), dim3(TW_BLOCK), 0, s,
@@ -2202,7 +2277,7 @@ hipError_t static_scratch(int device, int32_t** out) {
 }
 hipError_t launch_trace_any(const ff_dev_scene& S, const float4* rays, uint32_t n, uint8_t* occ, uint32_t* fetch,
                             int32_t* ovf, unsigned long long* counts, int variant, hipStream_t s) {
-    hipLaunchKernelGGL(k_reset_counters, dim3(1), dim3(256), 0, s, nullptr, 0u, fetch, 1u << F_TRACE);
+    hipLaunchKernelGGL(k_reset_fetch, dim3(1), dim3(64), 0, s, fetch);
     TraceArgs T{S, rays, n, nullptr, occ, 0, fetch + F_TRACE * FETCH_SEGS * FETCH_STRIDE, ovf, counts};
     if (!counts && S.wide) {
         hipLaunchKernelGGL(k_trace_any_wide, dim3(traverse_grid(k_trace_any_wide, n)), dim3(TW_BLOCK), 0, s, T);

@@ -170,6 +170,16 @@ struct ff_dev_request {
     const ff_dev_gtarget* gt;  // adjoint: [1 + n_tex] targets (buf null = not wanted)
 };
 
+// What k_begin writes before a pass over the batches: for a call of one request
+// (n_req 1) the request itself and its gradient targets.
+#define FF_BEGIN_GT 16
+struct ff_begin {
+    ff_dev_request req;
+    ff_dev_gtarget gt[FF_BEGIN_GT];
+    ff_dev_gtarget* gt_dst;
+    int32_t n_req, n_gt, clear_stats;
+};
+
 // device-resident batch state (graph-replay safe): [0] batch index
 #define B_BATCH 0
 #define B_COUNT 4
