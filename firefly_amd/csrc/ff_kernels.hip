@@ -1506,47 +1506,91 @@ __global__ __launch_bounds__(FF_BLOCK) void k_shade(ff_paths P, int next_q, int 
 // MIS weights and Russian roulette are those of the forward.
 
 // One term of d loss / d parameter into gradient target element i.
-__device__ __forceinline__ void grad_add(const ff_paths& P, const ff_dev_gtarget& T, uint32_t i, float v) {
+__device__ __forceinline__ void grad_add(const ff_paths& P, float* buf, uint64_t off, uint32_t i, float v) {
     if (v == 0.f) return;
     if (P.gmode == GM_FLOAT) {
-        unsafeAtomicAdd(T.buf + i, v);
+        unsafeAtomicAdd(buf + i, v);
     } else if (P.gmode == GM_BOUND) {
-        uint64_t a = T.off + i;
+        uint64_t a = off + i;
         atomicMax(&P.g_max[a], __float_as_uint(fabsf(v)));
         atomicAdd(&P.g_cnt[a], 1u);
     } else {
-        uint64_t a = T.off + i;
+        uint64_t a = off + i;
         int e = fixed_exponent(P.g_max[a], P.g_cnt[a]);
         long long qv = __double2ll_rn(ldexp((double)v, e));
         atomicAdd(&P.g_fx[a], (unsigned long long)qv);
     }
 }
-// d loss / d Le(dir) = val (per channel) onto the environment texels
-__device__ __forceinline__ void grad_env(const ff_paths& P, const ff_dev_request& R, f3 dir, f3 val) {
-    const ff_dev_gtarget& T = R.gt[GT_ENV];
-    if (!T.buf) return;
-    float u, v;
-    sph_map(dir, u, v);
-    Taps tp = taps_of(R.E.w, R.E.h, u, v);
-#pragma unroll
-    for (int k = 0; k < 4; k++) {
-        grad_add(P, T, 3 * tp.i[k] + 0, tp.w[k] * val.x);
-        grad_add(P, T, 3 * tp.i[k] + 1, tp.w[k] * val.y);
-        grad_add(P, T, 3 * tp.i[k] + 2, tp.w[k] * val.z);
-    }
-}
-// d loss / d (texture t value at (u, v)) = val[0..c) onto its texels
+// Scatter of bilinear footprints onto gradient texels, the wave together.
+// Atomics run at the memory side at about 15 G requests/s, however many
+// elements a request carries.  With a lane issuing its footprint's 4 x C
+// elements one by one, each is a request of its own; here the footprints go
+// through LDS and consecutive lanes take consecutive elements, so the texels
+// of a row (2 C floats side by side) leave in one request.
+struct Scatter {  // of one wave
+    uint32_t idx[4][64];
+    float w[4][64];
+    float val[3][64];
+    float* buf[64];
+    uint64_t off[64];
+};
+// on: the lane has a footprint tp of target T with value val[0..C) (per
+// channel, before the tap weights).  Every lane of the wave calls it.
 template <int C>
-__device__ __forceinline__ void grad_tex(const ff_paths& P, const ff_dev_request& R, int t, float u, float v,
-                                         const float* val) {
-    const ff_dev_gtarget& T = R.gt[1 + t];
-    if (!T.buf) return;
-    const ff_tex_desc& td = R.S.tex[t];
-    Taps tp = taps_of(td.w, td.h, u, v);
+__device__ __forceinline__ void scatter(const ff_paths& P, Scatter& S, bool on, const ff_dev_gtarget& T,
+                                        const Taps& tp, f3 val) {
+    const uint64_t m = __ballot(on);
+    if (m == 0) return;
+    if (on) {
+        const uint32_t f = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 #pragma unroll
-    for (int k = 0; k < 4; k++)
-#pragma unroll
-        for (int c = 0; c < C; c++) grad_add(P, T, C * tp.i[k] + c, tp.w[k] * val[c]);
+        for (int k = 0; k < 4; k++) {
+            S.idx[k][f] = tp.i[k];
+            S.w[k][f] = tp.w[k];
+        }
+        S.val[0][f] = val.x;
+        S.val[1][f] = val.y;
+        S.val[2][f] = val.z;
+        S.buf[f] = T.buf;
+        S.off[f] = T.off;
+    }
+    __threadfence_block();
+    __builtin_amdgcn_wave_barrier();
+    const uint32_t total = (uint32_t)__popcll(m) * (4u * C);
+    for (uint32_t e = __lane_id(); e < total; e += 64u) {
+        const uint32_t f = e / (4u * C), r = e % (4u * C), k = r / C, c = r % C;
+        grad_add(P, S.buf[f], S.off[f], C * S.idx[k][f] + c, S.w[k][f] * S.val[c][f]);
+    }
+    __threadfence_block();
+    __builtin_amdgcn_wave_barrier();
+}
+// d loss / d Le(dir) = val (per channel) onto the environment texels
+__device__ __forceinline__ void scatter_env(const ff_paths& P, Scatter& S, bool on, const ff_dev_request& R, f3 dir,
+                                            f3 val) {
+    ff_dev_gtarget T{nullptr, 0};
+    Taps tp{};
+    if (on) T = R.gt[GT_ENV];
+    on = on && T.buf;
+    if (on) {
+        float u, v;
+        sph_map(dir, u, v);
+        tp = taps_of(R.E.w, R.E.h, u, v);
+    }
+    scatter<3>(P, S, on, T, tp, val);
+}
+// d loss / d (texture t value at (u, v)) = val (C channels) onto its texels
+template <int C>
+__device__ __forceinline__ void scatter_tex(const ff_paths& P, Scatter& S, bool on, const ff_dev_request& R, int t,
+                                            float u, float v, f3 val) {
+    ff_dev_gtarget T{nullptr, 0};
+    Taps tp{};
+    if (on) T = R.gt[1 + t];
+    on = on && T.buf;
+    if (on) {
+        const ff_tex_desc& td = R.S.tex[t];
+        tp = taps_of(td.w, td.h, u, v);
+    }
+    scatter<C>(P, S, on, T, tp, val);
 }
 
 // wf_logic of the replay: same termination, Russian roulette and routing as
@@ -1555,6 +1599,7 @@ __device__ __forceinline__ void grad_tex(const ff_paths& P, const ff_dev_request
 template <bool UNI>
 __global__ __launch_bounds__(FF_BLOCK) void k_logic_adj(ff_paths P, int q) {
     __shared__ QStage<FF_BLOCK, 4, QSTAGE_CAP> st;
+    __shared__ Scatter sc[FF_BLOCK / 64];
     const int qidx[4] = {C_MAT0, C_MAT0 + 1, C_MAT0 + 2, C_MAT0 + 3};
     uint32_t* const qs[4] = {P.q_mat[0], P.q_mat[1], P.q_mat[2], P.q_mat[3]};
     st.init();
@@ -1568,8 +1613,10 @@ __global__ __launch_bounds__(FF_BLOCK) void k_logic_adj(ff_paths P, int q) {
         int route = -1;
         bool term = false, primary = false;
         uint32_t id = live ? queue[i] : 0u;
+        bool esc = false;  // an escaped camera or delta ray: its Le term
+        f3 d = V3(0.f, 0.f, 0.f), gval = d;
+        const ff_dev_request& R = P.reqs[req_of(P, id)];
         if (live) {
-            const ff_dev_request& R = P.reqs[req_of(P, id)];
             const ff_dev_scene& S = scene_of<UNI>(P, R);
             float4 bw = P.beta[id];
             uint32_t stw = __float_as_uint(bw.w);
@@ -1583,7 +1630,6 @@ __global__ __launch_bounds__(FF_BLOCK) void k_logic_adj(ff_paths P, int q) {
             term = (len > R.depth) || !found || (stw & ST_DEAD);
             int mtype = -1;
             // the direction is read only by the two cases that use it
-            f3 d = V3(0.f, 0.f, 0.f);
             if ((found && (stw & ST_INSIDE)) || (!found && (stw & ST_PREV_DELTA))) d = xyz(P.ray[2 * id + 1]);
             if (found) {
                 mtype = (int)(S.mat[slot] >> MAT_TYPE_SHIFT);
@@ -1594,7 +1640,8 @@ __global__ __launch_bounds__(FF_BLOCK) void k_logic_adj(ff_paths P, int q) {
             }
             if (!found && (stw & ST_PREV_DELTA)) {
                 Lrem = vsub(Lrem, vmul(beta, env_L(env_view(env_of<UNI>(P, R)), d)));
-                grad_env(P, R, d, vmul(xyz(P.dlt[id]), beta));
+                esc = true;
+                gval = vmul(xyz(P.dlt[id]), beta);
             }
             if (!(stw & ST_DEAD) && len > 3) {
                 float qrr = fmaxf(0.05f, 1.f - beta.y);
@@ -1607,6 +1654,7 @@ __global__ __launch_bounds__(FF_BLOCK) void k_logic_adj(ff_paths P, int q) {
                 route = mtype;
             }
         }
+        scatter_env(P, sc[threadIdx.x >> 6], esc, R, d, gval);
         c_prim += (live && primary) ? 1u : 0u;
         c_ext += (live && !primary) ? 1u : 0u;
         c_paths += (live && term) ? 1u : 0u;
@@ -1663,6 +1711,7 @@ __global__ __launch_bounds__(FF_BLOCK) void k_shade_nee(ff_paths P) {
 // next extension ray.
 template <int TYPE, bool UNI>
 __global__ __launch_bounds__(FF_BLOCK) void k_shade_adj(ff_paths P, int next_q) {
+    __shared__ Scatter sc[TYPE == MAT_DIELECTRIC ? 1 : FF_BLOCK / 64];
     const uint32_t n = P.counters[C_MAT0 + TYPE];
     const uint32_t* queue = P.q_mat[TYPE];
     const uint32_t n_round = (n + FF_BLOCK - 1) / FF_BLOCK * FF_BLOCK;
@@ -1670,54 +1719,45 @@ __global__ __launch_bounds__(FF_BLOCK) void k_shade_adj(ff_paths P, int next_q) 
     for (uint32_t i = gtid(); i < n_round; i += gstride()) {
         bool live = i < n;
         uint32_t id = live ? queue[i] : 0u;
+        // what the vertex scatters: NEE terms onto the environment (light, spec,
+        // diffuse direction), NEE and continuation onto its albedo and roughness
+        const ff_dev_request& R = P.reqs[req_of(P, id)];
+        ShadeOut so;
+        bool visL = false, visS = false, visD = false, alb_on = false, rough_on = false;
+        f3 w = V3(0.f, 0.f, 0.f), g_alb = w, g_rough = w;
         if (live) {
-            const ff_dev_request& R = P.reqs[req_of(P, id)];
-            ShadeOut so;
             shade_core<TYPE, TYPE != MAT_DIELECTRIC, UNI>(P, id, so);
             f3 beta = xyz(P.beta[id]);
             uint32_t nst = so.nst;
             if (TYPE != MAT_DIELECTRIC) {
                 f3 Lrem = xyz(P.Lp[id]);
                 f3 dl = xyz(P.dlt[id]);
-                bool visL = so.needL && P.vis[3 * id + 0];
-                bool visS = visL && so.needS && P.vis[3 * id + 1];
-                bool visD = visL && so.needD && P.vis[3 * id + 2];
+                visL = so.needL && P.vis[3 * id + 0];
+                visS = visL && so.needS && P.vis[3 * id + 1];
+                visD = visL && so.needD && P.vis[3 * id + 2];
+                alb_on = so.at >= 0;
+                rough_on = so.rt >= 0 && so.rough_live;
                 if (visL) {
                     f3 lb = so.A;
                     if (visS) lb = vadd(lb, so.Bs);
                     if (visD) lb = vadd(lb, so.Cd);
                     Lrem = vsub(Lrem, vmul(lb, beta));
-                    f3 w = vmul(dl, beta);
-                    if (so.at >= 0) {
-                        f3 ga = so.dA_alb;
-                        if (visS) ga = vadd(ga, so.dB_alb);
-                        if (visD) ga = vadd(ga, so.dC_alb);
-                        float g3[3] = {w.x * ga.x, w.y * ga.y, w.z * ga.z};
-                        grad_tex<3>(P, R, so.at, so.tu, so.tv, g3);
-                    }
-                    if (so.rt >= 0 && so.rough_live) {
-                        f3 gr = so.dA_r;
-                        if (visS) gr = vadd(gr, so.dB_r);
-                        float g1 = vdot(w, gr);
-                        grad_tex<1>(P, R, so.rt, so.tu, so.tv, &g1);
-                    }
-                    if (so.a_on) grad_env(P, R, so.wi, vmul(w, so.kA));
-                    if (visS) grad_env(P, R, so.wi_s, vmul(w, so.kB));
-                    if (visD) grad_env(P, R, so.wi_d, vmul(w, so.kC));
+                    w = vmul(dl, beta);
+                    f3 ga = so.dA_alb;
+                    if (visS) ga = vadd(ga, so.dB_alb);
+                    if (visD) ga = vadd(ga, so.dC_alb);
+                    g_alb = vmul(w, ga);
+                    f3 gr = so.dA_r;
+                    if (visS) gr = vadd(gr, so.dB_r);
+                    g_rough.x = vdot(w, gr);
                 }
                 bool dead = vzero(so.fext) || so.pdf_ext == 0.f;
                 if (!dead) {
                     f3 qv = V3(so.fext.x != 0.f ? dl.x * Lrem.x / so.fext.x : 0.f,
                                so.fext.y != 0.f ? dl.y * Lrem.y / so.fext.y : 0.f,
                                so.fext.z != 0.f ? dl.z * Lrem.z / so.fext.z : 0.f);
-                    if (so.at >= 0) {
-                        float g3[3] = {qv.x * so.dext_alb.x, qv.y * so.dext_alb.y, qv.z * so.dext_alb.z};
-                        grad_tex<3>(P, R, so.at, so.tu, so.tv, g3);
-                    }
-                    if (so.rt >= 0 && so.rough_live) {
-                        float g1 = vdot(qv, so.dext_r);
-                        grad_tex<1>(P, R, so.rt, so.tu, so.tv, &g1);
-                    }
+                    g_alb = vadd(g_alb, vmul(qv, so.dext_alb));
+                    g_rough.x = g_rough.x + vdot(qv, so.dext_r);
                     beta = vmul(beta, vdiv(vscl(so.fext, so.cos_ext), so.pdf_ext));
                 }
                 nst = (nst & (ST_LEN_MASK | ST_INSIDE)) | (dead ? ST_DEAD : 0u);
@@ -1726,6 +1766,14 @@ __global__ __launch_bounds__(FF_BLOCK) void k_shade_adj(ff_paths P, int next_q) 
             P.beta[id] = f4(beta, __uint_as_float(nst));
             P.ray[2 * id] = f4(so.next_o, __uint_as_float(so.base));
             P.ray[2 * id + 1] = f4(so.next_d, __uint_as_float(nst));
+        }
+        if (TYPE != MAT_DIELECTRIC) {
+            Scatter& S = sc[threadIdx.x >> 6];
+            scatter_tex<3>(P, S, alb_on, R, so.at, so.tu, so.tv, g_alb);
+            if (TYPE != MAT_DIFFUSE) scatter_tex<1>(P, S, rough_on, R, so.rt, so.tu, so.tv, g_rough);
+            scatter_env(P, S, visL && so.a_on, R, so.wi, vmul(w, so.kA));
+            if (TYPE != MAT_DIFFUSE) scatter_env(P, S, visS, R, so.wi_s, vmul(w, so.kB));
+            if (TYPE != MAT_CONDUCTOR) scatter_env(P, S, visD, R, so.wi_d, vmul(w, so.kC));
         }
         if (live) P.q_ext[next_q][ebase + i] = id;
     }
