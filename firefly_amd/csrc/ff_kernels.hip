@@ -1318,11 +1318,13 @@ __device__ __forceinline__ void shade_core(const ff_paths& P, uint32_t id, Shade
     so.wi = wi;
     double diff_pdf = (double)(1.f / (2.f * F_PI));
     // light-sample term of BRDF_L (CRT/dMaterial.cu:376-402)
-    f3 Li = env_L(E, wi);
     float ndwi = vdot(nrm, wi);
     if (ndwi > 0.f) {
+        float eu, ev;
+        sph_map(wi, eu, ev);
+        f3 Li = env_L(E, eu, ev);
         double sp = do_spec ? (double)spec_pdf(nrm, wi, wo, rough) : 0.0;
-        double lp = (double)env_pdf(E, wi);
+        double lp = (double)env_pdf(E, wi, eu, ev);
         // lp is infinite where sin(acos(wi.z)) == 0; the term's limit there is 0
         if (lp > 0.f && lp < (double)INFINITY && !vzero(Li)) {
             double dwt = power_heur(lp, diff_pdf), swt = power_heur(lp, sp);
@@ -1364,11 +1366,13 @@ __device__ __forceinline__ void shade_core(const ff_paths& P, uint32_t id, Shade
     if (do_spec) {
         float nd = vdot(nrm, wi_s);
         if (nd > 0.f) {
+            float eu, ev;
+            sph_map(wi_s, eu, ev);
             double sp = (double)spec_pdf(nrm, wi_s, wo, rough);
-            double lp = (double)env_pdf(E, wi_s);
+            double lp = (double)env_pdf(E, wi_s, eu, ev);
             double wt = power_heur(sp, lp);
             f3 f = vscl(spec_f(nrm, wi_s, wo, rough, metal, alb, fres), nd);
-            f3 L2 = env_L(E, wi_s);
+            f3 L2 = env_L(E, eu, ev);
             if (!vzero(f) && sp > 0.f && !vzero(L2)) {
                 so.Bs = vdiv(vscl(vmul(f, L2), (float)wt), (float)sp);
                 so.needS = true;
@@ -1386,10 +1390,12 @@ __device__ __forceinline__ void shade_core(const ff_paths& P, uint32_t id, Shade
     if (do_diff) {
         float nd = vdot(nrm, wi_d);
         if (nd > 0.f) {
-            double lp = (double)env_pdf(E, wi_d);
+            float eu, ev;
+            sph_map(wi_d, eu, ev);
+            double lp = (double)env_pdf(E, wi_d, eu, ev);
             double wt = power_heur(diff_pdf, lp);
             f3 f = vscl(diff_f(wi_d, wo, metal, alb, fres), nd);
-            f3 L3 = env_L(E, wi_d);
+            f3 L3 = env_L(E, eu, ev);
             if (!vzero(f) && diff_pdf > 0.f && !vzero(L3)) {
                 so.Cd = vdiv(vscl(vmul(f, L3), (float)wt), (float)diff_pdf);
                 so.needD = true;
