@@ -652,7 +652,7 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         if (!ctx->own_stream) HIP_TRY(hipStreamCreate(&ctx->own_stream));
         hs = ctx->own_stream;
     }
-    ffk::prepare_traversal();
+    ffk::prepare_launches();
     ff_paths p = ctx->paths.p;
     const bool adjoint = (reqs[0].mode & RQ_ADJOINT) != 0;
     for (const HostReq& q : reqs)
@@ -820,19 +820,21 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         HIP_TRY(timed(4, [&] { return ffk::launch_generate(p, hs); }));
         int cur = 0;
         for (int32_t it = 1; it <= max_depth + 1; it++) {
-            // the iteration's extension rays and its vertices' shadow rays
-            // are independent: one launch traces both (with per-launch timing
-            // a launch each, so that each time is its own)
-            if (timing) {
-                HIP_TRY(timed(0, [&] { return ffk::launch_extend(p, cur, hs); }));
-                HIP_TRY(timed(1, [&] { return ffk::launch_shadow(p, hs); }));
-            } else {
+            // Two launches an iteration: its extension rays and its vertices'
+            // shadow rays are independent, and its paths are routed and shaded
+            // by one kernel.  With per-launch timing every stage is a launch of
+            // its own, so that each time is its own.
+            if (!timing) {
                 HIP_TRY(ffk::launch_extend_shadow(p, cur, hs));
-            }
-            HIP_TRY(timed(2, [&] { return ffk::launch_logic(p, cur, it, p.n_slots, hs); }));
-            if (it <= max_depth) {
-                for (int m = 0; m < 4; m++)
-                    if (has_type[m]) HIP_TRY(timed(3, [&] { return ffk::launch_shade(m, p, 1 - cur, it == 1, p.n_slots, hs); }));
+                HIP_TRY(ffk::launch_logic_shade(p, cur, it, it > max_depth, hs));
+            } else {
+                HIP_TRY(timed(0, [&] { return ffk::launch_extend(p, cur, hs); }));
+                HIP_TRY(timed(1, [&] { return ffk::launch_shadow(p, cur, hs); }));
+                HIP_TRY(timed(2, [&] { return ffk::launch_logic(p, cur, it, p.n_slots, hs); }));
+                if (it <= max_depth) {
+                    for (int m = 0; m < 4; m++)
+                        if (has_type[m]) HIP_TRY(timed(3, [&] { return ffk::launch_shade(m, p, 1 - cur, it == 1, p.n_slots, hs); }));
+                }
             }
             cur = 1 - cur;
         }
@@ -850,7 +852,7 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
             if (it <= max_depth) {
                 for (int m = 0; m < 3; m++)
                     if (has_type[m]) HIP_TRY(timed(3, [&] { return ffk::launch_shade_nee(m, p, p.n_slots, hs); }));
-                HIP_TRY(timed(1, [&] { return ffk::launch_shadow(p, hs); }));
+                HIP_TRY(timed(1, [&] { return ffk::launch_shadow(p, 0, hs); }));
                 for (int m = 0; m < 4; m++)
                     if (has_type[m])
                         HIP_TRY(timed(3, [&] { return ffk::launch_shade_adj(m, p, 1 - cur, p.n_slots, hs); }));

@@ -16,13 +16,14 @@ extern const int kTravBlock[];
 extern const int kTravRefill[];
 extern const int kTravWhileWhile[];
 extern const int kTravWidth[];  // BVH record width of the variant (2 or 4)
-// computes the grid sizes of the wavefront's traversal kernels (call before a graph capture)
-void prepare_traversal();
+// computes the grid sizes of the wavefront's resident kernels (call before a graph capture)
+void prepare_launches();
 hipError_t launch_begin(const ff_paths& P, const ff_begin& B, hipStream_t s);
 hipError_t launch_batch_begin(const ff_paths& P, hipStream_t s);
 hipError_t launch_generate(const ff_paths& P, hipStream_t s);
 hipError_t launch_extend(const ff_paths& P, int q, hipStream_t s);
-hipError_t launch_shadow(const ff_paths& P, hipStream_t s);
+hipError_t launch_shadow(const ff_paths& P, int q, hipStream_t s);
+hipError_t launch_logic_shade(const ff_paths& P, int q, int iter, int last, hipStream_t s);
 hipError_t launch_extend_shadow(const ff_paths& P, int q, hipStream_t s);
 hipError_t launch_logic(const ff_paths& P, int q, int iter, uint32_t n_max, hipStream_t s);
 hipError_t launch_shade(int type, const ff_paths& P, int next_q, int first, uint32_t n_max, hipStream_t s);

@@ -41,8 +41,9 @@
 // device counters
 #define C_EXT0 0
 #define C_EXT1 1
-#define C_SHADOW 2
+#define C_SHD0 2
 #define C_MAT0 3
+#define C_SHD1 7
 #define C_COUNT 16
 
 // Work counters of the persistent traversal kernels: the queue is split into
