@@ -28,8 +28,8 @@ hipError_t launch_extend_shadow(const ff_paths& P, int q, hipStream_t s);
 hipError_t launch_logic(const ff_paths& P, int q, int iter, uint32_t n_max, hipStream_t s);
 hipError_t launch_shade(int type, const ff_paths& P, int next_q, int first, uint32_t n_max, hipStream_t s);
 hipError_t launch_logic_adj(const ff_paths& P, int q, uint32_t n_max, hipStream_t s);
-hipError_t launch_shade_nee(int type, const ff_paths& P, uint32_t n_max, hipStream_t s);
-hipError_t launch_shade_adj(int type, const ff_paths& P, int next_q, uint32_t n_max, hipStream_t s);
+hipError_t launch_shade_nee(int type, const ff_paths& P, int next_q, uint32_t n_max, hipStream_t s);
+hipError_t launch_shade_adj(int type, const ff_paths& P, int q, uint32_t n_max, hipStream_t s);
 hipError_t launch_fixed_to_float(const unsigned long long* fx, const uint32_t* mx, const uint32_t* cnt, uint64_t n,
                                  float* out, hipStream_t s);
 hipError_t launch_fill4(float4* p, uint32_t n, hipStream_t s);

@@ -65,6 +65,7 @@ __device__ __forceinline__ uint32_t req_of(const ff_paths& P, uint32_t id) {
 // the queue counters of iteration parity q: entries traced in it
 __device__ __forceinline__ int ext_counter(int q) { return q == 0 ? C_EXT0 : C_EXT1; }
 __device__ __forceinline__ int shadow_counter(int q) { return q == 0 ? C_SHD0 : C_SHD1; }
+__device__ __forceinline__ int mat_counter(int q) { return q == 0 ? C_MAT0 : C_MAT1; }  // the first of four
 
 // request owning a slot: last r with slot_base <= id
 __device__ __forceinline__ uint32_t find_req(const ff_dev_request* __restrict__ reqs, uint32_t n, uint32_t id) {
@@ -911,7 +912,7 @@ __device__ __forceinline__ void extend_rays(const ff_paths& P, int q, uint32_t b
     // the counters that the coming stages of the iteration add to (nothing
     // reads them during the traversal; those it reads are cleared by the logic)
     if (block == 0 && threadIdx.x < 6)
-        P.counters[threadIdx.x < 4 ? C_MAT0 + threadIdx.x
+        P.counters[threadIdx.x < 4 ? mat_counter(q) + threadIdx.x
                                    : (threadIdx.x == 4 ? ext_counter(1 - q) : shadow_counter(1 - q))] = 0u;
     const ExtSrc<UNI> src{P, P.q_ext[q]};
     const uint32_t n = P.counters[ext_counter(q)];
@@ -1138,7 +1139,7 @@ __device__ __forceinline__ void add_counts(const ff_paths& P, const LogicCounts&
 template <bool UNI, int NP>
 __global__ __launch_bounds__(FF_BLOCK, NP == 1 ? 8 : 5) void k_logic(ff_paths P, int q, int iter) {
     __shared__ QStage<FF_BLOCK, 4, QSTAGE_CAP> st;
-    const int qidx[4] = {C_MAT0, C_MAT0 + 1, C_MAT0 + 2, C_MAT0 + 3};
+    const int qidx[4] = {mat_counter(q), mat_counter(q) + 1, mat_counter(q) + 2, mat_counter(q) + 3};
     uint32_t* const qs[4] = {P.q_mat[0], P.q_mat[1], P.q_mat[2], P.q_mat[3]};
     st.init();
     clear_traversed(P);
@@ -1168,17 +1169,20 @@ __global__ __launch_bounds__(FF_BLOCK, NP == 1 ? 8 : 5) void k_logic(ff_paths P,
 }
 
 // ======================================================= material queues
-// Every shaded event continues to the next extension stage, so the next
-// extension queue is the material queues one after another: material queue
-// TYPE starts after the entries of the types below it.  The first workgroup
-// adds the queue's length to the extension counter (one atomic per launch).
+// Every shaded event continues to the next extension stage, so the extension
+// queue of parity 1 - q is the material queues of q one after another: material
+// queue TYPE starts after the entries of the types below it.
 template <int TYPE>
-__device__ __forceinline__ uint32_t ext_base(const ff_paths& P, int next_q, uint32_t n) {
+__device__ __forceinline__ uint32_t ext_base(const ff_paths& P, int q) {
     uint32_t b = 0u;
 #pragma unroll
-    for (int t = 0; t < TYPE; t++) b += P.counters[C_MAT0 + t];
-    if (blockIdx.x == 0 && threadIdx.x == 0 && n) atomicAdd(&P.counters[ext_counter(next_q)], n);
+    for (int t = 0; t < TYPE; t++) b += P.counters[mat_counter(q) + t];
     return b;
+}
+// The first workgroup adds a material queue's n entries to the extension
+// counter (one atomic per launch).
+__device__ __forceinline__ void add_extensions(const ff_paths& P, int next_q, uint32_t n) {
+    if (blockIdx.x == 0 && threadIdx.x == 0 && n) atomicAdd(&P.counters[ext_counter(next_q)], n);
 }
 
 // Everything the shading of one vertex produces.  With GRAD the partial
@@ -1213,14 +1217,20 @@ struct ShadeOut {
 #define SW_RAY 2      // a later forward vertex: the ray's .w holds the previous
                       // shading word, which wf_logic turns into this vertex's
                       // word by adding one to the length and keeping the flags
+struct Vertex {
+    float4 hit, r0, r1;  // hit record; ray that found it
+};
+__device__ __forceinline__ Vertex load_vertex(const ff_paths& P, uint32_t id) {
+    return {P.hit[id], P.ray[2 * id], P.ray[2 * id + 1]};
+}
 template <int TYPE, bool GRAD, bool UNI>
-__device__ __forceinline__ void shade_core(const ff_paths& P, uint32_t id, ShadeOut& so, int sw_src = SW_RECORD) {
+__device__ __forceinline__ void shade_core(const ff_paths& P, uint32_t id, const Vertex& vx, ShadeOut& so,
+                                           int sw_src = SW_RECORD) {
     const ff_dev_request& R = P.reqs[req_of(P, id)];
     const ff_dev_scene& S = scene_of<UNI>(P, R);
     EnvView E = env_view(env_of<UNI>(P, R));
-    float4 hh = P.hit[id];
+    const float4 hh = vx.hit, r0 = vx.r0, r1 = vx.r1;
     int slot = __float_as_int(hh.w);
-    float4 r0 = P.ray[2 * id], r1 = P.ray[2 * id + 1];
     f3 o = xyz(r0), d = xyz(r1);
     uint32_t stw;
     if (sw_src == SW_START) {
@@ -1462,7 +1472,7 @@ __device__ __forceinline__ void shade_core(const ff_paths& P, uint32_t id, Shade
 template <int TYPE, bool UNI>
 __device__ __forceinline__ bool shade_path(const ff_paths& P, uint32_t id, bool first, uint32_t& shadow) {
     ShadeOut so;
-    shade_core<TYPE, false, UNI>(P, id, so, first ? SW_START : SW_RAY);
+    shade_core<TYPE, false, UNI>(P, id, load_vertex(P, id), so, first ? SW_START : SW_RAY);
     const bool needL = so.needL, needS = so.needS, needD = so.needD;
     if (needL) {
         P.sray[6 * id + 0] = f4(so.lo, 0.f);
@@ -1498,12 +1508,13 @@ __device__ __forceinline__ bool shade_path(const ff_paths& P, uint32_t id, bool 
 template <int TYPE, bool UNI>
 __global__ __launch_bounds__(FF_BLOCK) void k_shade(ff_paths P, int next_q, int first) {
     __shared__ QStage<FF_BLOCK, 1, QSTAGE_CAP> st;
-    const uint32_t n = P.counters[C_MAT0 + TYPE];
+    const uint32_t n = P.counters[mat_counter(1 - next_q) + TYPE];
     const uint32_t* queue = P.q_mat[TYPE];
     const uint32_t n_round = (n + FF_BLOCK - 1) / FF_BLOCK * FF_BLOCK;
     const int qidx[1] = {shadow_counter(next_q)};
     uint32_t* const qs[1] = {P.q_shadow};
-    const uint32_t ebase = ext_base<TYPE>(P, next_q, n);
+    const uint32_t ebase = ext_base<TYPE>(P, 1 - next_q);
+    add_extensions(P, next_q, n);
     st.init();
     for (uint32_t i = gtid(); i < n_round; i += gstride()) {
         const bool live = i < n;
@@ -1757,11 +1768,10 @@ template <bool UNI>
 __global__ __launch_bounds__(FF_BLOCK) void k_logic_adj(ff_paths P, int q) {
     __shared__ QStage<FF_BLOCK, 4, QSTAGE_CAP> st;
     __shared__ Scatter sc[FF_BLOCK / 64];
-    const int qidx[4] = {C_MAT0, C_MAT0 + 1, C_MAT0 + 2, C_MAT0 + 3};
+    const int qidx[4] = {mat_counter(q), mat_counter(q) + 1, mat_counter(q) + 2, mat_counter(q) + 3};
     uint32_t* const qs[4] = {P.q_mat[0], P.q_mat[1], P.q_mat[2], P.q_mat[3]};
     st.init();
     clear_traversed(P);
-    if (blockIdx.x == 0 && threadIdx.x == 0) P.counters[C_SHD0] = 0;  // traced by the previous vertex
     const uint32_t n = P.counters[ext_counter(q)];
     const uint32_t* queue = P.q_ext[q];
     const uint32_t n_round = (n + FF_BLOCK - 1) / FF_BLOCK * FF_BLOCK;  // uniform trip count per workgroup
@@ -1826,15 +1836,20 @@ __global__ __launch_bounds__(FF_BLOCK) void k_logic_adj(ff_paths P, int q) {
     wave_sum_add(sr + S_PATHS, c_paths);
 }
 
-// Replay of a vertex's shadow rays: the same rays k_shade queues.
+// Replay of a vertex's rays: the shadow rays and the continuation that k_shade
+// queues.  The vertex itself (its hit and the ray that found it) is kept in the
+// path's NEE terms, which the replay does not store, for k_shade_adj, which
+// follows the rays' traversal.  (A dielectric vertex has no more to replay.)
 template <int TYPE, bool UNI>
-__global__ __launch_bounds__(FF_BLOCK) void k_shade_nee(ff_paths P) {
+__global__ __launch_bounds__(FF_BLOCK) void k_shade_nee(ff_paths P, int next_q) {
     __shared__ QStage<FF_BLOCK, 1, QSTAGE_CAP> st;
-    const uint32_t n = P.counters[C_MAT0 + TYPE];
+    const uint32_t n = P.counters[mat_counter(1 - next_q) + TYPE];
     const uint32_t* queue = P.q_mat[TYPE];
     const uint32_t n_round = (n + FF_BLOCK - 1) / FF_BLOCK * FF_BLOCK;
-    const int qidx[1] = {C_SHD0};
+    const int qidx[1] = {shadow_counter(next_q)};
     uint32_t* const qs[1] = {P.q_shadow};
+    const uint32_t ebase = ext_base<TYPE>(P, 1 - next_q);
+    add_extensions(P, next_q, n);
     st.init();
     for (uint32_t i = gtid(); i < n_round; i += gstride()) {
         bool live = i < n;
@@ -1842,21 +1857,35 @@ __global__ __launch_bounds__(FF_BLOCK) void k_shade_nee(ff_paths P) {
         bool needL = false, needS = false, needD = false;
         if (live) {
             ShadeOut so;
-            shade_core<TYPE, false, UNI>(P, id, so);
-            needL = so.needL; needS = so.needS; needD = so.needD;
-            if (needL) {
-                P.sray[6 * id + 0] = f4(so.lo, 0.f);
-                P.sray[6 * id + 1] = f4(so.wi, 0.f);
+            const Vertex vx = load_vertex(P, id);
+            shade_core<TYPE, false, UNI>(P, id, vx, so);
+            uint32_t nst = so.nst;
+            if (TYPE != MAT_DIELECTRIC) {
+                needL = so.needL; needS = so.needS; needD = so.needD;
+                if (needL) {
+                    P.sray[6 * id + 0] = f4(so.lo, 0.f);
+                    P.sray[6 * id + 1] = f4(so.wi, 0.f);
+                }
+                if (needS) {
+                    P.sray[6 * id + 2] = f4(so.so, 0.f);
+                    P.sray[6 * id + 3] = f4(so.wi_s, 0.f);
+                }
+                if (needD) {
+                    P.sray[6 * id + 4] = f4(so.dd_o, 0.f);
+                    P.sray[6 * id + 5] = f4(so.wi_d, 0.f);
+                }
+                nst &= ST_LEN_MASK | ST_INSIDE;
+                P.nee[3 * id] = vx.hit;
+                P.nee[3 * id + 1] = vx.r0;
+                P.nee[3 * id + 2] = vx.r1;
+            } else {
+                P.beta[id].w = __uint_as_float(nst);
             }
-            if (needS) {
-                P.sray[6 * id + 2] = f4(so.so, 0.f);
-                P.sray[6 * id + 3] = f4(so.wi_s, 0.f);
-            }
-            if (needD) {
-                P.sray[6 * id + 4] = f4(so.dd_o, 0.f);
-                P.sray[6 * id + 5] = f4(so.wi_d, 0.f);
-            }
+            P.ray[2 * id] = f4(so.next_o, __uint_as_float(so.base));
+            P.ray[2 * id + 1] = f4(so.next_d, __uint_as_float(nst));
+            P.q_ext[next_q][ebase + i] = id;
         }
+        if (TYPE == MAT_DIELECTRIC) continue;
         st.add(needL ? 0 : -1, (id << 2) | (needS ? 1u : 0u) | (needD ? 2u : 0u));
         st.flush_if_full(P.counters, qidx, qs);
     }
@@ -1865,15 +1894,14 @@ __global__ __launch_bounds__(FF_BLOCK) void k_shade_nee(ff_paths P) {
 
 // Replay of a vertex once its shadow rays are traced: its visibility-gated
 // NEE terms leave L_rem (with their gradients), then the continuation's
-// gradient L_rem * (df/dtheta) / f, the throughput update of wf_logic and the
-// next extension ray.
+// gradient L_rem * (df/dtheta) / f and the throughput update of wf_logic.  The
+// paths are those of extension queue q's part for TYPE.
 template <int TYPE, bool UNI>
-__global__ __launch_bounds__(FF_BLOCK) void k_shade_adj(ff_paths P, int next_q) {
-    __shared__ Scatter sc[TYPE == MAT_DIELECTRIC ? 1 : FF_BLOCK / 64];
-    const uint32_t n = P.counters[C_MAT0 + TYPE];
-    const uint32_t* queue = P.q_mat[TYPE];
+__global__ __launch_bounds__(FF_BLOCK) void k_shade_adj(ff_paths P, int q) {
+    __shared__ Scatter sc[FF_BLOCK / 64];
+    const uint32_t n = P.counters[mat_counter(1 - q) + TYPE];
+    const uint32_t* queue = P.q_ext[q] + ext_base<TYPE>(P, 1 - q);
     const uint32_t n_round = (n + FF_BLOCK - 1) / FF_BLOCK * FF_BLOCK;
-    const uint32_t ebase = ext_base<TYPE>(P, next_q, n);
     for (uint32_t i = gtid(); i < n_round; i += gstride()) {
         bool live = i < n;
         uint32_t id = live ? queue[i] : 0u;
@@ -1884,56 +1912,49 @@ __global__ __launch_bounds__(FF_BLOCK) void k_shade_adj(ff_paths P, int next_q) 
         bool visL = false, visS = false, visD = false, alb_on = false, rough_on = false;
         f3 w = V3(0.f, 0.f, 0.f), g_alb = w, g_rough = w;
         if (live) {
-            shade_core<TYPE, TYPE != MAT_DIELECTRIC, UNI>(P, id, so);
+            shade_core<TYPE, true, UNI>(P, id, {P.nee[3 * id], P.nee[3 * id + 1], P.nee[3 * id + 2]}, so);
             f3 beta = xyz(P.beta[id]);
             uint32_t nst = so.nst;
-            if (TYPE != MAT_DIELECTRIC) {
-                f3 Lrem = xyz(P.Lp[id]);
-                f3 dl = xyz(P.dlt[id]);
-                visL = so.needL && P.vis[3 * id + 0];
-                visS = visL && so.needS && P.vis[3 * id + 1];
-                visD = visL && so.needD && P.vis[3 * id + 2];
-                alb_on = so.at >= 0;
-                rough_on = so.rt >= 0 && so.rough_live;
-                if (visL) {
-                    f3 lb = so.A;
-                    if (visS) lb = vadd(lb, so.Bs);
-                    if (visD) lb = vadd(lb, so.Cd);
-                    Lrem = vsub(Lrem, vmul(lb, beta));
-                    w = vmul(dl, beta);
-                    f3 ga = so.dA_alb;
-                    if (visS) ga = vadd(ga, so.dB_alb);
-                    if (visD) ga = vadd(ga, so.dC_alb);
-                    g_alb = vmul(w, ga);
-                    f3 gr = so.dA_r;
-                    if (visS) gr = vadd(gr, so.dB_r);
-                    g_rough.x = vdot(w, gr);
-                }
-                bool dead = vzero(so.fext) || so.pdf_ext == 0.f;
-                if (!dead) {
-                    f3 qv = V3(so.fext.x != 0.f ? dl.x * Lrem.x / so.fext.x : 0.f,
-                               so.fext.y != 0.f ? dl.y * Lrem.y / so.fext.y : 0.f,
-                               so.fext.z != 0.f ? dl.z * Lrem.z / so.fext.z : 0.f);
-                    g_alb = vadd(g_alb, vmul(qv, so.dext_alb));
-                    g_rough.x = g_rough.x + vdot(qv, so.dext_r);
-                    beta = vmul(beta, vdiv(vscl(so.fext, so.cos_ext), so.pdf_ext));
-                }
-                nst = (nst & (ST_LEN_MASK | ST_INSIDE)) | (dead ? ST_DEAD : 0u);
-                P.Lp[id] = f4(Lrem, 0.f);
+            f3 Lrem = xyz(P.Lp[id]);
+            f3 dl = xyz(P.dlt[id]);
+            visL = so.needL && P.vis[3 * id + 0];
+            visS = visL && so.needS && P.vis[3 * id + 1];
+            visD = visL && so.needD && P.vis[3 * id + 2];
+            alb_on = so.at >= 0;
+            rough_on = so.rt >= 0 && so.rough_live;
+            if (visL) {
+                f3 lb = so.A;
+                if (visS) lb = vadd(lb, so.Bs);
+                if (visD) lb = vadd(lb, so.Cd);
+                Lrem = vsub(Lrem, vmul(lb, beta));
+                w = vmul(dl, beta);
+                f3 ga = so.dA_alb;
+                if (visS) ga = vadd(ga, so.dB_alb);
+                if (visD) ga = vadd(ga, so.dC_alb);
+                g_alb = vmul(w, ga);
+                f3 gr = so.dA_r;
+                if (visS) gr = vadd(gr, so.dB_r);
+                g_rough.x = vdot(w, gr);
             }
+            bool dead = vzero(so.fext) || so.pdf_ext == 0.f;
+            if (!dead) {
+                f3 qv = V3(so.fext.x != 0.f ? dl.x * Lrem.x / so.fext.x : 0.f,
+                           so.fext.y != 0.f ? dl.y * Lrem.y / so.fext.y : 0.f,
+                           so.fext.z != 0.f ? dl.z * Lrem.z / so.fext.z : 0.f);
+                g_alb = vadd(g_alb, vmul(qv, so.dext_alb));
+                g_rough.x = g_rough.x + vdot(qv, so.dext_r);
+                beta = vmul(beta, vdiv(vscl(so.fext, so.cos_ext), so.pdf_ext));
+            }
+            nst = (nst & (ST_LEN_MASK | ST_INSIDE)) | (dead ? ST_DEAD : 0u);
+            P.Lp[id] = f4(Lrem, 0.f);
             P.beta[id] = f4(beta, __uint_as_float(nst));
-            P.ray[2 * id] = f4(so.next_o, __uint_as_float(so.base));
-            P.ray[2 * id + 1] = f4(so.next_d, __uint_as_float(nst));
         }
-        if (TYPE != MAT_DIELECTRIC) {
-            Scatter& S = sc[threadIdx.x >> 6];
-            scatter_tex<3>(P, S, alb_on, R, so.at, so.tu, so.tv, g_alb);
-            if (TYPE != MAT_DIFFUSE) scatter_tex<1>(P, S, rough_on, R, so.rt, so.tu, so.tv, g_rough);
-            scatter_env(P, S, visL && so.a_on, R, so.wi, vmul(w, so.kA));
-            if (TYPE != MAT_DIFFUSE) scatter_env(P, S, visS, R, so.wi_s, vmul(w, so.kB));
-            if (TYPE != MAT_CONDUCTOR) scatter_env(P, S, visD, R, so.wi_d, vmul(w, so.kC));
-        }
-        if (live) P.q_ext[next_q][ebase + i] = id;
+        Scatter& S = sc[threadIdx.x >> 6];
+        scatter_tex<3>(P, S, alb_on, R, so.at, so.tu, so.tv, g_alb);
+        if (TYPE != MAT_DIFFUSE) scatter_tex<1>(P, S, rough_on, R, so.rt, so.tu, so.tv, g_rough);
+        scatter_env(P, S, visL && so.a_on, R, so.wi, vmul(w, so.kA));
+        if (TYPE != MAT_DIFFUSE) scatter_env(P, S, visS, R, so.wi_s, vmul(w, so.kB));
+        if (TYPE != MAT_CONDUCTOR) scatter_env(P, S, visD, R, so.wi_d, vmul(w, so.kC));
     }
 }
 
@@ -2425,33 +2446,34 @@ hipError_t launch_logic_adj(const ff_paths& P, int q, uint32_t n_max, hipStream_
     return uni_shading(P) ? logic_adj_launch<true>(P, q, n_max, s) : logic_adj_launch<false>(P, q, n_max, s);
 }
 template <bool UNI>
-hipError_t shade_nee_launch(int type, const ff_paths& P, uint32_t n_max, hipStream_t s) {
+hipError_t shade_nee_launch(int type, const ff_paths& P, int next_q, uint32_t n_max, hipStream_t s) {
     dim3 g(grid_for(n_max, FF_GRID_CAP)), b(FF_BLOCK);
     switch (type) {
-        case MAT_MIX: hipLaunchKernelGGL((k_shade_nee<MAT_MIX, UNI>), g, b, 0, s, P); break;
-        case MAT_DIFFUSE: hipLaunchKernelGGL((k_shade_nee<MAT_DIFFUSE, UNI>), g, b, 0, s, P); break;
-        case MAT_CONDUCTOR: hipLaunchKernelGGL((k_shade_nee<MAT_CONDUCTOR, UNI>), g, b, 0, s, P); break;
-        default: return hipSuccess;  // a dielectric vertex has no NEE rays
+        case MAT_MIX: hipLaunchKernelGGL((k_shade_nee<MAT_MIX, UNI>), g, b, 0, s, P, next_q); break;
+        case MAT_DIFFUSE: hipLaunchKernelGGL((k_shade_nee<MAT_DIFFUSE, UNI>), g, b, 0, s, P, next_q); break;
+        case MAT_CONDUCTOR: hipLaunchKernelGGL((k_shade_nee<MAT_CONDUCTOR, UNI>), g, b, 0, s, P, next_q); break;
+        default: hipLaunchKernelGGL((k_shade_nee<MAT_DIELECTRIC, UNI>), g, b, 0, s, P, next_q); break;
     }
     return hipGetLastError();
 }
-hipError_t launch_shade_nee(int type, const ff_paths& P, uint32_t n_max, hipStream_t s) {
-    return uni_shading(P) ? shade_nee_launch<true>(type, P, n_max, s) : shade_nee_launch<false>(type, P, n_max, s);
+hipError_t launch_shade_nee(int type, const ff_paths& P, int next_q, uint32_t n_max, hipStream_t s) {
+    return uni_shading(P) ? shade_nee_launch<true>(type, P, next_q, n_max, s)
+                          : shade_nee_launch<false>(type, P, next_q, n_max, s);
 }
 template <bool UNI>
-hipError_t shade_adj_launch(int type, const ff_paths& P, int next_q, uint32_t n_max, hipStream_t s) {
+hipError_t shade_adj_launch(int type, const ff_paths& P, int q, uint32_t n_max, hipStream_t s) {
     dim3 g(grid_for(n_max, FF_GRID_CAP)), b(FF_BLOCK);
     switch (type) {
-        case MAT_MIX: hipLaunchKernelGGL((k_shade_adj<MAT_MIX, UNI>), g, b, 0, s, P, next_q); break;
-        case MAT_DIFFUSE: hipLaunchKernelGGL((k_shade_adj<MAT_DIFFUSE, UNI>), g, b, 0, s, P, next_q); break;
-        case MAT_CONDUCTOR: hipLaunchKernelGGL((k_shade_adj<MAT_CONDUCTOR, UNI>), g, b, 0, s, P, next_q); break;
-        default: hipLaunchKernelGGL((k_shade_adj<MAT_DIELECTRIC, UNI>), g, b, 0, s, P, next_q); break;
+        case MAT_MIX: hipLaunchKernelGGL((k_shade_adj<MAT_MIX, UNI>), g, b, 0, s, P, q); break;
+        case MAT_DIFFUSE: hipLaunchKernelGGL((k_shade_adj<MAT_DIFFUSE, UNI>), g, b, 0, s, P, q); break;
+        case MAT_CONDUCTOR: hipLaunchKernelGGL((k_shade_adj<MAT_CONDUCTOR, UNI>), g, b, 0, s, P, q); break;
+        default: break;  // a dielectric vertex ends with its rays
     }
     return hipGetLastError();
 }
-hipError_t launch_shade_adj(int type, const ff_paths& P, int next_q, uint32_t n_max, hipStream_t s) {
-    return uni_shading(P) ? shade_adj_launch<true>(type, P, next_q, n_max, s)
-                          : shade_adj_launch<false>(type, P, next_q, n_max, s);
+hipError_t launch_shade_adj(int type, const ff_paths& P, int q, uint32_t n_max, hipStream_t s) {
+    return uni_shading(P) ? shade_adj_launch<true>(type, P, q, n_max, s)
+                          : shade_adj_launch<false>(type, P, q, n_max, s);
 }
 hipError_t launch_fixed_to_float(const unsigned long long* fx, const uint32_t* mx, const uint32_t* cnt, uint64_t n,
                                  float* out, hipStream_t s) {

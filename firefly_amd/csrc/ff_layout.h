@@ -44,6 +44,7 @@
 #define C_SHD0 2
 #define C_MAT0 3
 #define C_SHD1 7
+#define C_MAT1 8
 #define C_COUNT 16
 
 // Work counters of the persistent traversal kernels: the queue is split into

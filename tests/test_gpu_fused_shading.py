@@ -2,7 +2,9 @@
 their own (per-launch timing asks for those): every film value and ray count is
 the same, at the limit between its two forms, at tile and chunk edges, with
 paths left over from one tile to the next, with one and with all material
-types, and with scenes that differ between requests."""
+types, and with scenes that differ between requests.  Likewise the adjoint's
+replay, whose vertices wait for their shadow rays until the next extension rays
+are traced with them: its deterministic sums are the same either way."""
 import numpy as np
 import pytest
 
@@ -62,3 +64,31 @@ def test_one_launch_equals_stage_launches_of_several_scenes(gpu, sizes, k):
     for f, g in zip(films, want):
         assert np.array_equal(f, g)
     assert counts == want_counts
+
+
+@pytest.mark.parametrize("types", [ALL, [abi.FF_MAT_DIFFUSE], [abi.FF_MAT_MIX, abi.FF_MAT_DIELECTRIC]])
+@pytest.mark.parametrize("width,height,k,spp,depth", [(33, 17, 2, 3, 4), (512, 300, 1, 2, 3), (5, 1, 1, 1, 1)])
+def test_replay_with_rays_traced_together(gpu, width, height, k, spp, depth, types):
+    import torch
+    sd = scenes.textured_spheres_scene(width=width, height=height, spp=spp, max_depth=depth, tex_size=16, env_w=32,
+                                       env_h=16, segments=16, rings=8)
+    mats = sd.materials.copy()
+    mats[:, 0] = np.resize(types, len(mats))
+    sc = abi.Scene(gpu, sd.positions, sd.normals, sd.uvs, sd.material_ids, mats, textures=sd.textures)
+    env, cam = abi.EnvMap(gpu, sd.env), abi.make_camera(sd.inv_vp)
+    paths = torch.zeros((spp, height, width, 4), dtype=torch.float32, device="cuda")
+    film = torch.zeros((height, width, 4), dtype=torch.float32, device="cuda")
+    abi.render_paths(gpu, sc, env, cam, width, height, spp, depth, 5, film, paths, spp_batch=k)
+    d = torch.from_numpy(np.random.default_rng(1).normal(size=(height, width, 4)).astype(np.float32)).cuda()
+    out = []
+    for flags in (0, abi.FF_RENDER_TIMING):
+        g_env = torch.zeros(sd.env.shape, dtype=torch.float32, device="cuda")
+        g_tex = [torch.zeros(t.shape, dtype=torch.float32, device="cuda") for t in sd.textures]
+        abi.adjoint(gpu, sc, env, cam, width, height, spp, depth, 5, paths, d, env_grad=g_env, tex_grads=g_tex,
+                    flags=flags | abi.FF_ADJOINT_DETERMINISTIC, spp_batch=k)
+        torch.cuda.synchronize()
+        st = abi.last_render_stats(gpu)
+        out.append([g_env.cpu().numpy(), *(t.cpu().numpy() for t in g_tex), [getattr(st, c) for c in COUNTS]])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    assert np.any(out[0][0] != 0)
