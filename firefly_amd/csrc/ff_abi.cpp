@@ -366,9 +366,18 @@ ff_status ff_scene_create(ff_context* ctx, const ff_scene_desc* d, ff_scene** ou
     s->ctx = ctx;
     s->n_tris = d->n_tris;
     s->n_mats = d->n_materials;
-    auto cleanup = [&](ff_status st) { ff_scene_destroy(s); return st; };
+    ffk::PackScratch tmp;
+    auto cleanup = [&](ff_status st) {
+        dfree(tmp.mem);
+        ff_scene_destroy(s);
+        return st;
+    };
     int32_t max_prims = d->max_prims_in_node > 0 ? d->max_prims_in_node : 8;
-    hipError_t e;
+    const ffk::SceneArrays arrays{d->normals, d->uvs, d->tangents, d->materials, d->material_ids, d->n_tris,
+                                  d->n_materials};
+    hipError_t e, up = hipSuccess;
+    // the other arrays go up while the GPU builds the tree
+    auto meanwhile = [&] { up = ffk::upload_arrays(arrays, tmp); };
     if (d->builder == FF_BVH_SAH) {
         std::vector<ffh::BvhNode> nodes;
         std::vector<int32_t> ordered;
@@ -377,9 +386,11 @@ ff_status ff_scene_create(ff_context* ctx, const ff_scene_desc* d, ff_scene** ou
         if (e != hipSuccess)
             return cleanup(fail(e == hipErrorOutOfMemory ? FF_ERR_ALLOC : FF_ERR_HIP, "ff_scene_create: upload: %s",
                                 hipGetErrorString(e)));
+        meanwhile();
     } else {
-        e = d->builder == FF_BVH_LBVH ? ffk::build_lbvh(d->positions, d->n_tris, max_prims, s->bvh)
-                                      : ffk::build_ploc(d->positions, d->n_tris, max_prims, s->bvh);
+        e = d->builder == FF_BVH_LBVH
+                ? ffk::build_lbvh(d->positions, d->n_tris, max_prims, s->bvh, nullptr, meanwhile)
+                : ffk::build_ploc(d->positions, d->n_tris, max_prims, s->bvh, nullptr, meanwhile);
         if (e != hipSuccess)
             return cleanup(fail(FF_ERR_HIP, "ff_scene_create: GPU BVH build failed: %s", hipGetErrorString(e)));
     }
@@ -388,8 +399,7 @@ ff_status ff_scene_create(ff_context* ctx, const ff_scene_desc* d, ff_scene** ou
     if (s->bvh.n_nodes / 2 >= (1 << 26))
         return cleanup(fail(FF_ERR_CAPACITY, "ff_scene_create: %d BVH records exceed the 2^26 limit of the traversal "
                                             "kernels", s->bvh.n_nodes / 2));
-    ffk::SceneArrays arrays{d->normals, d->uvs, d->tangents, d->materials, d->material_ids, d->n_tris, d->n_materials};
-    e = ffk::pack_scene(s->bvh, arrays, s->pack);
+    e = up != hipSuccess ? up : ffk::pack_scene(s->bvh, arrays, tmp, s->pack);
     if (e != hipSuccess)
         return cleanup(fail(e == hipErrorOutOfMemory ? FF_ERR_ALLOC : FF_ERR_HIP, "ff_scene_create: packing: %s",
                             hipGetErrorString(e)));

@@ -2,6 +2,7 @@
 // the host BVH builder and the kernel launchers.  Not part of the public ABI.
 #pragma once
 
+#include <functional>
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -97,11 +98,14 @@ struct DevBvh {
     int32_t n_nodes = 0, max_depth = 0, max_leaf = 1;
 };
 // Linear BVH on the GPU (Morton order, Karras hierarchy); positions on the
-// host (gpu_ms, if given: device time of the build kernels).
-hipError_t build_lbvh(const float* positions, int32_t n, int32_t max_prims, DevBvh& out, float* gpu_ms = nullptr);
+// host (gpu_ms, if given: device time of the build kernels; meanwhile: host
+// work to do while the GPU builds).
+hipError_t build_lbvh(const float* positions, int32_t n, int32_t max_prims, DevBvh& out, float* gpu_ms = nullptr,
+                      const std::function<void()>& meanwhile = nullptr);
 // PLOC tree on the GPU (locally-ordered clustering of the Morton-sorted
 // triangles, SAH leaf collapse), same arguments.
-hipError_t build_ploc(const float* positions, int32_t n, int32_t max_prims, DevBvh& out, float* gpu_ms = nullptr);
+hipError_t build_ploc(const float* positions, int32_t n, int32_t max_prims, DevBvh& out, float* gpu_ms = nullptr,
+                      const std::function<void()>& meanwhile = nullptr);
 // A host tree and its positions on the device.
 hipError_t upload_bvh(const std::vector<ffh::BvhNode>& nodes, const std::vector<int32_t>& ordered, int32_t max_depth,
                       const float* positions, DevBvh& out);
@@ -121,5 +125,15 @@ struct ScenePack {
     uint32_t* mat = nullptr;
     int32_t wide_levels = 0;
 };
-hipError_t pack_scene(const DevBvh& bvh, const SceneArrays& a, ScenePack& out);
+// Packing's scratch, which holds the uploaded arrays (`mem`: one allocation;
+// pack_scene frees it).
+struct PackScratch {
+    void *mem = nullptr, *q0 = nullptr, *q1 = nullptr;
+    uint32_t* rank = nullptr;
+    float *nrm = nullptr, *uv = nullptr, *tan = nullptr;
+    int32_t* mid = nullptr;
+    char* scan_tmp = nullptr;
+};
+hipError_t upload_arrays(const SceneArrays& a, PackScratch& tmp);
+hipError_t pack_scene(const DevBvh& bvh, const SceneArrays& a, PackScratch& tmp, ScenePack& out);
 }  // namespace ffk

@@ -317,7 +317,38 @@ hipError_t upload_bvh(const std::vector<ffh::BvhNode>& nodes, const std::vector<
     return e;
 }
 
-hipError_t pack_scene(const DevBvh& bvh, const SceneArrays& a, ScenePack& out) {
+// (n triangles make a tree of at most 2n - 1 nodes)
+static auto interior_flags(const ffh::BvhNode* nodes) {
+    return rocprim::make_transform_iterator(nodes, IsInterior());
+}
+hipError_t upload_arrays(const SceneArrays& a, PackScratch& tmp) {
+    const size_t n = (size_t)a.n;
+    size_t scan_bytes = 0;
+    hipError_t e = rocprim::exclusive_scan(nullptr, scan_bytes, interior_flags(nullptr), tmp.rank, 0u, 2 * n,
+                                           rocprim::plus<uint32_t>(), nullptr);
+    if (e != hipSuccess) return e;
+    auto carve = [&](Carver c) {
+        tmp.rank = c.take<uint32_t>(2 * n);
+        tmp.nrm = c.take<float>(9 * n);
+        tmp.uv = c.take<float>(a.uv ? 6 * n : 0);
+        tmp.tan = c.take<float>(a.tan ? 18 * n : 0);
+        tmp.mid = c.take<int32_t>(n);
+        tmp.q0 = c.take<WItem>(n);
+        tmp.q1 = c.take<WItem>(n);
+        tmp.scan_tmp = c.take<char>(scan_bytes);
+        return c.off;
+    };
+    e = hipMalloc(&tmp.mem, carve(Carver{}));
+    if (e != hipSuccess) return e;
+    carve(Carver{(char*)tmp.mem});
+    e = hipMemcpy(tmp.nrm, a.nrm, 36 * n, hipMemcpyHostToDevice);
+    if (e == hipSuccess && a.uv) e = hipMemcpy(tmp.uv, a.uv, 24 * n, hipMemcpyHostToDevice);
+    if (e == hipSuccess && a.tan) e = hipMemcpy(tmp.tan, a.tan, 72 * n, hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = hipMemcpy(tmp.mid, a.mid, 4 * n, hipMemcpyHostToDevice);
+    return e;
+}
+
+hipError_t pack_scene(const DevBvh& bvh, const SceneArrays& a, PackScratch& tmp, ScenePack& out) {
     const size_t n = (size_t)a.n, n_int = ((size_t)bvh.n_nodes - 1) / 2;  // a full binary tree
     // a group with fewer than four children holds single triangles only, so
     // n triangles make at most 2n/3 + 1 groups
@@ -325,6 +356,7 @@ hipError_t pack_scene(const DevBvh& bvh, const SceneArrays& a, ScenePack& out) {
     int32_t split = 0;
     while ((1 << split) < bvh.max_leaf) split++;
     const int32_t max_levels = bvh.max_depth + split + 2;
+    uint32_t* cnt = nullptr;  // [levels + 1] wide nodes of each level, then the groups handed out
     auto carve = [&](Carver c) {
         out.nodes = c.take<float4>(4 * n_int);
         out.nodes4 = c.take<float4>(8 * n_int);
@@ -337,69 +369,55 @@ hipError_t pack_scene(const DevBvh& bvh, const SceneArrays& a, ScenePack& out) {
         out.mat = c.take<uint32_t>(n);
         float* tan = c.take<float>(a.tan ? 18 * n : 0);
         out.tan = a.tan ? tan : nullptr;
-        return c.off;
-    };
-    uint32_t* rank = nullptr;
-    float *nrm = nullptr, *uv = nullptr, *tan = nullptr;
-    int32_t* mid = nullptr;
-    WItem *q0 = nullptr, *q1 = nullptr;
-    uint32_t* cnt = nullptr;  // [levels + 1] wide nodes of each level, then the groups handed out
-    char* scan_tmp = nullptr;
-    size_t scan_bytes = 0;
-    auto interior = rocprim::make_transform_iterator((const ffh::BvhNode*)bvh.nodes, IsInterior());
-    hipError_t e = rocprim::exclusive_scan(nullptr, scan_bytes, interior, rank, 0u, (size_t)bvh.n_nodes,
-                                           rocprim::plus<uint32_t>(), nullptr);
-    if (e != hipSuccess) return e;
-    auto carve_tmp = [&](Carver c) {
-        rank = c.take<uint32_t>((size_t)bvh.n_nodes);
-        nrm = c.take<float>(9 * n);
-        uv = c.take<float>(a.uv ? 6 * n : 0);
-        tan = c.take<float>(a.tan ? 18 * n : 0);
-        mid = c.take<int32_t>(n);
-        q0 = c.take<WItem>(n);
-        q1 = c.take<WItem>(n);
         cnt = c.take<uint32_t>((size_t)max_levels + 2);
-        scan_tmp = c.take<char>(scan_bytes);
         return c.off;
     };
-    void* tmp = nullptr;
+    hipError_t e = hipSuccess;
     auto ok = [&](hipError_t x) { if (e == hipSuccess) e = x; return e == hipSuccess; };
     std::vector<uint32_t> h((size_t)max_levels + 2, 0u);
     h[0] = 1u;                       // level 0: the root
     h[(size_t)max_levels + 1] = 1u;  // groups: the root's own
-    if (ok(hipMalloc(&out.mem, carve(Carver{}))) && ok(hipMalloc(&tmp, carve_tmp(Carver{})))) {
+    size_t scan_bytes = 0;
+    auto interior = interior_flags(bvh.nodes);
+    if (ok(rocprim::exclusive_scan(nullptr, scan_bytes, interior, tmp.rank, 0u, (size_t)bvh.n_nodes,
+                                   rocprim::plus<uint32_t>(), nullptr)) &&
+        ok(hipMalloc(&out.mem, carve(Carver{})))) {
         carve(Carver{(char*)out.mem});
-        carve_tmp(Carver{(char*)tmp});
-        ok(hipMemcpy(nrm, a.nrm, 36 * n, hipMemcpyHostToDevice));
-        if (a.uv) ok(hipMemcpy(uv, a.uv, 24 * n, hipMemcpyHostToDevice));
-        if (a.tan) ok(hipMemcpy(tan, a.tan, 72 * n, hipMemcpyHostToDevice));
-        ok(hipMemcpy(mid, a.mid, 4 * n, hipMemcpyHostToDevice));
         ok(hipMemcpy(out.mats, a.mats, sizeof(float) * FF_MAT_FLOATS_DEV * a.n_mats, hipMemcpyHostToDevice));
         ok(hipMemcpy(cnt, h.data(), h.size() * 4, hipMemcpyHostToDevice));
         ok(hipMemsetAsync(out.leaf_count, 0, 4 * n, nullptr));
-        ok(rocprim::exclusive_scan(scan_tmp, scan_bytes, interior, rank, 0u, (size_t)bvh.n_nodes,
+        ok(rocprim::exclusive_scan(tmp.scan_tmp, scan_bytes, interior, tmp.rank, 0u, (size_t)bvh.n_nodes,
                                    rocprim::plus<uint32_t>(), nullptr));
     }
     if (e == hipSuccess) {
-        hipLaunchKernelGGL(k_pack_slots, dim3(pack_grid(n)), dim3(PK_BLOCK), 0, nullptr, bvh.ordered, bvh.pos, nrm,
-                           a.uv ? uv : nullptr, tan, mid, out.mats, a.n, out.tris, (float*)out.attr, out.mat, out.tan);
+        hipLaunchKernelGGL(k_pack_slots, dim3(pack_grid(n)), dim3(PK_BLOCK), 0, nullptr, bvh.ordered, bvh.pos, tmp.nrm,
+                           a.uv ? tmp.uv : nullptr, a.tan ? tmp.tan : nullptr, tmp.mid, out.mats, a.n, out.tris,
+                           (float*)out.attr, out.mat, out.tan);
         hipLaunchKernelGGL(k_pack_nodes, dim3(pack_grid((size_t)bvh.n_nodes)), dim3(PK_BLOCK), 0, nullptr, bvh.nodes,
-                           rank, bvh.n_nodes, out.nodes, out.nodes4, out.leaf_count, out.root);
+                           tmp.rank, bvh.n_nodes, out.nodes, out.nodes4, out.leaf_count, out.root);
+        WItem *q0 = (WItem*)tmp.q0, *q1 = (WItem*)tmp.q1;
         hipLaunchKernelGGL(k_wide_root, dim3(1), dim3(1), 0, nullptr, bvh.nodes, q0);
         ok(hipGetLastError());
+        // Four children to a node: a balanced tree ends after half the binary
+        // tree's levels, so the rest is launched only if the tree goes on there
+        // (of 82 k triangles 14 levels instead of 26 launched, 4.5 us each).
         size_t at_most = 1;
-        for (int32_t l = 0; l < max_levels && e == hipSuccess; l++) {
-            hipLaunchKernelGGL(k_wide_level, dim3(pack_grid(at_most)), dim3(PK_BLOCK), 0, nullptr, bvh.nodes, out.tris,
-                               q0, cnt + l, q1, cnt + l + 1, cnt + max_levels + 1, out.wide);
-            ok(hipGetLastError());
-            std::swap(q0, q1);
-            at_most = std::min<size_t>(at_most * 4, n);
+        int32_t l = 0;
+        for (int32_t stop : {max_levels / 2 + 1, max_levels}) {
+            for (stop = std::min(stop, max_levels); l < stop && e == hipSuccess; l++) {
+                hipLaunchKernelGGL(k_wide_level, dim3(pack_grid(at_most)), dim3(PK_BLOCK), 0, nullptr, bvh.nodes,
+                                   out.tris, q0, cnt + l, q1, cnt + l + 1, cnt + max_levels + 1, out.wide);
+                ok(hipGetLastError());
+                std::swap(q0, q1);
+                at_most = std::min<size_t>(at_most * 4, n);
+            }
+            if (!ok(hipMemcpy(h.data(), cnt, h.size() * 4, hipMemcpyDeviceToHost)) || !h[(size_t)l]) break;
         }
-        ok(hipMemcpy(h.data(), cnt, h.size() * 4, hipMemcpyDeviceToHost));
         out.wide_levels = 0;
         while (e == hipSuccess && out.wide_levels < max_levels && h[(size_t)out.wide_levels]) out.wide_levels++;
     }
-    if (tmp) (void)hipFree(tmp);
+    if (tmp.mem) (void)hipFree(tmp.mem);
+    tmp.mem = nullptr;
     if (e != hipSuccess && out.mem) {
         (void)hipFree(out.mem);
         out.mem = nullptr;
