@@ -2039,17 +2039,10 @@ __global__ void k_gen_rays(ff_dev_camera cam, int32_t W, int32_t H, uint32_t see
 // FP64 CDF build replacing the serial <<<1,1>>> passes of
 // g_compute_pdf_denom / g_compute_marginal_dist / g_compute_conditional_dist /
 // g_write_pdf_texture (CRT/kernel.cu:65-149).  Same per-texel terms; sums are
-// fixed-order tree reductions and blocked scans (deterministic, FP64).
-__global__ void k_env_lum(const float* rgb, int32_t w, int32_t h, float* lum) {
-    uint32_t n = (uint32_t)w * (uint32_t)h;
-    for (uint32_t k = gtid(); k < n; k += gstride()) {
-        int i = (int)(k % (uint32_t)w), j = (int)(k / (uint32_t)w);
-        float s[3];
-        bilinear(rgb, w, h, 3, (float)i / (float)w, (float)j / (float)h, s);
-        lum[k] = lum_of(s);
-    }
-}
-
+// fixed-order tree reductions and blocked scans (deterministic, FP64).  Three
+// launches: rows, conditionals (with denom, guides, pdf and render-time
+// texels), marginal; 48 us for 2048 x 1024 texels, where about 100 MB have to
+// move (22 us); with every part a launch of its own (seven) it took 105 us.
 __device__ __forceinline__ double block_sum(double v, double* red) {
     red[threadIdx.x] = v;
     __syncthreads();
@@ -2062,90 +2055,175 @@ __device__ __forceinline__ double block_sum(double v, double* red) {
     return r;
 }
 
-// one workgroup per row: row_sum[j] = sum_i lum(i,j) * sin_theta_j
-__global__ __launch_bounds__(FF_BLOCK) void k_env_rows(const float* lum, int32_t w, int32_t h, double* row_sum) {
+// One workgroup per row: the row's luminances, and
+// row_sum[j] = sum_i lum(i,j) * sin_theta_j
+__global__ __launch_bounds__(FF_BLOCK) void k_env_rows(const float* rgb, int32_t w, int32_t h, float* lum,
+                                                       double* row_sum) {
     __shared__ double red[FF_BLOCK];
     int j = blockIdx.x;
     float v = (float)j / (float)h;
     double st = (double)f_sin(F_PI * v);
     double acc = 0.0;
-    for (int i = threadIdx.x; i < w; i += FF_BLOCK) acc += (double)lum[(size_t)j * w + i] * st;
+    for (int i = threadIdx.x; i < w; i += FF_BLOCK) {
+        float s[3];
+        bilinear(rgb, w, h, 3, (float)i / (float)w, v, s);
+        const float l = lum_of(s);
+        lum[(size_t)j * w + i] = l;
+        acc += (double)l * st;
+    }
     double s = block_sum(acc, red);
     if (threadIdx.x == 0) row_sum[j] = s;
 }
 
-// single workgroup: denom = sum of the row sums (h values)
-__global__ __launch_bounds__(FF_BLOCK) void k_env_denom(const double* row_sum, int32_t h, double* denom_out) {
-    __shared__ double red[FF_BLOCK];
-    double acc = 0.0;
-    for (int j = threadIdx.x; j < h; j += FF_BLOCK) acc += row_sum[j];
-    double denom = block_sum(acc, red);
-    if (threadIdx.x == 0) *denom_out = denom;
+// Guide table of an environment's inverse-CDF search, formed with the list
+// itself.  Entry g is the upper bound of g / ENV_GUIDE (first element greater,
+// compared in double as the sampler compares), so the upper bound of any val
+// in [g, g+1) / ENV_GUIDE lies in [entry g, entry g+1].  In a list that never
+// decreases, element x + 1 is the upper bound from the first entry that is not
+// below element x on: every element marks that entry, and the running maximum
+// of the marks is the table.  (A search of the list for each of 4097 entries of
+// 1024 rows of 2048 took 39 us; letting each element's thread write all its
+// entries takes as long as the brightest texel has entries: 93 us for a whole
+// build's rows.)  A list with a NaN or a decreasing step gets flagged entries
+// (searched whole).  Every entry also carries list[0] != 0 and list[1] != 0
+// (ENV_GUIDE_NZ0 / ENV_GUIDE_NZ1).
+constexpr uint32_t GUIDE_PER = ENV_GUIDE / FF_BLOCK + 1;  // entries of a thread (odd: no bank conflicts)
+static_assert(GUIDE_PER % 2 == 1 && GUIDE_PER * FF_BLOCK > ENV_GUIDE, "one run of entries for each thread");
+struct CdfScan {  // of one workgroup
+    double red[FF_BLOCK];
+    uint32_t mark[GUIDE_PER * FF_BLOCK], wave[FF_BLOCK / 64];
+    uint32_t nz;
+};
+// list[i] = the sum of term(0..i): thread t owns elements [t*c, (t+1)*c), the
+// threads' sums are added up in order by one thread, eight loads at a time.
+template <class Term>
+__device__ __forceinline__ void cdf_scan(CdfScan& S, int size, Term term, double* list, uint32_t* guide) {
+    const int c = (size + FF_BLOCK - 1) / FF_BLOCK;
+    const int lo = threadIdx.x * c, hi = lo + c < size ? lo + c : size;
+    double local = 0.0;
+    int x = lo;
+    for (; x + 4 <= hi; x += 4) {  // (four at a time: one wide load)
+        double q[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k] = term(x + k);
+#pragma unroll
+        for (int k = 0; k < 4; k++) local += q[k];
+    }
+    for (; x < hi; x++) local += term(x);
+    S.red[threadIdx.x] = local;
+    for (uint32_t g = threadIdx.x; g < GUIDE_PER * FF_BLOCK; g += FF_BLOCK) S.mark[g] = 0u;
+    if (threadIdx.x == 0) S.nz = 0u;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        double run = 0.0;
+        for (int t = 0; t < FF_BLOCK; t += 8) {
+            double q[8];
+#pragma unroll
+            for (int k = 0; k < 8; k++) q[k] = S.red[t + k];
+#pragma unroll
+            for (int k = 0; k < 8; k++) {
+                S.red[t + k] = run;
+                run += q[k];
+            }
+        }
+    }
+    __syncthreads();
+    double run = S.red[threadIdx.x], head = 0.0;
+    int bad = 0;
+    uint32_t nz = 0u;
+    auto element = [&](int i, double q) {  // adds q; the list's element i
+        const double prev = run;
+        run += q;
+        if (i == lo) head = run;
+        if (run != run || (i > lo && run < prev)) bad = 1;
+        if (i < 2 && run != 0.0) nz |= i == 0 ? ENV_GUIDE_NZ0 : ENV_GUIDE_NZ1;
+        const double e = ceil(run * (double)ENV_GUIDE);  // (the first entry not below the element; exact)
+        if (e <= (double)ENV_GUIDE) atomicMax(&S.mark[e > 0.0 ? (int)e : 0], (uint32_t)i + 1u);
+        return run;
+    };
+    x = lo;
+    for (; x + 4 <= hi; x += 4) {
+        double q[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k] = term(x + k);
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k] = element(x + k, q[k]);
+#pragma unroll
+        for (int k = 0; k < 4; k++) list[x + k] = q[k];
+    }
+    for (; x < hi; x++) list[x] = element(x, term(x));
+    if (nz) atomicOr(&S.nz, nz);
+    __syncthreads();
+    S.red[threadIdx.x] = run;  // the thread's last element
+    __syncthreads();
+    if (lo > 0 && lo < hi && head < S.red[threadIdx.x - 1]) bad = 1;
+    // running maximum: of the thread's entries, of the wave's threads, of the waves
+    uint32_t* const m = S.mark + threadIdx.x * GUIDE_PER;
+    uint32_t top = 0u;
+    for (uint32_t k = 0; k < GUIDE_PER; k++) {
+        top = m[k] > top ? m[k] : top;
+        m[k] = top;
+    }
+    const uint32_t lane = __lane_id(), w = threadIdx.x >> 6;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+        const uint32_t o = __shfl_up(top, off);
+        if (lane >= (uint32_t)off && o > top) top = o;
+    }
+    if (lane == 63u) S.wave[w] = top;
+    bad = __syncthreads_or(bad);
+    uint32_t before = __shfl_up(top, 1);
+    if (lane == 0u) before = 0u;
+    for (uint32_t k = 0; k < w; k++) before = S.wave[k] > before ? S.wave[k] : before;
+    for (uint32_t k = 0; k < GUIDE_PER; k++) m[k] = m[k] > before ? m[k] : before;
+    __syncthreads();
+    for (uint32_t g = threadIdx.x; g <= ENV_GUIDE; g += FF_BLOCK)
+        guide[g] = (bad ? ENV_GUIDE_FULL : S.mark[g]) | S.nz;
 }
 
-// one workgroup per row: marginal_p[y] = sum_x lum * (sin_theta_y / denom)
-// (g_compute_marginal_dist's term), then the row's conditional CDF (blocked
-// scan of lum * sin_theta_y / (denom * marginal_p[y])) and its pdf texels
-__global__ __launch_bounds__(FF_BLOCK) void k_env_conditional(const float* lum, int32_t w, int32_t h,
-                                                              const double* denom_p, double* marg_p,
-                                                              double* conds, float* pdf) {
-    __shared__ double red[FF_BLOCK];
+// One workgroup per row: denom = the sum of the row sums, marginal_p[y] =
+// sum_x lum * (sin_theta_y / denom) (g_compute_marginal_dist's term), then the
+// row's conditional CDF (blocked scan of lum * sin_theta_y / (denom *
+// marginal_p[y])) with its guide table, its pdf texels and its render-time
+// texels (r, g, b, pdf).  Every workgroup forms denom itself (h values from the
+// L2), which spares a launch of one workgroup.
+__global__ __launch_bounds__(FF_BLOCK) void k_env_conditional(const float* rgb, const float* lum, int32_t w, int32_t h,
+                                                              const double* row_sum, double* denom_out,
+                                                              double* marg_p, double* conds, float* pdf,
+                                                              uint32_t* guide_c, float4* rgbp) {
+    __shared__ CdfScan S;
     int y = blockIdx.x;
-    double denom = *denom_p;
+    double acc = 0.0;
+    for (int j = threadIdx.x; j < h; j += FF_BLOCK) acc += row_sum[j];
+    const double denom = block_sum(acc, S.red);
+    if (y == 0 && threadIdx.x == 0) *denom_out = denom;
     float v = (float)y / (float)h;
     double st = (double)f_sin(F_PI * v);
     const float* row = lum + (size_t)y * w;
     double stn = st / denom;
     double mp = 0.0;
-    for (int x = threadIdx.x; x < w; x += FF_BLOCK) mp += (double)row[x] * stn;
-    mp = block_sum(mp, red);
-    if (threadIdx.x == 0) marg_p[y] = mp;
-    double val = st / (denom * mp);
-    double* crow = conds + (size_t)y * w;
-    int c = (w + FF_BLOCK - 1) / FF_BLOCK;
-    int lo = threadIdx.x * c, hi = lo + c < w ? lo + c : w;
-    double local = 0.0;
-    for (int x = lo; x < hi; x++) local += (double)row[x] * val;
-    red[threadIdx.x] = local;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double run = 0.0;
-        for (int t = 0; t < FF_BLOCK; t++) { double q = red[t]; red[t] = run; run += q; }
-    }
-    __syncthreads();
-    double run = red[threadIdx.x];
-    for (int x = lo; x < hi; x++) { run += (double)row[x] * val; crow[x] = run; }
     float scale = (float)(w * h) / (2.f * F_PI * F_PI);
     for (int x = threadIdx.x; x < w; x += FF_BLOCK) {
-        float p = (float)(((double)row[x] * st) / denom);
+        const float l = row[x];
+        mp += (double)l * stn;
+        float p = (float)(((double)l * st) / denom);
         p *= scale;
-        pdf[(size_t)y * w + x] = p;
+        const size_t k = (size_t)y * w + x;
+        pdf[k] = p;
+        rgbp[k] = make_float4(rgb[3 * k], rgb[3 * k + 1], rgb[3 * k + 2], p);
     }
+    mp = block_sum(mp, S.red);
+    if (threadIdx.x == 0) marg_p[y] = mp;
+    const double val = st / (denom * mp);
+    cdf_scan(S, w, [&](int x) { return (double)row[x] * val; }, conds + (size_t)y * w,
+             guide_c + (size_t)y * (ENV_GUIDE + 1));
 }
 
-// the render-time texel array: (r, g, b, pdf) per texel
-__global__ void k_env_pack(const float* rgb, const float* pdf, uint32_t n, float4* rgbp) {
-    for (uint32_t k = gtid(); k < n; k += gstride())
-        rgbp[k] = make_float4(rgb[3 * (size_t)k], rgb[3 * (size_t)k + 1], rgb[3 * (size_t)k + 2], pdf[k]);
-}
-
-// single workgroup: marginal_y = inclusive scan of marginal_p (thread t
-// owns rows [t*c, (t+1)*c), block offsets scanned in order)
-__global__ __launch_bounds__(FF_BLOCK) void k_env_marginal_scan(const double* marg_p, int32_t h, double* marg_y) {
-    __shared__ double red[FF_BLOCK];
-    int c = (h + FF_BLOCK - 1) / FF_BLOCK;
-    int lo = threadIdx.x * c, hi = lo + c < h ? lo + c : h;
-    double local = 0.0;
-    for (int j = lo; j < hi; j++) local += marg_p[j];
-    red[threadIdx.x] = local;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        double run = 0.0;
-        for (int t = 0; t < FF_BLOCK; t++) { double x = red[t]; red[t] = run; run += x; }
-    }
-    __syncthreads();
-    double run = red[threadIdx.x];
-    for (int j = lo; j < hi; j++) { run += marg_p[j]; marg_y[j] = run; }
+// single workgroup: marginal_y = inclusive scan of marginal_p, and its guide table
+__global__ __launch_bounds__(FF_BLOCK) void k_env_marginal(const double* marg_p, int32_t h, double* marg_y,
+                                                           uint32_t* guide_m) {
+    __shared__ CdfScan S;
+    cdf_scan(S, h, [&](int j) { return marg_p[j]; }, marg_y, guide_m);
 }
 
 // ============================================================ film resolve
@@ -2263,38 +2341,6 @@ hipError_t trav_dispatch(int which, int variant, const TraceArgs& T, hipStream_t
         FF_TRAV_VARIANT_LIST(FF_TRAV_CASE)
 #undef FF_TRAV_CASE
         default: return hipErrorInvalidValue;
-    }
-}
-
-// Guide tables of the environment's inverse-CDF searches (block r < h: row
-// r of the conditional CDF, block h: the marginal).  Entry g is the upper
-// bound of g / ENV_GUIDE (first element greater, compared in double as the
-// sampler compares), so the upper bound of any val in [g, g+1) / ENV_GUIDE
-// lies in [entry g, entry g+1].  A list with a NaN or a decreasing step gets
-// flagged entries (searched whole).  Every entry also carries list[0] != 0
-// and list[1] != 0 (ENV_GUIDE_NZ0 / ENV_GUIDE_NZ1).
-__global__ void k_env_guide(const double* marg_y, const double* conds, int32_t w, int32_t h, uint32_t* guide_m,
-                            uint32_t* guide_c) {
-    const bool marg = (int)blockIdx.x == h;
-    const double* list = marg ? marg_y : conds + (size_t)blockIdx.x * w;
-    const int size = marg ? h : w;
-    uint32_t* out = marg ? guide_m : guide_c + (size_t)blockIdx.x * (ENV_GUIDE + 1);
-    int mine = 0;
-    for (int i = threadIdx.x; i < size; i += blockDim.x) {
-        double v = list[i];
-        if (v != v || (i > 0 && v < list[i - 1])) mine = 1;
-    }
-    const int bad = __syncthreads_or(mine);
-    const uint32_t nz = (list[0] != 0.0 ? ENV_GUIDE_NZ0 : 0u) | (list[1] != 0.0 ? ENV_GUIDE_NZ1 : 0u);
-    for (int g = threadIdx.x; g <= ENV_GUIDE; g += blockDim.x) {
-        float val = (float)g / (float)ENV_GUIDE;
-        int left = 0, right = size;
-        while (left < right) {
-            int middle = (right - left) / 2 + left;
-            if ((double)val >= list[middle]) left = middle + 1;
-            else right = middle;
-        }
-        out[g] = (bad ? ENV_GUIDE_FULL : (uint32_t)left) | nz;
     }
 }
 
@@ -2549,15 +2595,10 @@ hipError_t launch_gen_rays(const ff_dev_camera& cam, int W, int H, uint32_t seed
 hipError_t launch_env_build(const float* rgb, int w, int h, float* lum, double* row_sum, double* denom,
                             double* marg_p, double* marg_y, double* conds, float* pdf, uint32_t* guide_m,
                             uint32_t* guide_c, float4* rgbp, hipStream_t s) {
-    hipLaunchKernelGGL(k_env_lum, dim3(grid_for((uint64_t)w * h, FF_GRID_CAP)), dim3(FF_BLOCK), 0, s, rgb, w, h,
-                       lum);
-    hipLaunchKernelGGL(k_env_rows, dim3(h), dim3(FF_BLOCK), 0, s, lum, w, h, row_sum);
-    hipLaunchKernelGGL(k_env_denom, dim3(1), dim3(FF_BLOCK), 0, s, row_sum, h, denom);
-    hipLaunchKernelGGL(k_env_conditional, dim3(h), dim3(FF_BLOCK), 0, s, lum, w, h, denom, marg_p, conds, pdf);
-    hipLaunchKernelGGL(k_env_marginal_scan, dim3(1), dim3(FF_BLOCK), 0, s, marg_p, h, marg_y);
-    hipLaunchKernelGGL(k_env_guide, dim3(h + 1), dim3(FF_BLOCK), 0, s, marg_y, conds, w, h, guide_m, guide_c);
-    hipLaunchKernelGGL(k_env_pack, dim3(grid_for((uint64_t)w * h, FF_GRID_CAP)), dim3(FF_BLOCK), 0, s, rgb, pdf,
-                       (uint32_t)((size_t)w * h), rgbp);
+    hipLaunchKernelGGL(k_env_rows, dim3(h), dim3(FF_BLOCK), 0, s, rgb, w, h, lum, row_sum);
+    hipLaunchKernelGGL(k_env_conditional, dim3(h), dim3(FF_BLOCK), 0, s, rgb, lum, w, h, row_sum, denom, marg_p, conds,
+                       pdf, guide_c, rgbp);
+    hipLaunchKernelGGL(k_env_marginal, dim3(1), dim3(FF_BLOCK), 0, s, marg_p, h, marg_y, guide_m);
     return hipGetLastError();
 }
 hipError_t launch_film_resolve(const float4* film, uint32_t n, float exposure, float* avg, uint8_t* rgba,
