@@ -726,6 +726,19 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
     src.count(__lane_id() == 0 ? c_rays : 0u, __lane_id() == 0 ? c_gated : 0u);
 }
 
+// Rays that a wave of the four-lane walk holds at once: where rays are few,
+// fewer to a wave, so that a wave waits for fewer others.
+__host__ __device__ __forceinline__ uint32_t quad_rays(uint32_t n) {
+    return n >= QUAD_SPREAD * 16u ? 16u : n / QUAD_SPREAD + 1u;
+}
+// Waves that hold all n rays at once take theirs by their own number: the work
+// counters are not touched, so a query needs no launch that clears them first
+// (two queries of 77 rays: 51 -> 38 us; a 160x120 4-bounce
+// render 0.384 -> 0.342 ms, a 320x180 one 0.451 -> 0.385 ms, where every one of
+// up to 6144 waves asked a counter first and then looked for more).
+__host__ __device__ __forceinline__ bool quad_fixed(uint32_t n, uint32_t waves) {
+    return (uint64_t)waves * quad_rays(n) >= n;
+}
 // The same walk with four lanes to a ray, for launches of few rays: there a
 // launch lasts as long as its slowest ray's chain of dependent visits, and a
 // visit is a third of the instructions when every lane tests one child.
@@ -734,11 +747,12 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
 // overflow area: the launcher takes this walk only where LDS * 4 entries hold
 // the deepest stack).
 template <int BS, bool ANY, class Src>
-__device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t block, uint32_t* fetch,
+__device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t block, uint32_t blocks, uint32_t* fetch,
                                           unsigned long long* cnt, int* smem) {
     constexpr uint32_t IDLE = 0xffffffffu;
+    const uint32_t wave = block * (BS / 64) + (threadIdx.x >> 6);
     SegFetch F;
-    F.init(fetch, n, block * (BS / 64) + (threadIdx.x >> 6));
+    F.init(fetch, n, wave);
     const uint32_t lane = __lane_id(), k = lane & 3u, lead = lane & ~3u;
     const uint64_t below = ((1ull << lead) - 1ull) & 0x1111111111111111ull;
     QuadStack<BS> st;
@@ -756,8 +770,8 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
     float t_hit = K_HUGE;           // of the quad
     Hit best = no_hit();            // of the lane
     float redo_t = -1.f;            // a distance that the reference's order decides
-    // few rays: fewer to a wave, so that a wave waits for fewer others
-    const uint32_t cap = n >= QUAD_SPREAD * 16u ? 16u : n / QUAD_SPREAD + 1u;
+    const uint32_t cap = quad_rays(n);
+    const bool fixed = quad_fixed(n, blocks * (BS / 64));
     const bool mine = (lane >> 2) < cap;
     auto start = [&](f3 o, f3 d) {
         wide_begin(o, d, R);
@@ -784,9 +798,14 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
         const uint64_t idle = __ballot(mine && id == IDLE && k == 0u);
         if (idle != 0) {
             if (more) {
-                uint32_t got;
-                bool done;
-                uint32_t first = F.take_chunked((uint32_t)__popcll(idle), got, done);
+                uint32_t got, first;
+                bool done = true;
+                if (fixed) {
+                    first = wave * cap;
+                    got = first < n ? (n - first < cap ? n - first : cap) : 0u;
+                } else {
+                    first = F.take_chunked((uint32_t)__popcll(idle), got, done);
+                }
                 if (done) more = false;
                 c_rays += got;
                 const uint32_t rank = (uint32_t)__popcll(idle & below);
@@ -895,12 +914,12 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
     src.count(lane == 0 ? c_rays : 0u, lane == 0 ? c_gated : 0u);
 }
 
-// block: the workgroup's number among those that draw from the same queue (its
-// waves start on the queue's segments in turn)
+// block: the workgroup's number among the `blocks` that draw from the same queue
+// (its waves start on the queue's segments in turn)
 template <bool ANY, class Src>
-__device__ __forceinline__ void traverse(const Src& src, uint32_t n, uint32_t block, bool quad, uint32_t* fetch,
-                                         int32_t* ovf, unsigned long long* cnt, int* smem) {
-    if (quad && n <= QUAD_MAX) trav_quad<TW_BLOCK, ANY>(src, n, block, fetch, cnt, smem);
+__device__ __forceinline__ void traverse(const Src& src, uint32_t n, uint32_t block, uint32_t blocks, bool quad,
+                                         uint32_t* fetch, int32_t* ovf, unsigned long long* cnt, int* smem) {
+    if (quad && n <= QUAD_MAX) trav_quad<TW_BLOCK, ANY>(src, n, block, blocks, fetch, cnt, smem);
     else trav_wide<TW_BLOCK, ANY>(src, n, block, fetch, ovf, cnt, smem);
 }
 // LDS words of a traversal workgroup: the stacks, for closest hits the hit words too
@@ -908,7 +927,7 @@ constexpr int TW_LDS_ANY = FF_LDS_STACK * TW_BLOCK, TW_LDS_CLOSEST = (FF_LDS_STA
 
 // SMALL: a call with at most QUAD_MAX paths in flight
 template <bool UNI, bool SMALL>
-__device__ __forceinline__ void extend_rays(const ff_paths& P, int q, uint32_t block, int* smem) {
+__device__ __forceinline__ void extend_rays(const ff_paths& P, int q, uint32_t block, uint32_t blocks, int* smem) {
     // the counters that the coming stages of the iteration add to (nothing
     // reads them during the traversal; those it reads are cleared by the logic)
     if (block == 0 && threadIdx.x < 6)
@@ -918,27 +937,27 @@ __device__ __forceinline__ void extend_rays(const ff_paths& P, int q, uint32_t b
     const uint32_t n = P.counters[ext_counter(q)];
     uint32_t* const fetch = P.fetch + F_EXT * FETCH_SEGS * FETCH_STRIDE;
     unsigned long long* const cnt = stats_rep(P) + S_EXT_NODES;
-    if (SMALL) trav_quad<TW_BLOCK, false>(src, n, block, fetch, cnt, smem);
-    else traverse<false>(src, n, block, P.quad != 0, fetch, P.ovf, cnt, smem);
+    if (SMALL) trav_quad<TW_BLOCK, false>(src, n, block, blocks, fetch, cnt, smem);
+    else traverse<false>(src, n, block, blocks, P.quad != 0, fetch, P.ovf, cnt, smem);
 }
 template <bool UNI, bool SMALL>
-__device__ __forceinline__ void shadow_rays(const ff_paths& P, int q, uint32_t block, int* smem) {
+__device__ __forceinline__ void shadow_rays(const ff_paths& P, int q, uint32_t block, uint32_t blocks, int* smem) {
     const ShadowSrc<UNI> src{P};
     const uint32_t n = P.counters[shadow_counter(q)];
     uint32_t* const fetch = P.fetch + F_SHD * FETCH_SEGS * FETCH_STRIDE;
     unsigned long long* const cnt = stats_rep(P) + S_SHD_NODES;
-    if (SMALL) trav_quad<TW_BLOCK, true>(src, n, block, fetch, cnt, smem);
-    else traverse<true>(src, n, block, P.quad != 0, fetch, P.ovf_shd, cnt, smem);
+    if (SMALL) trav_quad<TW_BLOCK, true>(src, n, block, blocks, fetch, cnt, smem);
+    else traverse<true>(src, n, block, blocks, P.quad != 0, fetch, P.ovf_shd, cnt, smem);
 }
 template <bool UNI>
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_CLOSEST];
-    extend_rays<UNI, false>(P, q, blockIdx.x, smem);
+    extend_rays<UNI, false>(P, q, blockIdx.x, gridDim.x, smem);
 }
 template <bool UNI>
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_shadow(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_ANY];
-    shadow_rays<UNI, false>(P, q, blockIdx.x, smem);
+    shadow_rays<UNI, false>(P, q, blockIdx.x, gridDim.x, smem);
 }
 // An iteration's extension rays and its vertices' shadow rays (both come from
 // the previous shading pass) in one launch: workgroups alternate between the
@@ -947,10 +966,13 @@ __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_shadow(ff_paths P, int q) 
 template <bool UNI>
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend_shadow(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_CLOSEST];
-    const uint32_t block = (blockIdx.x >> 4) * 8u + (blockIdx.x & 7u);
+    const uint32_t blocks = gridDim.x / 2u;
     for (uint32_t ph = 0; ph < 2; ph++) {
-        if ((((blockIdx.x >> 3) + ph) & 1u) == 0u) extend_rays<UNI, false>(P, q, block, smem);
-        else shadow_rays<UNI, false>(P, q, block, smem);
+        // (a queue's guests are numbered after its own workgroups, whose waves
+        // may hold all its rays by their number)
+        const uint32_t block = (blockIdx.x >> 4) * 8u + (blockIdx.x & 7u) + ph * blocks;
+        if ((((blockIdx.x >> 3) + ph) & 1u) == 0u) extend_rays<UNI, false>(P, q, block, blocks, smem);
+        else shadow_rays<UNI, false>(P, q, block, blocks, smem);
     }
 }
 // The same for a call with at most QUAD_MAX paths in flight: each queue has
@@ -959,8 +981,8 @@ template <bool UNI>
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend_shadow_small(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_ANY];
     const uint32_t block = (blockIdx.x >> 4) * 8u + (blockIdx.x & 7u);
-    if (blockIdx.x & 8u) shadow_rays<UNI, true>(P, q, block, smem);
-    else extend_rays<UNI, true>(P, q, block, smem);
+    if (blockIdx.x & 8u) shadow_rays<UNI, true>(P, q, block, gridDim.x / 2u, smem);
+    else extend_rays<UNI, true>(P, q, block, gridDim.x / 2u, smem);
 }
 
 // clears the work counters of the standalone traces (a kernel: graph-safe)
@@ -2017,12 +2039,12 @@ __global__ __launch_bounds__(BS) void k_trace_any(TraceArgs a) {
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_trace_closest_wide(TraceArgs a) {
     __shared__ int smem[TW_LDS_CLOSEST];
     RaySrc src{a.S, a.rays, a.hits, nullptr, a.two_sided};
-    traverse<false>(src, a.n, blockIdx.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
+    traverse<false>(src, a.n, blockIdx.x, gridDim.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
 }
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_trace_any_wide(TraceArgs a) {
     __shared__ int smem[TW_LDS_ANY];
     RaySrc src{a.S, a.rays, nullptr, a.occ, 0};
-    traverse<true>(src, a.n, blockIdx.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
+    traverse<true>(src, a.n, blockIdx.x, gridDim.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
 }
 __global__ void k_gen_rays(ff_dev_camera cam, int32_t W, int32_t H, uint32_t seed, uint32_t sample,
                            float4* rays) {
@@ -2539,16 +2561,22 @@ hipError_t launch_resolve_layers(const float4* layers, uint32_t K, uint32_t WH, 
                        film);
     return hipGetLastError();
 }
+// a query's launch: its workgroups, after one that clears the work counters if
+// it uses them
+template <class K>
+static hipError_t trace_wide(K kernel, const TraceArgs& T, uint32_t* fetch, hipStream_t s) {
+    const uint32_t g = traverse_grid(kernel, T.n);
+    if (!(T.n <= QUAD_MAX && quad_fits(T.S.wide_levels, T.S.max_depth) && quad_fixed(T.n, g * (TW_BLOCK / 64))))
+        hipLaunchKernelGGL(k_reset_fetch, dim3(1), dim3(64), 0, s, fetch);
+    hipLaunchKernelGGL(kernel, dim3(g), dim3(TW_BLOCK), 0, s, T);
+    return hipGetLastError();
+}
 hipError_t launch_trace_closest(const ff_dev_scene& S, const float4* rays, uint32_t n, float4* hits,
                                 int two_sided, uint32_t* fetch, int32_t* ovf, unsigned long long* counts,
                                 int variant, hipStream_t s) {
-    hipLaunchKernelGGL(k_reset_fetch, dim3(1), dim3(64), 0, s, fetch);
     TraceArgs T{S, rays, n, hits, nullptr, two_sided, fetch + F_TRACE * FETCH_SEGS * FETCH_STRIDE, ovf, counts};
-    if (!counts && S.wide) {
-        hipLaunchKernelGGL(k_trace_closest_wide, dim3(traverse_grid(k_trace_closest_wide, n)), dim3(TW_BLOCK), 0, s,
-                           T);
-        return hipGetLastError();
-    }
+    if (!counts && S.wide) return trace_wide(k_trace_closest_wide, T, fetch, s);
+    hipLaunchKernelGGL(k_reset_fetch, dim3(1), dim3(64), 0, s, fetch);
     return trav_dispatch(3, variant, T, s);
 }
 // Device address of `scratch` on `device` (looked up once per device, with
@@ -2578,12 +2606,9 @@ hipError_t static_scratch(int device, int32_t** out) {
 }
 hipError_t launch_trace_any(const ff_dev_scene& S, const float4* rays, uint32_t n, uint8_t* occ, uint32_t* fetch,
                             int32_t* ovf, unsigned long long* counts, int variant, hipStream_t s) {
-    hipLaunchKernelGGL(k_reset_fetch, dim3(1), dim3(64), 0, s, fetch);
     TraceArgs T{S, rays, n, nullptr, occ, 0, fetch + F_TRACE * FETCH_SEGS * FETCH_STRIDE, ovf, counts};
-    if (!counts && S.wide) {
-        hipLaunchKernelGGL(k_trace_any_wide, dim3(traverse_grid(k_trace_any_wide, n)), dim3(TW_BLOCK), 0, s, T);
-        return hipGetLastError();
-    }
+    if (!counts && S.wide) return trace_wide(k_trace_any_wide, T, fetch, s);
+    hipLaunchKernelGGL(k_reset_fetch, dim3(1), dim3(64), 0, s, fetch);
     return trav_dispatch(4, variant, T, s);
 }
 hipError_t launch_gen_rays(const ff_dev_camera& cam, int W, int H, uint32_t seed, uint32_t sample, float4* rays,
