@@ -963,8 +963,16 @@ __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_shadow(ff_paths P, int q) 
 // the previous shading pass) in one launch: workgroups alternate between the
 // two queues by eights (one to each XCD), and each goes on to the other queue,
 // so that either queue's waves fill the other's tail.
-template <bool UNI>
-__global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend_shadow(ff_paths P, int q) {
+//
+// OCC, waves a SIMD: a call of few paths lasts as long as its slowest rays, and
+// 5 waves (96 VGPRs) spill nothing; a call of many is bound by the latency of
+// its visits, and 7 waves (72 VGPRs) hide more of it, spills and all.  5, 6 and
+// 7 waves at 256 k paths (spheres, 16 samples): 3.10, 3.25, 3.45 ms; at 460 k
+// (327 k triangles): 1.57, 1.61, 1.56; at 4.7 M: 4.02, 3.99, 4.06; at 33 M
+// (327 k triangles): 16.0, 15.4, 15.0; at 133 M: 62.3, 59.2, 58.0.
+constexpr uint32_t EXTEND_FEW = 2u << 20, EXTEND_MANY = 16u << 20;
+template <bool UNI, int OCC>
+__global__ __launch_bounds__(TW_BLOCK, OCC) void k_extend_shadow(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_CLOSEST];
     const uint32_t blocks = gridDim.x / 2u;
     for (uint32_t ph = 0; ph < 2; ph++) {
@@ -2436,9 +2444,14 @@ hipError_t extend_shadow_launch(const ff_paths& P, int q, hipStream_t s) {
         const uint32_t g = (traverse_grid(k_extend_shadow_small<UNI>, P.n_slots) + 7u) / 8u * 16u;
         hipLaunchKernelGGL(k_extend_shadow_small<UNI>, dim3(g), dim3(TW_BLOCK), 0, s, P, q);
     } else {
-        const uint32_t g = std::min((traverse_grid(k_extend_shadow<UNI>, P.n_slots) + 7u) / 8u * 16u,
-                                    resident_grid(k_extend_shadow<UNI>, TW_BLOCK));
-        hipLaunchKernelGGL(k_extend_shadow<UNI>, dim3(g), dim3(TW_BLOCK), 0, s, P, q);
+        auto launch = [&](auto kernel) {
+            const uint32_t g = std::min((traverse_grid(kernel, P.n_slots) + 7u) / 8u * 16u,
+                                        std::max(resident_grid(kernel, TW_BLOCK) / 16u, 1u) * 16u);
+            hipLaunchKernelGGL(kernel, dim3(g), dim3(TW_BLOCK), 0, s, P, q);
+        };
+        if (P.n_slots <= EXTEND_FEW) launch(k_extend_shadow<UNI, 5>);
+        else if (P.n_slots < EXTEND_MANY) launch(k_extend_shadow<UNI, 6>);
+        else launch(k_extend_shadow<UNI, 7>);
     }
     return hipGetLastError();
 }
@@ -2475,8 +2488,12 @@ void prepare_launches() {
     (void)resident_grid(k_extend<false>, TW_BLOCK);
     (void)resident_grid(k_shadow<true>, TW_BLOCK);
     (void)resident_grid(k_shadow<false>, TW_BLOCK);
-    (void)resident_grid(k_extend_shadow<true>, TW_BLOCK);
-    (void)resident_grid(k_extend_shadow<false>, TW_BLOCK);
+    (void)resident_grid(k_extend_shadow<true, 5>, TW_BLOCK);
+    (void)resident_grid(k_extend_shadow<false, 5>, TW_BLOCK);
+    (void)resident_grid(k_extend_shadow<true, 6>, TW_BLOCK);
+    (void)resident_grid(k_extend_shadow<false, 6>, TW_BLOCK);
+    (void)resident_grid(k_extend_shadow<true, 7>, TW_BLOCK);
+    (void)resident_grid(k_extend_shadow<false, 7>, TW_BLOCK);
     (void)resident_grid(k_extend_shadow_small<true>, TW_BLOCK);
     (void)resident_grid(k_extend_shadow_small<false>, TW_BLOCK);
     (void)resident_grid(k_logic_shade_large<true>, 512);
