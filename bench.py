@@ -30,22 +30,13 @@ HBM_PEAK_GBS = 8000.0  # MI355X HBM3E, 8 TB/s
 METRIC = "Mrays/s incoherent + spp/s at 1080p; adjoint/fwd time at grad rel-err≤1e-3"
 
 # algorithmic bytes per unit of work: extend ray = 24 (ray) + 16 (hit) +
-# 32 per box tested + 36 per triangle tested; shadow ray = 24 + 4 + same.
-EXT_RAY_BYTES, SHD_RAY_BYTES, NODE_BYTES, TRI_BYTES = 40, 28, 32, 36
+# 16 per box tested (a 64-byte record holds four) + 64 per triangle tested (its
+# record); shadow ray = 24 + 4 + same.
+EXT_RAY_BYTES, SHD_RAY_BYTES, NODE_BYTES, TRI_BYTES = 40, 28, 16, 64
 
 
 def log(msg: str) -> None:
     print(f"[bench] {msg}", file=sys.stderr, flush=True)
-
-
-def _shape_of(variant: int, spp_batch: int) -> dict:
-    """Launch shape of a fixed traversal variant (no autotuning)."""
-    from firefly_amd import abi
-    for v, block, lds, refill, ww, width in abi.traversal_variants():
-        if v == variant:
-            return {"variant": v, "block": block, "lds_entries": lds, "refill": refill, "while_while": ww,
-                    "bvh_width": width, "spp_batch": spp_batch}
-    return {"variant": variant, "spp_batch": spp_batch}
 
 
 def load_counters(kernel: str, workload: str):
@@ -234,8 +225,7 @@ def run_batch(args) -> dict:
     wl = f"batch{len(built)}_uneven"
     ext_bytes = EXT_RAY_BYTES * ext_rays + NODE_BYTES * st.ext_nodes + TRI_BYTES * st.ext_tris
     alg = ext_bytes / (st.ms_extend / 1e3) / 1e9
-    ctr = load_counters("k_extend", wl) if (args.variant == 23 and args.tail_variant == 0 and args.tail_from == 4
-                                            and kp == 16) else None
+    ctr = load_counters("k_extend", wl) if kp == 16 else None
     traffic = round(ctr["dram_bytes_per_dispatch"]) if ctr else None
     dram = traffic * st.launches_extend / (st.ms_extend / 1e3) / 1e9 if traffic else None
     out = {
@@ -504,8 +494,7 @@ def run_multiview(args) -> dict:
     ext_rays = st_t.rays_primary + st_t.rays_extension
     ext_bytes = EXT_RAY_BYTES * ext_rays + NODE_BYTES * st_t.ext_nodes + TRI_BYTES * st_t.ext_tris
     alg = ext_bytes / (st_t.ms_extend / 1e3) / 1e9
-    ctr = load_counters("k_extend", wl) if (args.variant == 23 and args.tail_variant == 0 and
-                                            args.tail_from == 4 and kb == 8) else None
+    ctr = load_counters("k_extend", wl) if kb == 8 else None
     traffic = round(ctr["dram_bytes_per_dispatch"]) if ctr else None
     dram = traffic * st_t.launches_extend / (st_t.ms_extend / 1e3) / 1e9 if traffic else None
     out = {
@@ -574,7 +563,7 @@ def main() -> int:
     ap.add_argument("--cpu-seconds", type=float, default=20.0)
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--variant", type=int, default=23,
-                    help="traversal kernel variant (default: the autotuner's usual pick for the frame)")
+                    help="traversal variant of counted traces (renders do not use it)")
     ap.add_argument("--workload", choices=("all", "frame", "batch", "adjoint", "multiview", "bvh"), default="all")
     ap.add_argument("--adj-spp-batch", type=int, default=16)
     ap.add_argument("--views", type=int, default=32)
@@ -592,7 +581,7 @@ def main() -> int:
                     help="frame: let the autotuner pick the launch shape instead of --variant/--tail-variant")
     ap.add_argument("--no-autotune", action="store_true", help="(the default; kept for older command lines)")
     ap.add_argument("--tail-variant", type=int, default=0,
-                    help="traversal variant of the bounce iterations from --tail-from on (-1: none)")
+                    help="accepted as before (-1: none); renders do not use it")
     ap.add_argument("--tail-from", type=int, default=4)
     ap.add_argument("--copy-mb", type=int, default=0,
                     help="run a plain device copy of this many MiB first (PMC calibration)")
@@ -771,7 +760,8 @@ def run_frame(args) -> dict:
     ms_step = elapsed / args.steps * 1e3
     # stage times and the roofline: one more frame with every launch timed by
     # hipEvents (FF_RENDER_TIMING runs the stages one after another; the timed
-    # frames above overlap each iteration's shadow and extension traversals)
+    # frames above trace each iteration's shadow and extension rays in one launch
+    # and route and shade in another)
     frame(abi.FF_RENDER_TIMING)
     tim = abi.last_render_stats(ctx).as_dict()
 
@@ -789,10 +779,8 @@ def run_frame(args) -> dict:
     b, ms, nl = kern[dom]
     workload = f"icosphere{args.subdiv}_{sd.width}x{sd.height}_{args.spp}spp_d{args.depth}"
     alg = b / (ms / 1e3) / 1e9  # GB/s of algorithmic bytes (every box and triangle tested)
-    # the committed counters describe this launch shape only
-    same_shape = (not args.autotune and args.variant == 23 and args.tail_variant == 0 and args.tail_from == 4 and
-                  args.spp_batch == args.spp)
-    ctr = load_counters(dom, workload) if same_shape else None
+    # the committed counters describe a frame with all its samples in flight
+    ctr = load_counters(dom, workload) if args.spp_batch == args.spp else None
     traffic = round(ctr["dram_bytes_per_dispatch"]) if ctr else None
     dram = traffic * nl / (ms / 1e3) / 1e9 if traffic else None  # GB/s of measured HBM bytes
     roofline = {
@@ -812,7 +800,7 @@ def run_frame(args) -> dict:
             "bytes_per_launch": round(b / nl),
             "gbs": round(alg, 2),
             "over_hbm_peak": round(alg / HBM_PEAK_GBS, 5),
-            "basis": "40 B per ray + 32 B per box + 36 B per triangle tested (this run's counters); "
+            "basis": "40 B per ray + 16 B per box + 64 B per triangle tested (this run's counters); "
                      "cache-inclusive, so not bounded by the HBM peak",
         },
         "limiter": limiter_of(ctr, dram / HBM_PEAK_GBS if dram else None),
@@ -846,9 +834,9 @@ def run_frame(args) -> dict:
         "config": {"workload": workload, "width": sd.width, "height": sd.height, "spp": args.spp,
                    "max_depth": args.depth, "tris": sd.n_tris, "env": f"{sd.env.shape[1]}x{sd.env.shape[0]}",
                    "spp_batch": args.spp_batch},
-        "launch_shape": (tuned["best"] if tuned else dict(_shape_of(max(args.variant, 0), args.spp_batch),
-                                                           tail_variant=args.tail_variant,
-                                                           tail_from=args.tail_from if args.tail_variant >= 0 else 0)),
+        # (a render's walk follows its number of paths; the variants are shapes of
+        # counted traces)
+        "launch_shape": tuned["best"] if tuned else {"walk": "4-wide compressed records", "spp_batch": args.spp_batch},
         "spp_per_s_1080p": round(spp_s, 3),
         "total_mrays_s": round(total_rays / elapsed / 1e6, 3),
         "rays_per_step": {k: int(tot[k] / args.steps) for k in ("rays_primary", "rays_extension", "rays_shadow")},
@@ -857,7 +845,8 @@ def run_frame(args) -> dict:
         "rays_shadow_gated_per_step": int(tot["rays_shadow_gated"] / args.steps),
         "stage_ms_per_step": stages,
         "stage_ms_note": ("one more frame with every launch timed by hipEvents, which runs the stages one after "
-                          "another; the timed frames overlap each iteration's shadow and extension traversals"),
+                          "another; the timed frames trace each iteration's shadow and extension rays in one launch "
+                          "and route and shade in another"),
         "traversal": per_ray,
         "envmap_update_ms": round(env_ms, 4),
         "roofline": roofline,
