@@ -853,25 +853,29 @@ ff_status render_requests(ff_context* ctx, const std::vector<HostReq>& reqs, int
         return FF_OK;
     };
     // One batch of the adjoint replay.  As in the forward, a vertex's shadow
-    // rays are traced with the next extension rays; the vertex's gradient
-    // kernel, which needs their visibility, follows.  (Apart, with the shadow
-    // rays of few paths in a launch of their own: eight 192x192 views 9.36
-    // against 8.22 ms with their forward, 201x151 deterministic 4.25 against
-    // 3.65 ms, 512x512 16 samples 8.40 against 8.16 ms.)
+    // rays are traced with the next extension rays; the vertex's gradients,
+    // which need their visibility, follow with the next routing and shading in
+    // one launch.  (With the shadow rays in a launch of their own eight 192x192
+    // views took 9.36 against 8.22 ms with their forward, 201x151 deterministic
+    // 4.25 against 3.65 ms.)
     auto batch_adj = [&]() -> ff_status {
         HIP_TRY(ffk::launch_batch_begin(p, hs));
         HIP_TRY(timed(4, [&] { return ffk::launch_generate(p, hs); }));
         int cur = 0;
         for (int32_t it = 1; it <= max_depth + 1; it++) {
             HIP_TRY(trace(cur));
-            if (it > 1) {
-                for (int m = 0; m < 3; m++)
-                    if (has_type[m]) HIP_TRY(timed(3, [&] { return ffk::launch_shade_adj(m, p, cur, p.n_slots, hs); }));
-            }
-            HIP_TRY(timed(2, [&] { return ffk::launch_logic_adj(p, cur, p.n_slots, hs); }));
-            if (it <= max_depth) {
-                for (int m = 0; m < 4; m++)
-                    if (has_type[m]) HIP_TRY(timed(3, [&] { return ffk::launch_shade_nee(m, p, 1 - cur, p.n_slots, hs); }));
+            if (!timing) {
+                HIP_TRY(ffk::launch_replay(p, cur, it, it > max_depth, hs));
+            } else {
+                if (it > 1) {
+                    for (int m = 0; m < 3; m++)
+                        if (has_type[m]) HIP_TRY(timed(3, [&] { return ffk::launch_shade_adj(m, p, cur, p.n_slots, hs); }));
+                }
+                HIP_TRY(timed(2, [&] { return ffk::launch_logic_adj(p, cur, p.n_slots, hs); }));
+                if (it <= max_depth) {
+                    for (int m = 0; m < 4; m++)
+                        if (has_type[m]) HIP_TRY(timed(3, [&] { return ffk::launch_shade_nee(m, p, 1 - cur, p.n_slots, hs); }));
+                }
             }
             cur = 1 - cur;
         }

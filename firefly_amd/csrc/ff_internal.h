@@ -24,6 +24,7 @@ hipError_t launch_batch_begin(const ff_paths& P, hipStream_t s);
 hipError_t launch_generate(const ff_paths& P, hipStream_t s);
 hipError_t launch_extend(const ff_paths& P, int q, hipStream_t s);
 hipError_t launch_shadow(const ff_paths& P, int q, hipStream_t s);
+hipError_t launch_replay(const ff_paths& P, int q, int iter, int last, hipStream_t s);
 hipError_t launch_logic_shade(const ff_paths& P, int q, int iter, int last, hipStream_t s);
 hipError_t launch_extend_shadow(const ff_paths& P, int q, hipStream_t s);
 hipError_t launch_logic(const ff_paths& P, int q, int iter, uint32_t n_max, hipStream_t s);

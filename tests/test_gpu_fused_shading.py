@@ -92,3 +92,30 @@ def test_replay_with_rays_traced_together(gpu, width, height, k, spp, depth, typ
     for a, b in zip(*out):
         assert np.array_equal(a, b)
     assert np.any(out[0][0] != 0)
+
+
+@pytest.mark.parametrize("width,height,k", [(SMALL // 512, 512, 1), (SMALL // 512 + 1, 512, 1), (1031, 400, 2)])
+def test_replay_forms_by_paths_in_flight(gpu, width, height, k):
+    """The replay's one-launch forms on either side of their limit, with paths
+    left over between tiles, of several scenes: deterministic sums as apart."""
+    import torch
+    depth, spp = 3, k
+    d = torch.from_numpy(np.random.default_rng(2).normal(size=(height, width, 4)).astype(np.float32)).cuda()
+    items, paths, grads = [], [], []
+    for i, (w, h) in enumerate([(width, height), (40, 30)]):
+        sc, env, cam = _scene(gpu, w, h, depth, i, ALL)
+        film = torch.zeros((h, w, 4), dtype=torch.float32, device="cuda")
+        items.append((sc, env, cam, w, h, spp, depth, 5 + i, film))
+        paths.append(torch.zeros((spp, h, w, 4), dtype=torch.float32, device="cuda"))
+    abi.render_batch(gpu, items, path_radiance=paths, spp_batch=k)
+    out = []
+    for flags in (0, abi.FF_RENDER_TIMING):
+        grads = [torch.zeros((it[1].hgt, it[1].w, 3), dtype=torch.float32, device="cuda") for it in items]
+        abi.adjoint_batch(gpu, items, paths, [d, d[:30, :40].contiguous()], env_grads=grads,
+                          flags=flags | abi.FF_ADJOINT_DETERMINISTIC, spp_batch=k)
+        torch.cuda.synchronize()
+        st = abi.last_render_stats(gpu)
+        out.append([*(g.cpu().numpy() for g in grads), [getattr(st, c) for c in COUNTS]])
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    assert np.any(out[0][0] != 0) and np.any(out[0][1] != 0)
