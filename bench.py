@@ -54,7 +54,8 @@ def load_counters(kernel: str, workload: str):
 
 def limiter_of(ctr, dram_frac):
     """The resource the committed counters put closest to its roof: VALU
-    issue (SQ_INSTS_VALU per CU-cycle, ceiling 1) or HBM bandwidth (this
+    issue (SQ_INSTS_VALU per CU-cycle; probes of single instructions reach 0.95
+    to 1.6, so 1 is taken as a mix's roof) or HBM bandwidth (this
     run's traffic rate over the 8 TB/s peak); latency when neither reaches
     0.6 of its roof."""
     if not ctr or dram_frac is None:
@@ -64,7 +65,7 @@ def limiter_of(ctr, dram_frac):
     return {"resource": res, "valu_issue_frac": round(v, 3), "hbm_frac": round(dram_frac, 3),
             "valu_lane_utilization": round(ctr["valu_lane_utilization"], 3),
             "l2_hit_rate": round(ctr["l2_hit_rate"], 3),
-            "basis": "SQ_INSTS_VALU / (256 CUs x cycles), ceiling 1; lanes SQ_THREAD_CYCLES_VALU / "
+            "basis": "SQ_INSTS_VALU / (256 CUs x cycles), roof of a mix about 1; lanes SQ_THREAD_CYCLES_VALU / "
                      "(64 x SQ_ACTIVE_INST_VALU); L2 TCC_HIT / (TCC_HIT + TCC_MISS); from " + ctr["source"]}
 
 
