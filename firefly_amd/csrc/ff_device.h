@@ -12,6 +12,7 @@
 #include <stdint.h>
 
 #include "ff_layout.h"
+#include "ff_refill.h"
 
 namespace ffd {
 
@@ -1369,91 +1370,27 @@ struct QStage {
     }
 };
 
-// Segmented work fetch of the persistent traversal: queue [0, n) is split
-// into FETCH_SEGS segments with a counter each; a wave draws from its current
-// segment and, once that is exhausted, finds the next segment with work left
-// by reading all FETCH_SEGS counters at once (lane k reads counter k with a
-// device-coherent load, one round trip).  It reports `done` only when such a
-// scan finds every segment exhausted.  Counters only grow, so a segment seen
-// exhausted stays exhausted and a wave fails at most FETCH_SEGS times.
-// Wave-uniform: every lane calls it with the same arguments.
+// The work counters in device memory (SegFetch): lane 0 claims; lane k reads
+// counter k with a device-coherent load, one round trip for all.
 static_assert(FETCH_SEGS == 64, "one segment per lane of the scan");
-struct SegFetch {
-    uint32_t* ctr;   // FETCH_SEGS counters, FETCH_STRIDE words apart
-    uint32_t n, seg_len, seg;
-    uint32_t res_first, res_left;  // items claimed by this wave and not yet handed out
-    uint32_t chunk;                // items claimed per atomic
-    __device__ __forceinline__ void init(uint32_t* c, uint32_t n_, uint32_t home) {
-        ctr = c;
-        n = n_;
-        seg_len = (n + FETCH_SEGS - 1) / FETCH_SEGS;
-        seg = home % FETCH_SEGS;
-        res_first = 0;
-        res_left = 0;
-        // a wave claims up to 1/256 of a segment (at most FETCH_CHUNK) per
-        // atomic, so refills of a few lanes rarely wait on the memory-side
-        // atomic, and the last claims of a segment stay small
-        uint32_t c8 = seg_len >> 8;
-        chunk = c8 < FETCH_CHUNK ? c8 : FETCH_CHUNK;
+struct DevCounters {
+    uint32_t* ctr;  // FETCH_SEGS counters, FETCH_STRIDE words apart
+    __device__ __forceinline__ uint32_t claim(uint32_t seg, uint32_t want) const {
+        uint32_t base = 0;
+        if (__lane_id() == 0) base = atomicAdd(ctr + (size_t)seg * FETCH_STRIDE, want);
+        return __shfl(base, 0);
     }
-    // Hands out up to `want` items from the wave's reservoir, refilling it
-    // from the counters when it is empty.  Same contract as take().
-    __device__ __forceinline__ uint32_t take_chunked(uint32_t want, uint32_t& got, bool& done) {
-        done = false;
-        if (res_left == 0) {
-            uint32_t g;
-            uint32_t f = take(want > chunk ? want : chunk, g, done);
-            res_first = __builtin_amdgcn_readfirstlane(f);
-            res_left = __builtin_amdgcn_readfirstlane(g);
-        }
-        got = res_left < want ? res_left : want;
-        uint32_t first = res_first;
-        res_first += got;
-        res_left -= got;
-        if (res_left > 0) done = false;
-        return first;
+    template <class F>
+    __device__ __forceinline__ uint64_t open(const F& f) const {
+        const uint32_t k = __lane_id();
+        const uint32_t lk = f.seg_size(k);
+        const uint32_t v = lk ? __hip_atomic_load(ctr + (size_t)k * FETCH_STRIDE, __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_AGENT)
+                              : 0u;
+        return __ballot(lk > 0 && v < lk);
     }
-    __device__ __forceinline__ uint32_t seg_size(uint32_t s) const {
-        uint32_t lo = s * seg_len;
-        return lo < n ? (n - lo < seg_len ? n - lo : seg_len) : 0u;
-    }
-    // Grants up to `want` items: returns the first item and the number
-    // granted; got == 0 with done == false means "try again later".
-    __device__ __forceinline__ uint32_t take(uint32_t want, uint32_t& got, bool& done) {
-        got = 0;
-        done = false;
-        for (int attempt = 0; attempt < 2; attempt++) {
-            uint32_t len = seg_size(seg);
-            if (len > 0) {
-                uint32_t base = 0;
-                if (__lane_id() == 0) base = atomicAdd(ctr + (size_t)seg * FETCH_STRIDE, want);
-                base = __shfl(base, 0);
-                if (base < len) {
-                    got = len - base < want ? len - base : want;
-                    return seg * seg_len + base;
-                }
-            }
-            // current segment exhausted: scan every counter (lane k -> segment k)
-            uint32_t k = __lane_id();
-            bool avail = false;
-            if (k < FETCH_SEGS) {
-                uint32_t lk = seg_size(k);
-                uint32_t v = lk ? __hip_atomic_load(ctr + (size_t)k * FETCH_STRIDE, __ATOMIC_RELAXED,
-                                                    __HIP_MEMORY_SCOPE_AGENT)
-                                : 0u;
-                avail = lk > 0 && v < lk;
-            }
-            uint64_t m = __ballot(avail);
-            if (m == 0) {
-                done = true;
-                return 0;
-            }
-            // next segment with work, searching upwards from the current one
-            uint32_t sh = (seg + 1) % 64u;
-            uint64_t rot = (m >> sh) | (sh ? (m << (64u - sh)) : 0ull);
-            seg = (sh + (uint32_t)(__ffsll((unsigned long long)rot) - 1)) % 64u;
-        }
-        return 0;
+    __device__ __forceinline__ uint32_t uniform(uint32_t v) const {
+        return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
     }
 };
 

@@ -305,8 +305,8 @@ struct RaySrc {  // a plain ray array (ff_trace_closest / ff_trace_any)
 template <int BS, int LDS, int REFILL, bool ANY, int WW, bool WIDE>
 __device__ __forceinline__ void trav_persistent(const RaySrc& src, uint32_t n, uint32_t* fetch, int32_t* ovf,
                                                 unsigned long long* cnt, int* smem) {
-    SegFetch F;
-    F.init(fetch, n, blockIdx.x * (BS / 64) + (threadIdx.x >> 6));
+    SegFetch<DevCounters> F;
+    F.init(DevCounters{fetch}, n, blockIdx.x * (BS / 64) + (threadIdx.x >> 6));
     Stack st;
     st.lds = (lds_int*)&smem[threadIdx.x];
     st.lds_stride = BS;
@@ -517,16 +517,15 @@ __device__ __forceinline__ void trav_persistent(const RaySrc& src, uint32_t n, u
 // at 16 24.2, at 48 29.1; testing held triangles once 2, 4, 8 or 16 lanes hold
 // one is alike there (24.1-24.4), and 2 is best where a launch lasts as long as
 // its slowest ray (160x120 frame: 0.86 ms, 0.87 at 4, 1.03 at 16).
-constexpr int TW_BLOCK = 256, TW_REFILL = 16, TW_LEAF = 2, TW_OCC = 6;
+constexpr int TW_BLOCK = 256, TW_LEAF = 2, TW_OCC = 6;  // (TW_REFILL: ff_refill.h)
 // Launches of at most QUAD_MAX rays give every ray four lanes: at 19200 rays a
 // launch takes 50 us instead of 70, at 131072 (16 rays on each of 8192 waves)
 // the two are even, at 262144 rays four lanes cost 1.2x (8 spheres, 256x256).
 constexpr uint32_t QUAD_MAX = 131072;
-// A launch of fewer rays than lanes spreads them over this many waves (one or
-// two to a SIMD), so that a wave waits for fewer of its neighbours' visits:
-// 160x120 frame 0.99 ms with full waves, 0.87 ms; four lanes to a ray over 1024
-// waves 0.725 ms, over 2048 0.737, over 4096 0.78.
-constexpr uint32_t TW_SPREAD = 2048, QUAD_SPREAD = 1024;
+// Waves that such a launch spreads its rays over (TW_SPREAD, of the one-lane
+// walk: ff_refill.h): 160x120 frame over 1024 waves 0.725 ms, over 2048 0.737,
+// over 4096 0.78.
+constexpr uint32_t QUAD_SPREAD = 1024;
 
 // Persistent traversal of the compressed wide records (see ff_device.h), with
 // the same work distribution: a lane owns a ray, a wave refills its idle lanes
@@ -538,8 +537,8 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
                                           int32_t* ovf, unsigned long long* cnt, int* smem) {
     constexpr uint32_t IDLE = 0xffffffffu;
     constexpr int LDS = FF_LDS_STACK;
-    SegFetch F;
-    F.init(fetch, n, block * (BS / 64) + (threadIdx.x >> 6));
+    SegFetch<DevCounters> F;
+    F.init(DevCounters{fetch}, n, block * (BS / 64) + (threadIdx.x >> 6));
     Stack st;
     st.lds = (lds_int*)&smem[threadIdx.x];
     st.lds_stride = BS;
@@ -579,11 +578,9 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
     // one distance, a NaN plane distance) park their lane; once many lanes are
     // parked, or no other work is left, those rays walk the binary records with
     // every other lane idle (the walk's registers then add nothing to the loop).
-    constexpr uint32_t PARK_MOST = 32;
     bool parked = false;
-    const uint32_t cap = n >= TW_SPREAD * 64u ? 64u : n / TW_SPREAD + 1u;
-    const bool mine = __lane_id() < cap;
-    const uint32_t refill = cap < (uint32_t)TW_REFILL ? cap : (uint32_t)TW_REFILL;
+    const uint32_t lanes = wide_lanes(n), refill = wide_refill_at(lanes);
+    const bool mine = __lane_id() < lanes;
     for (;;) {
         for (;;) {
             if (Src::kChain) {
@@ -600,14 +597,15 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
             }
             uint64_t idle = __ballot(mine && (id == IDLE || parked));
             if ((uint32_t)__popcll(idle) >= refill) {
-                const bool full = (uint32_t)__popcll(__ballot(parked)) >= PARK_MOST;
-                if (more && !full) {
-                    idle = __ballot(mine && id == IDLE);
+                idle = __ballot(mine && id == IDLE);
+                const WideRefill take =
+                    wide_refill(more, (uint32_t)__popcll(__ballot(parked)), (uint32_t)__popcll(idle), lanes);
+                if (take.want != 0u) {
                     uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(idle >> 32),
                                                               __builtin_amdgcn_mbcnt_lo((uint32_t)idle, 0u));
                     uint32_t got;
                     bool done;
-                    uint32_t first = F.take_chunked((uint32_t)__popcll(idle), got, done);
+                    uint32_t first = F.take_chunked(take.want, got, done);
                     if (done) more = false;
                     c_rays += got;
                     if (mine && id == IDLE && rank < got) {
@@ -618,7 +616,7 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
                     }
                 }
                 if (__ballot(id != IDLE && !parked) == 0) {
-                    if (!more || full) break;
+                    if (!more || take.full) break;
                     continue;
                 }
             }
@@ -764,8 +762,8 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
                                           unsigned long long* cnt, int* smem) {
     constexpr uint32_t IDLE = 0xffffffffu;
     const uint32_t wave = block * (BS / 64) + (threadIdx.x >> 6);
-    SegFetch F;
-    F.init(fetch, n, wave);
+    SegFetch<DevCounters> F;
+    F.init(DevCounters{fetch}, n, wave);
     const uint32_t lane = __lane_id(), k = lane & 3u, lead = lane & ~3u;
     const uint64_t below = ((1ull << lead) - 1ull) & 0x1111111111111111ull;
     QuadStack<BS> st;

@@ -16,6 +16,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "ff_refill.h"
+
 #define FF_BLOCK 256          // threads per workgroup of the stage kernels (4 waves of 64)
 #define FF_TRAV_THREADS 524288 // threads of the persistent traversal grids (any block size)
 #define FF_LDS_MIN 8          // smallest LDS stack of a traversal variant (sizes the overflow area)
@@ -46,17 +48,6 @@
 #define C_SHD1 7
 #define C_MAT1 8
 #define C_COUNT 16
-
-// Work counters of the persistent traversal kernels: the queue is split into
-// FETCH_SEGS segments with one counter each, every counter on its own 128-B
-// line (device-scope atomics on one address serialise at the memory side).
-#define FETCH_SEGS 64
-#define FETCH_STRIDE 32
-#define F_EXT 0
-#define F_SHD 1
-#define F_TRACE 2
-#define FETCH_WORDS (3 * FETCH_SEGS * FETCH_STRIDE)
-#define FETCH_CHUNK 256  // largest claim of one wave from a work counter
 
 // LDS stack entries of a traversal lane; the four-lane walk has four times as
 // many for its ray: three entries a wide level, or the binary tree's depth
