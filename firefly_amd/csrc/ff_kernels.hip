@@ -1726,20 +1726,25 @@ __global__ __launch_bounds__(BS, 4) void k_logic_shade(ff_paths P, int q, int it
 // (path replay backpropagation).  Sampling is detached: directions, pdfs,
 // MIS weights and Russian roulette are those of the forward.
 
-// One term of d loss / d parameter into gradient target element i.
-__device__ __forceinline__ void grad_add(const ff_paths& P, float* buf, uint64_t off, uint32_t i, float v) {
-    if (v == 0.f) return;
+// d loss / d parameter into gradient target element i: the terms v and u (0:
+// none).  The deterministic sums take each term by itself, as 64-bit fixed
+// point; the float sum takes both at once.
+__device__ __forceinline__ void grad_add(const ff_paths& P, float* buf, uint64_t off, uint32_t i, float v, float u) {
     if (P.gmode == GM_FLOAT) {
-        unsafeAtomicAdd(buf + i, v);
-    } else if (P.gmode == GM_BOUND) {
-        uint64_t a = off + i;
-        atomicMax(&P.g_max[a], __float_as_uint(fabsf(v)));
-        atomicAdd(&P.g_cnt[a], 1u);
+        const float s = v + u;
+        if (s != 0.f) unsafeAtomicAdd(buf + i, s);
+        return;
+    }
+    if (v == 0.f && u == 0.f) return;
+    const uint64_t a = off + i;
+    if (P.gmode == GM_BOUND) {
+        const uint32_t bv = __float_as_uint(fabsf(v)), bu = __float_as_uint(fabsf(u));
+        atomicMax(&P.g_max[a], bv > bu ? bv : bu);
+        atomicAdd(&P.g_cnt[a], (v != 0.f ? 1u : 0u) + (u != 0.f ? 1u : 0u));
     } else {
-        uint64_t a = off + i;
-        int e = fixed_exponent(P.g_max[a], P.g_cnt[a]);
-        long long qv = __double2ll_rn(ldexp((double)v, e));
-        atomicAdd(&P.g_fx[a], (unsigned long long)qv);
+        const int e = fixed_exponent(P.g_max[a], P.g_cnt[a]);
+        const long long q = __double2ll_rn(ldexp((double)v, e)) + __double2ll_rn(ldexp((double)u, e));
+        atomicAdd(&P.g_fx[a], (unsigned long long)q);
     }
 }
 // Scatter of bilinear footprints onto gradient texels, the wave together.
@@ -1751,19 +1756,28 @@ __device__ __forceinline__ void grad_add(const ff_paths& P, float* buf, uint64_t
 struct Scatter {  // of one wave
     uint32_t idx[4][64];
     float w[4][64];
-    float val[3][64];
+    float val[3][64], more[3][64];
     float* buf[64];
     uint64_t off[64];
 };
 // on: the lane has a footprint tp of target T with value val[0..C) (per
-// channel, before the tap weights).  Every lane of the wave calls it.
-template <int C>
+// channel, before the tap weights).  TWO: with the values of two terms, whose
+// atomics are shared: in float they are added first, in the deterministic sums
+// they stay apart.  Every lane of the wave calls it.
+template <int C, bool TWO = false>
 __device__ __forceinline__ void scatter(const ff_paths& P, Scatter& S, bool on, const ff_dev_gtarget& T,
-                                        const Taps& tp, f3 val) {
+                                        const Taps& tp, f3 val, f3 more = V3(0.f, 0.f, 0.f)) {
     const uint64_t m = __ballot(on);
     if (m == 0) return;
+    const bool apart = TWO && P.gmode != GM_FLOAT;
     if (on) {
         const uint32_t f = __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+        if (TWO && !apart) val = vadd(val, more);
+        if (apart) {
+            S.more[0][f] = more.x;
+            S.more[1][f] = more.y;
+            S.more[2][f] = more.z;
+        }
 #pragma unroll
         for (int k = 0; k < 4; k++) {
             S.idx[k][f] = tp.i[k];
@@ -1780,7 +1794,8 @@ __device__ __forceinline__ void scatter(const ff_paths& P, Scatter& S, bool on, 
     const uint32_t total = (uint32_t)__popcll(m) * (4u * C);
     for (uint32_t e = __lane_id(); e < total; e += 64u) {
         const uint32_t f = e / (4u * C), r = e % (4u * C), k = r / C, c = r % C;
-        grad_add(P, S.buf[f], S.off[f], C * S.idx[k][f] + c, S.w[k][f] * S.val[c][f]);
+        const float w = S.w[k][f];
+        grad_add(P, S.buf[f], S.off[f], C * S.idx[k][f] + c, w * S.val[c][f], apart ? w * S.more[c][f] : 0.f);
     }
     __threadfence_block();
     __builtin_amdgcn_wave_barrier();
@@ -1799,10 +1814,10 @@ __device__ __forceinline__ void scatter_env(const ff_paths& P, Scatter& S, bool 
     }
     scatter<3>(P, S, on, T, tp, val);
 }
-// d loss / d (texture t value at (u, v)) = val (C channels) onto its texels
+// d loss / d (texture t value at (u, v)) = val + more (C channels) onto its texels
 template <int C>
 __device__ __forceinline__ void scatter_tex(const ff_paths& P, Scatter& S, bool on, const ff_dev_request& R, int t,
-                                            float u, float v, f3 val) {
+                                            float u, float v, f3 val, f3 more) {
     ff_dev_gtarget T{nullptr, 0};
     Taps tp{};
     if (on) T = R.gt[1 + t];
@@ -1811,7 +1826,7 @@ __device__ __forceinline__ void scatter_tex(const ff_paths& P, Scatter& S, bool 
         const ff_tex_desc& td = R.S.tex[t];
         tp = taps_of(td.w, td.h, u, v);
     }
-    scatter<C>(P, S, on, T, tp, val);
+    scatter<C, true>(P, S, on, T, tp, val, more);
 }
 
 // wf_logic of the replay: same termination, Russian roulette and routing as
@@ -1968,7 +1983,8 @@ __device__ __forceinline__ void replay_gradients(const ff_paths& P, Scatter& S, 
     const ff_dev_request& R = P.reqs[req_of(P, id)];
     ShadeOut so;
     bool visL = false, visS = false, visD = false, alb_on = false, rough_on = false;
-    f3 w = V3(0.f, 0.f, 0.f), g_alb = w, g_rough = w;
+    f3 w = V3(0.f, 0.f, 0.f), g_alb = w, g_rough = w;  // NEE
+    f3 h_alb = w, h_rough = w;                         // continuation
     if (live) {
         shade_core<TYPE, true, UNI>(P, id, {P.nee[3 * id], P.nee[3 * id + 1], P.nee[3 * id + 2]}, so);
         f3 beta = xyz(P.beta[id]);
@@ -1999,16 +2015,16 @@ __device__ __forceinline__ void replay_gradients(const ff_paths& P, Scatter& S, 
             f3 qv = V3(so.fext.x != 0.f ? dl.x * Lrem.x / so.fext.x : 0.f,
                        so.fext.y != 0.f ? dl.y * Lrem.y / so.fext.y : 0.f,
                        so.fext.z != 0.f ? dl.z * Lrem.z / so.fext.z : 0.f);
-            g_alb = vadd(g_alb, vmul(qv, so.dext_alb));
-            g_rough.x = g_rough.x + vdot(qv, so.dext_r);
+            h_alb = vmul(qv, so.dext_alb);
+            h_rough.x = vdot(qv, so.dext_r);
             beta = vmul(beta, vdiv(vscl(so.fext, so.cos_ext), so.pdf_ext));
         }
         nst = (nst & (ST_LEN_MASK | ST_INSIDE)) | (dead ? ST_DEAD : 0u);
         P.Lp[id] = f4(Lrem, 0.f);
         P.beta[id] = f4(beta, __uint_as_float(nst));
     }
-    scatter_tex<3>(P, S, alb_on, R, so.at, so.tu, so.tv, g_alb);
-    if (TYPE != MAT_DIFFUSE) scatter_tex<1>(P, S, rough_on, R, so.rt, so.tu, so.tv, g_rough);
+    scatter_tex<3>(P, S, alb_on, R, so.at, so.tu, so.tv, g_alb, h_alb);
+    if (TYPE != MAT_DIFFUSE) scatter_tex<1>(P, S, rough_on, R, so.rt, so.tu, so.tv, g_rough, h_rough);
     scatter_env(P, S, visL && so.a_on, R, so.wi, vmul(w, so.kA));
     if (TYPE != MAT_DIFFUSE) scatter_env(P, S, visS, R, so.wi_s, vmul(w, so.kB));
     if (TYPE != MAT_CONDUCTOR) scatter_env(P, S, visD, R, so.wi_d, vmul(w, so.kC));
