@@ -579,7 +579,7 @@ def main() -> int:
     ap.add_argument("--batch-only", action="store_true",
                     help="batch workload: only the batched call at the first --batch-k value (for profiling)")
     ap.add_argument("--autotune", action="store_true",
-                    help="frame: let the autotuner pick the launch shape instead of --variant/--tail-variant")
+                    help="frame: let the autotuner pick the samples in flight (and the variant of counted traces)")
     ap.add_argument("--no-autotune", action="store_true", help="(the default; kept for older command lines)")
     ap.add_argument("--tail-variant", type=int, default=0,
                     help="accepted as before (-1: none); renders do not use it")
@@ -723,15 +723,12 @@ def run_frame(args) -> dict:
         from firefly_amd.autotune import autotune
         t0 = time.perf_counter()
         tuned = autotune(ctx, scene, env, cam, sd.width, sd.height, args.depth, sd.seed, probe_spp=4,
-                         batches=(1, 2, 4), refine_batches=(8, 16, 32, 64), refine_spp=args.spp,
-                         tail_candidates=(0, 1, 22, 25, 26), tail_from=(3, 4, 5))
+                         batches=(1, 2, 4), refine_batches=(8, 16, 32, 64), refine_spp=args.spp)
         args.spp_batch = tuned["best"]["spp_batch"]
         args.tuned_variant = tuned["best"]["variant"]
         args.tuned_tail = (tuned["best"].get("tail_variant", -1), tuned["best"].get("tail_from", 4))
         for c in tuned["candidates"]:
-            log(f"  variant {c['variant']} (block {c['block']}, lds {c['lds_entries']}, refill {c['refill']}, "
-                f"ww {c['while_while']}, width {c['bvh_width']}) "
-                f"spp_batch {c['spp_batch']} at {c.get('probe_spp', 4)} spp: {c['seconds'] * 1e3:.1f} ms")
+            log(f"  spp_batch {c['spp_batch']} at {c['probe_spp']} spp: {c['seconds'] * 1e3:.1f} ms")
         log(f"autotune ({time.perf_counter() - t0:.1f} s): {tuned['best']}")
 
     def frame(flags=0):

@@ -412,12 +412,13 @@ def traversal_variants():
 
 
 def set_traversal_variant(ctx: Context, variant: int) -> None:
+    """Variant of the context's traces that count; renders and uncounted traces do not read it."""
     check(_lib().ff_set_traversal_variant(ctx.h, variant))
 
 
 def set_traversal_tail(ctx: Context, variant: int, from_iteration: int = 4) -> None:
-    """Traversal variant of the bounce iterations from `from_iteration` on
-    (-1: the context's variant everywhere)."""
+    """Checks its arguments; no launch reads them (renders take their launch
+    shape from the number of rays)."""
     check(_lib().ff_set_traversal_tail(ctx.h, variant, from_iteration))
 
 
