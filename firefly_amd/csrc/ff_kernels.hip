@@ -534,7 +534,7 @@ constexpr uint32_t QUAD_SPREAD = 1024;
 // or when no lane can walk on.
 template <int BS, bool ANY, class Src>
 __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t block, uint32_t* fetch,
-                                          int32_t* ovf, unsigned long long* cnt, int* smem) {
+                                          int32_t* ovf, unsigned long long* cnt, lds_u32* again_lds, int* smem) {
     constexpr uint32_t IDLE = 0xffffffffu;
     constexpr int LDS = FF_LDS_STACK;
     SegFetch<DevCounters> F;
@@ -704,7 +704,7 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
                 const ff_dev_scene& S = src.scene(id);
                 f3 o, d;
                 src.load_again(id, aux, o, d, two);
-                const Hit h = reference_walk<ANY>(bvh_of(S), S.tris, o, d, two, st);
+                const Hit h = reference_walk<ANY>(bvh_of(S), S.tris, o, d, two, st, again_lds);
                 if (ANY) {
                     const bool occ = h.id >= 0;
                     src.occluded(id, aux, occ);
@@ -730,10 +730,7 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
         nxt = false;
         st.sp = 1;
     }
-    if (cnt && __lane_id() == 0) {
-        atomicAdd(&cnt[0], 4ull * cn);
-        atomicAdd(&cnt[1], (unsigned long long)ct);
-    }
+    if (cnt && __lane_id() == 0) add_tested(cnt, cn, ct, again_lds);
     src.count(__lane_id() == 0 ? c_rays : 0u, __lane_id() == 0 ? c_gated : 0u);
 }
 
@@ -759,7 +756,7 @@ __host__ __device__ __forceinline__ bool quad_fixed(uint32_t n, uint32_t waves) 
 // the deepest stack).
 template <int BS, bool ANY, class Src>
 __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t block, uint32_t blocks, uint32_t* fetch,
-                                          unsigned long long* cnt, int* smem) {
+                                          unsigned long long* cnt, lds_u32* again_lds, int* smem) {
     constexpr uint32_t IDLE = 0xffffffffu;
     const uint32_t wave = block * (BS / 64) + (threadIdx.x >> 6);
     SegFetch<DevCounters> F;
@@ -901,7 +898,7 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
                 win = k == 0u;
                 if (win) {
                     const ff_dev_scene& S = src.scene(id);
-                    best = reference_walk<ANY>(bvh_of(S), S.tris, R.o, R.d, two, st);
+                    best = reference_walk<ANY>(bvh_of(S), S.tris, R.o, R.d, two, st, again_lds);
                     if (ANY) occ = best.id >= 0;
                 }
             }
@@ -918,10 +915,7 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
         if (Src::kChain)
             c_gated += (uint32_t)(__popcll(__ballot(gated & 1u)) + 2 * __popcll(__ballot(gated & 2u))) / 4u;
     }
-    if (cnt && lane == 0) {
-        atomicAdd(&cnt[0], 4ull * cn);
-        atomicAdd(&cnt[1], (unsigned long long)ct);
-    }
+    if (cnt && lane == 0) add_tested(cnt, cn, ct, again_lds);
     src.count(lane == 0 ? c_rays : 0u, lane == 0 ? c_gated : 0u);
 }
 
@@ -929,16 +923,23 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
 // (its waves start on the queue's segments in turn)
 template <bool ANY, class Src>
 __device__ __forceinline__ void traverse(const Src& src, uint32_t n, uint32_t block, uint32_t blocks, bool quad,
-                                         uint32_t* fetch, int32_t* ovf, unsigned long long* cnt, int* smem) {
-    if (quad && n <= QUAD_MAX) trav_quad<TW_BLOCK, ANY>(src, n, block, blocks, fetch, cnt, smem);
-    else trav_wide<TW_BLOCK, ANY>(src, n, block, fetch, ovf, cnt, smem);
+                                         uint32_t* fetch, int32_t* ovf, unsigned long long* cnt, lds_u32* again_lds,
+                                         int* smem) {
+    if (quad && n <= QUAD_MAX) trav_quad<TW_BLOCK, ANY>(src, n, block, blocks, fetch, cnt, again_lds, smem);
+    else trav_wide<TW_BLOCK, ANY>(src, n, block, fetch, ovf, cnt, again_lds, smem);
 }
 // LDS words of a traversal workgroup: the stacks, for closest hits the hit words too
 constexpr int TW_LDS_ANY = FF_LDS_STACK * TW_BLOCK, TW_LDS_CLOSEST = (FF_LDS_STACK + 3) * TW_BLOCK;
 
+// the words in which a workgroup counts what rays traced again test
+__device__ __forceinline__ void clear_again(uint32_t* again, uint32_t n) {
+    if (threadIdx.x < n) again[threadIdx.x] = 0u;
+    __syncthreads();
+}
 // SMALL: a call with at most QUAD_MAX paths in flight
 template <bool UNI, bool SMALL>
-__device__ __forceinline__ void extend_rays(const ff_paths& P, int q, uint32_t block, uint32_t blocks, int* smem) {
+__device__ __forceinline__ void extend_rays(const ff_paths& P, int q, uint32_t block, uint32_t blocks, int* smem,
+                                            lds_u32* again) {
     // the counters that the coming stages of the iteration add to (nothing
     // reads them during the traversal; those it reads are cleared by the logic)
     if (block == 0 && threadIdx.x < 6)
@@ -948,27 +949,32 @@ __device__ __forceinline__ void extend_rays(const ff_paths& P, int q, uint32_t b
     const uint32_t n = P.counters[ext_counter(q)];
     uint32_t* const fetch = P.fetch + F_EXT * FETCH_SEGS * FETCH_STRIDE;
     unsigned long long* const cnt = stats_rep(P) + S_EXT_NODES;
-    if (SMALL) trav_quad<TW_BLOCK, false>(src, n, block, blocks, fetch, cnt, smem);
-    else traverse<false>(src, n, block, blocks, P.quad != 0, fetch, P.ovf, cnt, smem);
+    if (SMALL) trav_quad<TW_BLOCK, false>(src, n, block, blocks, fetch, cnt, again, smem);
+    else traverse<false>(src, n, block, blocks, P.quad != 0, fetch, P.ovf, cnt, again, smem);
 }
 template <bool UNI, bool SMALL>
-__device__ __forceinline__ void shadow_rays(const ff_paths& P, int q, uint32_t block, uint32_t blocks, int* smem) {
+__device__ __forceinline__ void shadow_rays(const ff_paths& P, int q, uint32_t block, uint32_t blocks, int* smem,
+                                            lds_u32* again) {
     const ShadowSrc<UNI> src{P};
     const uint32_t n = P.counters[shadow_counter(q)];
     uint32_t* const fetch = P.fetch + F_SHD * FETCH_SEGS * FETCH_STRIDE;
     unsigned long long* const cnt = stats_rep(P) + S_SHD_NODES;
-    if (SMALL) trav_quad<TW_BLOCK, true>(src, n, block, blocks, fetch, cnt, smem);
-    else traverse<true>(src, n, block, blocks, P.quad != 0, fetch, P.ovf_shd, cnt, smem);
+    if (SMALL) trav_quad<TW_BLOCK, true>(src, n, block, blocks, fetch, cnt, again, smem);
+    else traverse<true>(src, n, block, blocks, P.quad != 0, fetch, P.ovf_shd, cnt, again, smem);
 }
 template <bool UNI>
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_CLOSEST];
-    extend_rays<UNI, false>(P, q, blockIdx.x, gridDim.x, smem);
+    __shared__ uint32_t again[2];
+    clear_again(again, 2);
+    extend_rays<UNI, false>(P, q, blockIdx.x, gridDim.x, smem, (lds_u32*)again);
 }
 template <bool UNI>
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_shadow(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_ANY];
-    shadow_rays<UNI, false>(P, q, blockIdx.x, gridDim.x, smem);
+    __shared__ uint32_t again[2];
+    clear_again(again, 2);
+    shadow_rays<UNI, false>(P, q, blockIdx.x, gridDim.x, smem, (lds_u32*)again);
 }
 // An iteration's extension rays and its vertices' shadow rays (both come from
 // the previous shading pass) in one launch: workgroups alternate between the
@@ -985,13 +991,15 @@ constexpr uint32_t EXTEND_FEW = 2u << 20, EXTEND_MANY = 16u << 20;
 template <bool UNI, int OCC>
 __global__ __launch_bounds__(TW_BLOCK, OCC) void k_extend_shadow(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_CLOSEST];
+    __shared__ uint32_t again[4];
+    clear_again(again, 4);
     const uint32_t blocks = gridDim.x / 2u;
     for (uint32_t ph = 0; ph < 2; ph++) {
         // (a queue's guests are numbered after its own workgroups, whose waves
         // may hold all its rays by their number)
         const uint32_t block = (blockIdx.x >> 4) * 8u + (blockIdx.x & 7u) + ph * blocks;
-        if ((((blockIdx.x >> 3) + ph) & 1u) == 0u) extend_rays<UNI, false>(P, q, block, blocks, smem);
-        else shadow_rays<UNI, false>(P, q, block, blocks, smem);
+        if ((((blockIdx.x >> 3) + ph) & 1u) == 0u) extend_rays<UNI, false>(P, q, block, blocks, smem, (lds_u32*)again);
+        else shadow_rays<UNI, false>(P, q, block, blocks, smem, (lds_u32*)again + 2);
     }
 }
 // The same for a call with at most QUAD_MAX paths in flight: each queue has
@@ -999,9 +1007,11 @@ __global__ __launch_bounds__(TW_BLOCK, OCC) void k_extend_shadow(ff_paths P, int
 template <bool UNI>
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_extend_shadow_small(ff_paths P, int q) {
     __shared__ int smem[TW_LDS_ANY];
+    __shared__ uint32_t again[2];
+    clear_again(again, 2);
     const uint32_t block = (blockIdx.x >> 4) * 8u + (blockIdx.x & 7u);
-    if (blockIdx.x & 8u) shadow_rays<UNI, true>(P, q, block, gridDim.x / 2u, smem);
-    else extend_rays<UNI, true>(P, q, block, gridDim.x / 2u, smem);
+    if (blockIdx.x & 8u) shadow_rays<UNI, true>(P, q, block, gridDim.x / 2u, smem, (lds_u32*)again);
+    else extend_rays<UNI, true>(P, q, block, gridDim.x / 2u, smem, (lds_u32*)again);
 }
 
 // clears the work counters of the standalone traces (a kernel: graph-safe)
@@ -2226,12 +2236,12 @@ __global__ __launch_bounds__(BS) void k_trace_any(TraceArgs a) {
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_trace_closest_wide(TraceArgs a) {
     __shared__ int smem[TW_LDS_CLOSEST];
     RaySrc src{a.S, a.rays, a.hits, nullptr, a.two_sided};
-    traverse<false>(src, a.n, blockIdx.x, gridDim.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
+    traverse<false>(src, a.n, blockIdx.x, gridDim.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, nullptr, smem);
 }
 __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_trace_any_wide(TraceArgs a) {
     __shared__ int smem[TW_LDS_ANY];
     RaySrc src{a.S, a.rays, nullptr, a.occ, 0};
-    traverse<true>(src, a.n, blockIdx.x, gridDim.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, smem);
+    traverse<true>(src, a.n, blockIdx.x, gridDim.x, quad_fits(a.S.wide_levels, a.S.max_depth), a.fetch, a.ovf, nullptr, nullptr, smem);
 }
 __global__ void k_gen_rays(ff_dev_camera cam, int32_t W, int32_t H, uint32_t seed, uint32_t sample,
                            float4* rays) {

@@ -122,16 +122,23 @@ typedef struct {
 
 #define FF_RENDER_USE_GRAPH 1 /* capture the bounce loop in a hipGraph              */
 #define FF_RENDER_TIMING 2    /* time every stage launch with hipEvents (stats); the
-                                 stages then run one after another (otherwise each
-                                 iteration's shadow traversal overlaps its extension) */
+                                 stages then are launches of their own, one after
+                                 another (otherwise one launch traces an iteration's
+                                 extension and shadow rays and one routes and shades) */
 
 typedef struct {
     double rays_primary;   /* camera rays (closest hit)                     */
     double rays_extension; /* bounce >= 1 extension rays                     */
     double rays_shadow;    /* any-hit rays (light + BRDF-sampled visibility) */
     double paths;          /* completed samples                              */
-    double ext_nodes, ext_tris;       /* boxes / triangles tested by extend  */
-    double shadow_nodes, shadow_tris; /* boxes / triangles tested by shadow  */
+    /* Boxes and triangles tested by the walk that ran, over compressed wide
+     * records: four boxes a record, those of empty children among them, and the
+     * boxes and triangles of rays traced again in the reference's order.  They
+     * measure work, not the reference's visits (a trace with counts gives
+     * those): above 131072 rays a launch they also depend a little on which
+     * rays share a wave. */
+    double ext_nodes, ext_tris;       /* by extend */
+    double shadow_nodes, shadow_tris; /* by shadow */
     /* FF_RENDER_TIMING only: summed launch durations (ms) and launch counts */
     double ms_extend, ms_shadow, ms_logic, ms_shade, ms_other;
     double launches_extend, launches_shadow;
@@ -297,7 +304,7 @@ ff_status ff_adjoint_batch(ff_context *ctx, const ff_batch_item *items, int32_t 
 /* ---- traversal kernel variants of traces that count.  Renders, and traces
  * that ask for no counts, walk compressed wide records with one launch shape
  * and return the reference's hits; the counts of ff_last_render_stats are of
- * the boxes (four a record) and triangles that walk tests.  A trace that asks
+ * that walk (see ff_ray_stats).  A trace that asks
  * for counts walks the reference's tree in the reference's order with the
  * context's variant: workgroup size, LDS stack entries, the number of idle
  * lanes at which a wave fetches new rays, the loop shape: 0 = one step per
