@@ -881,6 +881,11 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
                     if (in && rank > 0) *st.at(st.sp + __popc(m) - 1 - rank) = (int)(w | k);
                 }
                 st.sp += __popc(m) - 1;
+                // The quad's lanes pop what any of them pushed.  A wave's LDS
+                // operations are carried out in order; the fence (no instruction)
+                // keeps the compiler from moving a pop above the pushes.
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront", "local");
+                __builtin_amdgcn_wave_barrier();
             } else {
                 cur = (uint32_t)st.pop();
             }
