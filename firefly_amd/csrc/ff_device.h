@@ -1222,31 +1222,6 @@ __device__ __forceinline__ void add_tested(unsigned long long* cnt, uint32_t rec
 }
 
 // ----------------------------------------------------- wave64 utilities --
-// Wave-aggregated queue append: one atomic per wave, lane offsets from the
-// 64-bit ballot (replaces the 32-lane atomicAggInc, CRT/kernel.cu:24-36).
-// Every lane of the wave must call it; returns the slot for lanes with pred.
-__device__ __forceinline__ uint32_t wave_append(uint32_t* counter, bool pred) {
-    uint64_t mask = __ballot(pred);
-    uint32_t rank = __builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32),
-                                              __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0u));
-    uint32_t base = 0;
-    if (mask) {
-        int leader = __ffsll((unsigned long long)mask) - 1;
-        if ((int)__lane_id() == leader) base = atomicAdd(counter, (uint32_t)__popcll(mask));
-        base = __shfl(base, leader);
-    }
-    return base + rank;
-}
-// Wave-aggregated 64-bit counter of lanes with pred.
-__device__ __forceinline__ void wave_count(unsigned long long* counter, bool pred) {
-    uint64_t mask = __ballot(pred);
-    uint64_t all = __ballot(1);
-    if (mask) {
-        int leader = __ffsll((unsigned long long)all) - 1;
-        if ((int)__lane_id() == leader) atomicAdd(counter, (unsigned long long)__popcll(mask));
-    }
-}
-
 // Sum of a per-lane value over a full wave, added once per wave.  Must be
 // called with every lane of the wave active (after the grid-stride loop).
 __device__ __forceinline__ void wave_sum_add(unsigned long long* counter, uint32_t v) {
@@ -1254,42 +1229,6 @@ __device__ __forceinline__ void wave_sum_add(unsigned long long* counter, uint32
 #pragma unroll
     for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off);
     if (__lane_id() == 0) atomicAdd(counter, s);
-}
-
-// Workgroup-aggregated queue allocation: thread t asks for cnt[q] (0..3)
-// slots of queue q; one atomic per queue per workgroup (device-scope atomics
-// on one address serialise at the memory side, so per-wave atomics on a few
-// queue counters throttle whole kernels).  Every thread of the workgroup must
-// call it the same number of times.  lds: NQ * (BS / 64 + 1) words.
-template <int BS, int NQ>
-__device__ __forceinline__ void block_alloc(uint32_t* counters, const int* qidx, const uint32_t* cnt,
-                                            uint32_t* first, uint32_t* lds) {
-    constexpr int NW = BS / 64;
-    const uint32_t w = threadIdx.x >> 6;
-    uint32_t pre[NQ];
-#pragma unroll
-    for (int q = 0; q < NQ; q++) {
-        uint64_t b0 = __ballot((cnt[q] & 1u) != 0), b1 = __ballot((cnt[q] & 2u) != 0);
-        uint32_t r0 = __builtin_amdgcn_mbcnt_hi((uint32_t)(b0 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b0, 0u));
-        uint32_t r1 = __builtin_amdgcn_mbcnt_hi((uint32_t)(b1 >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)b1, 0u));
-        pre[q] = r0 + 2u * r1;
-        if (__lane_id() == 0) lds[q * (NW + 1) + w] = (uint32_t)__popcll(b0) + 2u * (uint32_t)__popcll(b1);
-    }
-    __syncthreads();
-    if (threadIdx.x < NQ) {
-        const int q = threadIdx.x;
-        uint32_t tot = 0;
-        for (int k = 0; k < NW; k++) {
-            uint32_t c = lds[q * (NW + 1) + k];
-            lds[q * (NW + 1) + k] = tot;
-            tot += c;
-        }
-        lds[q * (NW + 1) + NW] = tot ? atomicAdd(&counters[qidx[q]], tot) : 0u;
-    }
-    __syncthreads();
-#pragma unroll
-    for (int q = 0; q < NQ; q++) first[q] = lds[q * (NW + 1) + NW] + lds[q * (NW + 1) + w] + pre[q];
-    __syncthreads();
 }
 
 // Queue appends staged in LDS.  A device-scope atomic on one address costs

@@ -490,7 +490,7 @@ __device__ __forceinline__ void trav_persistent(const RaySrc& src, uint32_t n, u
                     busy = false;
                 }
             } else {
-                // closest_step with the hit's u, v and slot in LDS
+                // one step, with the hit's u, v and slot in LDS
                 bool cont = true;
                 if (R.ref >= 0 && visit_node<WIDE, true>(B, R, lim, st, cn)) {
                 } else {
@@ -989,9 +989,11 @@ __global__ __launch_bounds__(TW_BLOCK, TW_OCC) void k_shadow(ff_paths P, int q) 
 // OCC, waves a SIMD: a call of few paths lasts as long as its slowest rays, and
 // 5 waves (96 VGPRs) spill nothing; a call of many is bound by the latency of
 // its visits, and 7 waves (72 VGPRs) hide more of it, spills and all.  5, 6 and
-// 7 waves at 256 k paths (spheres, 16 samples): 3.10, 3.25, 3.45 ms; at 460 k
-// (327 k triangles): 1.57, 1.61, 1.56; at 4.7 M: 4.02, 3.99, 4.06; at 33 M
-// (327 k triangles): 16.0, 15.4, 15.0; at 133 M: 62.3, 59.2, 58.0.
+// 7 waves at 256 k paths (spheres, 16 samples): 3.10, 3.25, 3.45 ms; at 33 M
+// (327 k triangles): 16.0, 15.4, 15.0; at 133 M: 62.3, 59.2, 58.0.  Between
+// these sizes the three are within 3 % of one another, and not always in that
+// order (460 k, 327 k triangles: 1.57, 1.61, 1.56; 4.7 M: 4.02, 3.99, 4.06): the
+// limits lie there.
 constexpr uint32_t EXTEND_FEW = 2u << 20, EXTEND_MANY = 16u << 20;
 template <bool UNI, int OCC>
 __global__ __launch_bounds__(TW_BLOCK, OCC) void k_extend_shadow(ff_paths P, int q) {
@@ -1192,8 +1194,9 @@ __device__ __forceinline__ void add_counts(const ff_paths& P, const LogicCounts&
     wave_sum_add(sr + S_EXTENSION, c.ext);
     wave_sum_add(sr + S_PATHS, c.paths);
 }
-template <bool UNI, int NP>
-__global__ __launch_bounds__(FF_BLOCK, NP == 1 ? 8 : 5) void k_logic(ff_paths P, int q, int iter) {
+template <bool UNI>
+__global__ __launch_bounds__(FF_BLOCK, 5) void k_logic(ff_paths P, int q, int iter) {
+    constexpr int NP = 2;
     __shared__ QStage<FF_BLOCK, 4, QSTAGE_CAP> st;
     const int qidx[4] = {mat_counter(q), mat_counter(q) + 1, mat_counter(q) + 2, mat_counter(q) + 3};
     uint32_t* const qs[4] = {P.q_mat[0], P.q_mat[1], P.q_mat[2], P.q_mat[3]};
@@ -2715,7 +2718,7 @@ void prepare_launches() {
 }
 template <bool UNI>
 hipError_t logic_launch(const ff_paths& P, int q, int iter, uint32_t n_max, hipStream_t s) {
-    hipLaunchKernelGGL((k_logic<UNI, 2>), dim3(grid_for(n_max, FF_GRID_CAP)), dim3(FF_BLOCK), 0, s, P, q, iter);
+    hipLaunchKernelGGL(k_logic<UNI>, dim3(grid_for(n_max, FF_GRID_CAP)), dim3(FF_BLOCK), 0, s, P, q, iter);
     return hipGetLastError();
 }
 hipError_t launch_logic(const ff_paths& P, int q, int iter, uint32_t n_max, hipStream_t s) {
