@@ -887,6 +887,7 @@ struct HitSlots {
     lds_float* u;
     lds_float* v;
     lds_int* id;
+    lds_float* redo;  // wide walk: smallest t whose outcome the reference's order decides
 };
 __device__ __forceinline__ void leaf_closest_slots(const Bvh& B, const float* __restrict__ tris, const TravRay& R,
                                                    float& t_hit, const HitSlots& hs, bool two_sided,
@@ -963,9 +964,19 @@ __device__ __forceinline__ int any_step(const Bvh& B, const float* __restrict__ 
 // passes the reference's test.  The closest hit is the smallest t, whatever
 // the visit order; where two triangles share it exactly, or a box plane
 // distance is NaN (0 * inf), the ray is traced again in the reference's order.
+//
+// Early hits: the t of a grazing hit is rounded so coarsely that it can lie
+// before the entry into its own leaf's box, beyond the pruning's slack (a
+// triangle 4.4 long met at an angle of 3e-6: t 20.4, entry 21.2).  Whether such
+// a triangle is reached depends on the hits found before it, so it is no
+// candidate and lowers no pruning limit; every triangle that is one is then
+// reached whatever the order.  A ray with an early hit nearer than its closest
+// candidate is traced again in the reference's order, which decides.  (An early
+// hit counts for less only where that order would enter its leaf's box before a
+// nearer one that holds a hit, and this walk, which enters nearer boxes first,
+// does not reach it.)
 #define WREF_INDEX 0x1fffffffu
 #define WREF_ROOT (4u << 29)  // record 0, an interior child
-#define WHIT_REDO 0x40000000  // hit word: trace the ray again in the reference's order
 // Slack of the conservative plane distances: a distance is fma(plane, inv, b)
 // with b = (org - o) * inv.  Against the reference's (lo - o) * inv the two
 // differ by at most 2.5 * 2^-23 |b| + 1.5 * 2^-23 |plane * inv|; the first is
@@ -1101,18 +1112,22 @@ __device__ __forceinline__ WideTri load_wide_tri(const float4* rec, uint32_t ref
     w.hi = V3(d.y, d.z, d.w);
     return w;
 }
-// The reference's test of the triangle's leaf box, as its walk makes it.
-// nanx: an x plane distance is NaN there, so ancestors may not follow.
-__device__ __forceinline__ bool wide_leaf_box(const WideTri& w, const WideRay& R, bool& nanx) {
+// The reference's test of the triangle's leaf box, as its walk makes it; tn:
+// the entry.  nanx: an x plane distance is NaN there, so ancestors may not follow.
+__device__ __forceinline__ bool wide_leaf_box(const WideTri& w, const WideRay& R, bool& nanx, float& tn) {
     f3 inv = R.inv;
-    float tn, tf;
+    float tf;
     nanx = false;
     if (__ballot(R.fl != 0u) == 0)
-        return slab_box(w.lo.x, w.lo.y, w.lo.z, w.hi.x, w.hi.y, w.hi.z, R.o, inv, R.nx, R.ny, R.nz, tn, tf);
+        return slab_box(w.lo.x, w.lo.y, w.lo.z, w.hi.x, w.hi.y, w.hi.z, R.o, inv, R.nx, R.ny, R.nz, tn, tf) &&
+               !(tf < -PRUNE_BEHIND);
     if (R.fl & WINV_CLAMPED) inv = V3(1.f / R.d.x, 1.f / R.d.y, 1.f / R.d.z);
     nanx = (R.fl & XNAN_RAY) != 0u && (!isfinite(R.o.x) || R.o.x == w.lo.x || R.o.x == w.hi.x);
-    return slab(w.lo.x, w.lo.y, w.lo.z, w.hi.x, w.hi.y, w.hi.z, R.o, inv, R.nx, R.ny, R.nz, tn, tf);
+    return slab(w.lo.x, w.lo.y, w.lo.z, w.hi.x, w.hi.y, w.hi.z, R.o, inv, R.nx, R.ny, R.nz, tn, tf) &&
+           !(tf < -PRUNE_BEHIND);
 }
+// an early hit: the leaf is entered (tn) beyond the pruning limit of the hit's own t
+__device__ __forceinline__ bool early_hit(float t, float tn) { return tn > prune_lim(t); }
 __device__ __forceinline__ void wide_leaf_closest(const float4* rec, uint32_t ref, const WideRay& R, float& t_hit,
                                                   const HitSlots& hs, bool two_sided) {
     WideTri w = load_wide_tri(rec, ref);
@@ -1120,14 +1135,15 @@ __device__ __forceinline__ void wide_leaf_closest(const float4* rec, uint32_t re
     bool ok = two_sided ? mt_two(w.T, R.o, R.d, t, u, v) : mt_cull(w.T, R.o, R.d, t, u, v);
     if (ok && !(t < 0.f) && t <= t_hit) {
         bool nanx;
-        if (wide_leaf_box(w, R, nanx)) {
-            if (t < t_hit) {
+        float tn;
+        if (wide_leaf_box(w, R, nanx, tn)) {
+            const bool early = early_hit(t, tn);
+            if (early || nanx || t == t_hit) *hs.redo = fminf(*hs.redo, t);
+            if (!early && t < t_hit) {
                 t_hit = t;
                 *hs.u = u;
                 *hs.v = v;
-                *hs.id = w.slot | (nanx ? WHIT_REDO : 0);
-            } else if (*hs.id >= 0) {
-                *hs.id |= WHIT_REDO;  // the same distance: the reference's order decides
+                *hs.id = w.slot;
             }
         }
     }
@@ -1138,7 +1154,8 @@ __device__ __forceinline__ int wide_leaf_any(const float4* rec, uint32_t ref, co
     float t = 0.f;
     if (!(mt_shadow(w.T, R.o, R.d, t) && t < K_HUGE)) return 0;
     bool nanx;
-    if (!wide_leaf_box(w, R, nanx)) return 0;
+    float tn;
+    if (!wide_leaf_box(w, R, nanx, tn)) return 0;
     return nanx ? 2 : 1;
 }
 

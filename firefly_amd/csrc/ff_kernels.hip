@@ -562,6 +562,7 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
     hs.u = ANY ? nullptr : (lds_float*)&smem[LDS * BS + threadIdx.x];
     hs.v = ANY ? nullptr : (lds_float*)&smem[LDS * BS + BS + threadIdx.x];
     hs.id = ANY ? nullptr : (lds_int*)&smem[LDS * BS + 2 * BS + threadIdx.x];
+    hs.redo = ANY ? nullptr : (lds_float*)&smem[LDS * BS + 3 * BS + threadIdx.x];
     auto start = [&](f3 o, f3 d) {
         wide_begin(o, d, R);
         if (!ANY) {
@@ -569,13 +570,14 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
             *hs.u = 0.f;
             *hs.v = 0.f;
             *hs.id = -1;
+            *hs.redo = INFINITY;
         }
         st.sp = 1;
         cur = WREF_ROOT;
         pend = 0;
     };
     // Rays whose outcome the reference's visit order decides (two triangles at
-    // one distance, a NaN plane distance) park their lane; once many lanes are
+    // one distance, a NaN plane distance, an early hit) park their lane; once many lanes are
     // parked, or no other work is left, those rays walk the binary records with
     // every other lane idle (the walk's registers then add nothing to the loop).
     bool parked = false;
@@ -687,7 +689,7 @@ __device__ __forceinline__ void trav_wide(const Src& src, uint32_t n, uint32_t b
                     h.t = t_hit;
                     h.u = *hs.u;
                     h.v = *hs.v;
-                    parked = h.id >= 0 && (h.id & WHIT_REDO);
+                    parked = *hs.redo <= t_hit;
                     if (!parked) {
                         src.hit(id, h);
                         id = IDLE;
@@ -777,7 +779,7 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
     R.fl = 0u;
     float t_hit = K_HUGE;           // of the quad
     Hit best = no_hit();            // of the lane
-    float redo_t = -1.f;            // a distance that the reference's order decides
+    float redo_t = INFINITY;        // smallest t whose outcome the reference's order decides (ANY: 0, if it does)
     const uint32_t cap = quad_rays(n);
     const bool fixed = quad_fixed(n, blocks * (BS / 64));
     const bool mine = (lane >> 2) < cap;
@@ -785,7 +787,7 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
         wide_begin(o, d, R);
         t_hit = K_HUGE;
         best = no_hit();
-        redo_t = -1.f;
+        redo_t = INFINITY;
         *st.at(0) = 0;  // popping the bottom ends the walk
         st.sp = 1;
         cur = WREF_ROOT;
@@ -846,9 +848,11 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
                         WideTri T = load_wide_tri(rec, w | k);
                         float u = 0.f, v = 0.f;
                         bool ok = two ? mt_two(T.T, R.o, R.d, t, u, v) : mt_cull(T.T, R.o, R.d, t, u, v), nanx;
-                        if (ok && !(t < 0.f) && t <= t_hit && wide_leaf_box(T, R, nanx)) {
-                            if (nanx || t == t_hit) redo_t = t;
-                            if (t < t_hit) {
+                        float entry;
+                        if (ok && !(t < 0.f) && t <= t_hit && wide_leaf_box(T, R, nanx, entry)) {
+                            const bool early = early_hit(t, entry);
+                            if (early || nanx || t == t_hit) redo_t = fminf(redo_t, t);
+                            if (!early && t < t_hit) {
                                 best.t = t;
                                 best.u = u;
                                 best.v = v;
@@ -893,7 +897,7 @@ __device__ __forceinline__ void trav_quad(const Src& src, uint32_t n, uint32_t b
         ct += (uint32_t)__popcll(__ballot(tri));
         const bool fin = id != IDLE && (occ || cur == 0u);
         if (__ballot(fin) == 0) continue;
-        const bool redo = quad_mask(ANY ? redo_t == 0.f && !occ : redo_t >= 0.f && redo_t == t_hit) != 0u ||
+        const bool redo = quad_mask(ANY ? redo_t == 0.f && !occ : redo_t <= t_hit) != 0u ||
                           (!ANY && __popc(quad_mask(best.id >= 0 && best.t == t_hit)) > 1);
         uint32_t gated = 0;
         if (fin) {
@@ -934,7 +938,7 @@ __device__ __forceinline__ void traverse(const Src& src, uint32_t n, uint32_t bl
     else trav_wide<TW_BLOCK, ANY>(src, n, block, fetch, ovf, cnt, again_lds, smem);
 }
 // LDS words of a traversal workgroup: the stacks, for closest hits the hit words too
-constexpr int TW_LDS_ANY = FF_LDS_STACK * TW_BLOCK, TW_LDS_CLOSEST = (FF_LDS_STACK + 3) * TW_BLOCK;
+constexpr int TW_LDS_ANY = FF_LDS_STACK * TW_BLOCK, TW_LDS_CLOSEST = (FF_LDS_STACK + 4) * TW_BLOCK;
 
 // the words in which a workgroup counts what rays traced again test
 __device__ __forceinline__ void clear_again(uint32_t* again, uint32_t n) {
