@@ -1178,7 +1178,8 @@ __device__ __forceinline__ Hit reference_walk(const Bvh& B, const float* __restr
     int ref = __float_as_int(ldg(B.root + 6));
     if (again) lds_count(again, 1u);
     if (!slab(ldg(B.root), ldg(B.root + 1), ldg(B.root + 2), ldg(B.root + 3), ldg(B.root + 4), ldg(B.root + 5), o, inv,
-              nx, ny, nz, tn, tf))
+              nx, ny, nz, tn, tf) ||
+        tf < -PRUNE_BEHIND)
         return h;
     st.sp = 0;
     for (;;) {
