@@ -972,9 +972,10 @@ __device__ __forceinline__ int any_step(const Bvh& B, const float* __restrict__ 
 // candidate and lowers no pruning limit; every triangle that is one is then
 // reached whatever the order.  A ray with an early hit nearer than its closest
 // candidate is traced again in the reference's order, which decides.  (An early
-// hit counts for less only where that order would enter its leaf's box before a
-// nearer one that holds a hit, and this walk, which enters nearer boxes first,
-// does not reach it.)
+// hit is missed only where the walk in that order tests its leaf's box before it
+// has a hit nearer than that box, and this walk after: 4 of 500000 grazing rays
+// through random slivers.  With pruning that walk itself misses 3 of the hits
+// that the same rays have without.)
 #define WREF_INDEX 0x1fffffffu
 #define WREF_ROOT (4u << 29)  // record 0, an interior child
 // Slack of the conservative plane distances: a distance is fma(plane, inv, b)
